@@ -335,7 +335,7 @@ PG_DEV FaceArrays face_arrays_of(const __attribute__((address_space(4))) FaceArr
 template <int DIM, int G, int S, bool FRESH>
 __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_bvoronoi_loop(BClipArgs args) {
     using C = VoroCfg<DIM, G, S>;
-    __shared__ SeedSmem<C::NS, C::MAXP> sm[C::SPW];
+    __shared__ VoroSmem<DIM, G, S> sm[C::SPW];
     if constexpr (FRESH) {
         bool first = true;
         for (;;) {
@@ -371,7 +371,7 @@ __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES))
     k_bvoronoi(const double* __restrict__ pts, const uint32_t* __restrict__ seeds, const int64_t* __restrict__ nq_dev,
                const uint32_t* __restrict__ knn, int k, int max_p, int max_t, FaceArrays fa) {
     using C = VoroCfg<DIM, G, S>;
-    __shared__ SeedSmem<C::NS, C::MAXP> sm[C::SPW];
+    __shared__ VoroSmem<DIM, G, S> sm[C::SPW];
     const int64_t nq = *nq_dev;
     const int64_t vb = blockIdx.x;
     if (vb * C::SPW >= nq) return;  // whole block

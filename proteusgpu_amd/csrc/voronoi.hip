@@ -17,7 +17,7 @@ __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_voronoi(con
                                                 const uint32_t* __restrict__ knn, int k, int max_p,
                                                 int max_t, FaceArrays fa) {
     using C = VoroCfg<DIM, G, S>;
-    __shared__ SeedSmem<C::NS, C::MAXP> sm[C::SPW];
+    __shared__ VoroSmem<DIM, G, S> sm[C::SPW];
     voronoi_group<DIM, G, S>(pts, n_total, seeds, nq, knn, k, max_p, max_t, fa, sm,
                              xcd_block(blockIdx.x, gridDim.x));
 }
@@ -30,7 +30,7 @@ __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_voronoi_res
                                                         const uint32_t* __restrict__ knn, int k, int max_p,
                                                         int max_t, FaceArrays fa) {
     using C = VoroCfg<DIM, G, S>;
-    __shared__ SeedSmem<C::NS, C::MAXP> sm[C::SPW];
+    __shared__ VoroSmem<DIM, G, S> sm[C::SPW];
     voronoi_group<DIM, G, S>(pts, n_total, seeds, nq, knn, k, max_p, max_t, fa, sm,
                              xcd_block(blockIdx.x, gridDim.x));
 }
@@ -43,7 +43,7 @@ __global__ void __launch_bounds__(64, 1) k_voronoi_exact(const double* __restric
                                                          const uint32_t* __restrict__ knn, int k, int max_p,
                                                          int max_t, FaceArrays fa) {
     using C = VoroCfg<DIM, 16, 8>;
-    __shared__ SeedSmem<C::NS, C::MAXP> sm[C::SPW];
+    __shared__ VoroSmem<DIM, 16, 8> sm[C::SPW];
     voronoi_group<DIM, 16, 8, true>(pts, n_total, seeds, nq, knn, k, max_p, max_t, fa, sm, blockIdx.x);
 }
 
@@ -54,7 +54,7 @@ __global__ void __launch_bounds__(64, 1) k_voronoi_ball(const double* __restrict
                                                         const uint32_t* __restrict__ knn, int k, int max_p,
                                                         int max_t, FaceArrays fa, BallGrid bg) {
     using C = VoroCfg<DIM, 16, 8>;
-    __shared__ SeedSmem<C::NS, C::MAXP> sm[C::SPW];
+    __shared__ VoroSmem<DIM, 16, 8> sm[C::SPW];
     __shared__ int32_t scr[C::SPW * (2 * 16 + 1)];
     bg.scr = scr;
     voronoi_group<DIM, 16, 8, false, true>(pts, n_total, seeds, nq, knn, k, max_p, max_t, fa, sm, blockIdx.x, bg);

@@ -13,6 +13,9 @@
 //     seed distance d2 and two float bounds (q, m) used by the filter below.
 //   * planes (FP64), plane->neighbour ids, vertex plane triples and the
 //     vertex adjacency (slot across each edge) live in LDS.
+//   * row entries are taken in windows of 16; the ones whose plane cannot
+//     reach the cell are passed over (see vertex_good), the matrix cores
+//     making the 16 x vertices products of a window.
 //   * a clip tests every live vertex in parallel.  The reference decides
 //     with a 4x4 (3x3 in 2D) FP64 determinant per vertex; here
 //     det ~= W * (e . p + e.w) is evaluated from the cached vertex and used
@@ -60,16 +63,13 @@ struct VoroCfg {
     static_assert(MAXP % G == 0, "planes tile the group");
 };
 
-constexpr int NB_CHUNK = 12;
-
-template <int NS, int MAXP>
+template <int NS, int MAXP, int G>
 struct SeedSmem {
     union {
         Plane plane[MAXP];      // planes while clipping
         double vpos[3 * NS];    // vertex positions during extraction
     };
     float pn1[MAXP];        // |x|+|y|+|z|+|w| rounded up
-    float pmx[MAXP];        // largest coefficient entering the eps test, rounded up
     int32_t pvid[MAXP];     // neighbour (sorted id) of each plane, -1 = box
     uint32_t tri[NS];       // planes of each vertex: a | b << 8 | c << 16
     uint8_t adj[3][NS];     // neighbour slot across edge/line e
@@ -79,12 +79,15 @@ struct SeedSmem {
             uint8_t newslot[NS];      // slot of the j-th new vertex
             uint8_t by_start[MAXP];   // 3D: boundary edge starting at a plane
             uint8_t by_end[MAXP];     // 3D: boundary edge ending at a plane
-            uint32_t nbi[NB_CHUNK];   // next chunk of the neighbour row (prefetched)
-            double nbp[NB_CHUNK][3];  // and the neighbours' positions
+            uint32_t nbi[G];   // window of the neighbour row, one entry per lane
+            double nbp[G][3];  // and the neighbours' positions
         };
         uint32_t first[MAXP];  // extraction: vertex of each plane with the lowest plane key
     };
 };
+
+template <int DIM, int G, int S>
+using VoroSmem = SeedSmem<VoroCfg<DIM, G, S>::NS, VoroCfg<DIM, G, S>::MAXP, G>;
 
 // Round a non-negative double up to float (next float above on inexact).
 PG_DEV float f2f_up(double d) {
@@ -168,21 +171,14 @@ PG_DEV bool conflict_exact(const Plane& p1, const Plane& p2, const Plane& p3, co
     return det > 0.0;
 }
 
-// n1: |x| + |y| + |z| + wm rounded up to float, wm = |w| (or, in exact
-// mode, the magnitude that bounds the rounding error of w, see XTOL)
-template <int DIM>
-PG_DEV void plane_bounds(const Plane& p, double wm, float& n1, float& mx) {
-    n1 = f2f_up(fabs(p.x) + fabs(p.y) + fabs(p.z) + wm);
-    double m = DIM == 2 ? fmax(fmax(fabs(p.x), fabs(p.y)), fabs(p.w))
-                        : fmax(fmax(fabs(p.x), fabs(p.y)), fabs(p.z));
-    mx = f2f_up(m);
-}
+// |x| + |y| + |z| + wm rounded up to float, wm = |w| (or, in exact mode, the
+// magnitude that bounds the rounding error of w, see XTOL)
+PG_DEV float plane_n1(const Plane& p, double wm) { return f2f_up(fabs(p.x) + fabs(p.y) + fabs(p.z) + wm); }
 
 // Per-seed register state of one lane.  Per slot: q bounds the product of
 // the vertex's plane 1-norms; e5 is the vertex's share of the reference's
-// eps, an upper bound (float, at least the smallest normal float) of
-// 1.0000001e-14 m^5 (m^4 in 2D), m the largest normal component among its
-// planes, made once with the vertex instead of at every conflict test.
+// eps (eps_bound of the largest 1-norm among its planes), made once with the
+// vertex instead of at every conflict test.
 template <int S>
 struct SlotRegs {
     double px[S], py[S], pz[S], pw[S], d2[S];
@@ -190,28 +186,27 @@ struct SlotRegs {
     uint32_t live;  // bit s = slot s holds a vertex
 };
 
-// 1.0000001e-14 M^5 (M^4 in 2D), the bound of the reference's conflict eps
-// (cell.cpp:175-221: 1e-14 times a product of five, or four, component
-// maxima each at most M), computed in double.  Rounding of the products is
+// An upper bound (float, at least the smallest normal float) of 1.0000001e-14
+// m^5 (m^4 in 2D): the reference's conflict eps (cell.cpp:175-221) is 1e-14
+// times a product of five, or four, component maxima, each at most the
+// largest 1-norm m of the planes involved.  Rounding of the products is
 // monotone, so the bound of max(a, b) is the max of the bounds.
 template <int DIM>
-PG_DEV double eps_bound(double M) {
-    const double M2 = M * M;
-    return DIM == 3 ? 1.0000001e-14 * M2 * M2 * M : 1.0000001e-14 * M2 * M2;
-}
-
-template <int DIM, int S>
-PG_DEV void slot_write(SlotRegs<S>& r, int s, double px, double py, double pz, double pw, double d2,
-                       float q, float m) {
-    // In float: the constant, 1.000001e-14 as a float (relative error below
-    // 6e-8), and at most four products, each within 2^-24 of the exact one,
-    // stay above 1.0000001e-14 m^5.  When that bound is a normal float every
+PG_DEV float eps_bound(float m) {
+    // The constant, 1.000001e-14 as a float (relative error below 6e-8), and
+    // at most four products, each within 2^-24 of the exact one, stay above
+    // 1.0000001e-14 m^5.  When that bound is a normal float every
     // intermediate is normal too (m^k >= m^5 / 1e-14 for m < 1); a result
     // below the smallest normal float, subnormal or flushed to zero, is
     // raised to it by the integer max on its bit pattern (non-negative).
     const float m2 = m * m;
     const float mp = DIM == 3 ? m2 * m2 * m : m2 * m2;
-    const float e5 = __uint_as_float(max(__float_as_uint(mp * 1.000001e-14f), 0x00800000u));
+    return __uint_as_float(max(__float_as_uint(mp * 1.000001e-14f), 0x00800000u));
+}
+
+template <int DIM, int S>
+PG_DEV void slot_write(SlotRegs<S>& r, int s, double px, double py, double pz, double pw, double d2,
+                       float q, float e5) {
 #pragma unroll
     for (int i = 0; i < S; i++) {
         if (i == s) {
@@ -248,7 +243,7 @@ PG_DEV void vertex_numerics(const Plane& a, const Plane& b, const Plane& c, doub
 // and adjacency, then the plane and live-vertex counts.
 struct ClipState {
     Plane plane[64];
-    float pn1[64], pmx[64];
+    float pn1[64];
     int32_t pvid[64];
     uint32_t tri[64];
     uint8_t adj[3][64];
@@ -258,8 +253,8 @@ static_assert(sizeof(ClipState) <= CLIP_STATE_BYTES, "clip state layout");
 
 // Exact decision of a degenerate conflict test (exact.h) from the vertex's
 // plane triple tt, the new plane's point b (sorted id z) and the seed.
-template <int DIM, int NS, int MAXP>
-__device__ __noinline__ int exact_conflict(uint32_t tt, const SeedSmem<NS, MAXP>& sm, const double* pts,
+template <int DIM, class SM>
+__device__ __noinline__ int exact_conflict(uint32_t tt, const SM& sm, const double* pts,
                                            uint32_t sid, const double* sp, uint32_t z, const double* bp,
                                            const uint32_t* key) {
     XRow rows[DIM + 1];
@@ -490,6 +485,70 @@ PG_DEV int32_t ball_search_group(const BallGrid& bg, const double* __restrict__ 
     return pick;
 }
 
+// ---- passing over row entries that cannot cut the cell
+//
+// In a uniform 3D set about 45 row entries are walked per seed and 16 of
+// them cut the cell; a step that cuts nothing costs a conflict test of every
+// vertex, and idles the wave's other seeds or waits for their cuts.  With
+// the entries passed over, a wave of four seeds takes 24 steps at k = 64,
+// 22 of which cut a cell of it, and 19.5 of which each seed uses.  Measured
+// (1M uniform seeds, first pass): k = 64 12.7 -> 10.8 ms (26.2k -> 19.9k
+// VALU per wave), k = 32 10.1 -> 9.3 ms, 2D k = 16 3.4 -> 3.1 ms.  An entry with offset d = b - s cuts nothing when
+// d . (v - s) < |d|^2 / 2 for every vertex v, and then neither it nor any
+// later test of it can cut the cell, which only shrinks: the vertices made
+// later lie in the hull of the present ones.  The filter tests that in
+// float with a margin of SKIP_MARGIN |d|^2 and a slack for its own rounding.
+//
+// What is passed over would have been tested exactly: the reference flags a
+// cell when a conflict determinant W f (f = |d|^2/2 - d . (v - s)) is below
+// its eps, which a tiny W can bring about whatever f is, and a vertex with a
+// tiny W has an uncertain position.  A vertex is good when its W < 0 and
+// |W| SKIP_F E^2 exceeds twice the bound the conflict test trusts its
+// filtered value above (5.4e-15 n1(e) q + the eps bounds) for every offset
+// length E of the window (E0 <= E <= E1; n1(e) <= a E, a = 1.75 + |s|_1 +
+// E1/2, since |w| = |d . (s + b)| / 2).  Its position is then within
+// SKIP_F E0 / 4 of exact, so with f >= SKIP_MARGIN E^2 at every vertex at the
+// time of the filter, f >= SKIP_F E^2 at every good vertex made later, and
+// every test passed over would have ended in "kept", unflagged.  While a
+// vertex that is not good lives, nothing is passed over.
+constexpr float SKIP_MARGIN = 1.0f / 32;
+constexpr float SKIP_F = 1.0f / 64;
+// clips after which the rest of a window is filtered again
+constexpr int REFILTER = 4;
+
+struct SkipBounds {
+    float g1, g2, g3;  // |W| SKIP_F > g1 q + g2 e5 + g3
+};
+PG_DEV bool vertex_good(const SkipBounds& g, double pw, float q, float e5) {
+    return (float)pw * -SKIP_F > fmaf(g.g1, q, fmaf(g.g2, e5, g.g3));
+}
+// wd2: squared distance of this lane's entry, ascending over the pend
+// entries of the window (lanes 0 ..).
+template <int D, int G>
+PG_DEV SkipBounds window_bounds(double wd2, uint32_t pend, double sx, double sy, double sz) {
+    const float l2 = (float)wd2;
+    const float lo = shfl(l2, 0, G), hi = shfl(l2, pend ? 31 - __builtin_clz(pend) : 0, G);
+    const float E0 = __builtin_amdgcn_sqrtf(lo) * 0.999f, E1 = __builtin_amdgcn_sqrtf(hi) * 1.001f;
+    const float a = 1.75f + (float)(fabs(sx) + fabs(sy) + fabs(sz)) + 0.5f * E1;
+    const float a2 = a * a;
+    SkipBounds g;
+    g.g1 = 1.2e-14f * a / E0;
+    g.g2 = 2.1f / (E0 * E0);
+    g.g3 = D == 3 ? 2.1e-14f * a2 * a2 * a * E1 * E1 * E1 : 2.1e-14f * a2 * a2 * E1 * E1;
+    return g;
+}
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+// Lane l's max over the lanes of equal l % 16 of m_(l / 16): the maxima of
+// the four rows' values, row r keeping that of m_r (two row swaps).
+PG_DEV int rows_max_scatter(int m0, int m1, int m2, int m3) {
+    const auto a = __builtin_amdgcn_permlane32_swap((uint32_t)m0, (uint32_t)m2, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)m1, (uint32_t)m3, false, false);
+    const int x = max((int)a[0], (int)a[1]), y = max((int)b[0], (int)b[1]);
+    const auto c = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y, false, false);
+    return max((int)c[0], (int)c[1]);
+}
+
 // Exact mode (fa.key set, or EXACT): a conflict test is trusted in floating
 // point only above XTOL times the product of its rows' 1-norms (w measured
 // by the magnitude its rounding is relative to), a valid bound on how far the
@@ -506,18 +565,19 @@ template <int DIM, int G, int S, bool EXACT = false, bool BALL = false>
 __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, const uint32_t* __restrict__ seeds,
                               int64_t nq, const uint32_t* __restrict__ knn, int k, int max_p,
                               int max_t, FaceArrays fa,
-                              SeedSmem<VoroCfg<DIM, G, S>::NS, VoroCfg<DIM, G, S>::MAXP>* smem,
+                              VoroSmem<DIM, G, S>* smem,
                               int64_t vblock, BallGrid bg = {}) {
     using C = VoroCfg<DIM, G, S>;
     constexpr int NS = C::NS, NW = C::NW, MAXP = C::MAXP;
     constexpr int D = DIM;
+    constexpr bool SKIP = !EXACT && G == 16;  // row entries may be passed over
     const int tid = (int)threadIdx.x;
     const int grp = tid / G, gl = tid % G;
     const int shift = grp * G;
     const uint64_t gmask = (G == 64) ? ~0ull : ((1ull << G) - 1ull);
     const int64_t qi = vblock * C::SPW + grp;
     const bool valid = qi < nq;
-    SeedSmem<NS, MAXP>& sm = smem[grp];
+    VoroSmem<DIM, G, S>& sm = smem[grp];
     if (max_p > FACE_SLOTS) max_p = FACE_SLOTS;
     // exact mode (a build with the exact-predicate fallback): every test
     // whose sign the rounding of the planes could flip is decided exactly
@@ -549,7 +609,6 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
         for (int p = gl; p < nb_v0; p += G) {
             sm.plane[p] = cst->plane[p];
             sm.pn1[p] = cst->pn1[p];
-            sm.pmx[p] = cst->pmx[p];
             sm.pvid[p] = cst->pvid[p];
         }
 #pragma unroll
@@ -573,7 +632,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
             default: p = {0.0, 0.0, -1.0, hi}; break;
         }
         sm.plane[gl] = p;
-        plane_bounds<D>(p, fabs(p.w), sm.pn1[gl], sm.pmx[gl]);
+        sm.pn1[gl] = plane_n1(p, fabs(p.w));
         sm.pvid[gl] = -1;
     }
     // Initial vertices (cell.cpp:84-103).
@@ -599,38 +658,27 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
         R.px[s] = R.py[s] = R.pz[s] = R.pw[s] = R.d2[s] = 0.0;
         R.q[s] = R.e5[s] = 0.f;
     }
-    // resumed cell: vertex numerics from the saved planes, with the same
-    // arithmetic (and operand order) as when the vertices were made
+    // vertex numerics of slot i from its planes (of a resumed cell: with the
+    // same arithmetic and operand order as when the vertex was made)
+    auto slot_from_planes = [&](int i, uint32_t t) {
+        const int ia = tri_p(t, 0), ib = tri_p(t, 1), ic = D == 3 ? tri_p(t, 2) : tri_p(t, 1);
+        double px, py, pz, pw, d2;
+        vertex_numerics<D>(sm.plane[ia], sm.plane[ib], sm.plane[ic], sx, sy, sz, px, py, pz, pw, d2);
+        const float na = sm.pn1[ia], nb = sm.pn1[ib], nc = sm.pn1[ic];
+        const float q = (D == 3 ? na * nb * nc : na * nb) * 1.000001f;
+        slot_write<D, S>(R, i, px, py, pz, pw, d2, q, eps_bound<D>(fmaxf(fmaxf(na, nb), nc)));
+    };
     if (v0) {
 #pragma unroll
         for (int i = 0; i < S; i++) {
             const uint32_t t = sm.tri[i * G + gl];
-            if (t == 0xffffffffu) continue;
-            const Plane& a = sm.plane[tri_p(t, 0)];
-            const Plane& b = sm.plane[tri_p(t, 1)];
-            const Plane& c = sm.plane[D == 3 ? tri_p(t, 2) : tri_p(t, 1)];
-            double px, py, pz, pw, d2;
-            vertex_numerics<D>(a, b, c, sx, sy, sz, px, py, pz, pw, d2);
-            float q = D == 3 ? sm.pn1[tri_p(t, 0)] * sm.pn1[tri_p(t, 1)] * sm.pn1[tri_p(t, 2)]
-                             : sm.pn1[tri_p(t, 0)] * sm.pn1[tri_p(t, 1)];
-            float m = fmaxf(sm.pmx[tri_p(t, 0)], sm.pmx[tri_p(t, 1)]);
-            if (D == 3) m = fmaxf(m, sm.pmx[tri_p(t, 2)]);
-            slot_write<D, S>(R, i, px, py, pz, pw, d2, q * 1.000001f, m);
+            if (t != 0xffffffffu) slot_from_planes(i, t);
         }
     }
     // NV0 <= G: initial vertex j lives in slot 0 of lane j.
     if (!v0 && gl < NV0) {
-        uint32_t t = sm.tri[gl];
-        const Plane& a = sm.plane[tri_p(t, 0)];
-        const Plane& b = sm.plane[tri_p(t, 1)];
-        const Plane& c = sm.plane[D == 3 ? tri_p(t, 2) : tri_p(t, 1)];
-        double px, py, pz, pw, d2;
-        vertex_numerics<D>(a, b, c, sx, sy, sz, px, py, pz, pw, d2);
-        float q = D == 3 ? sm.pn1[tri_p(t, 0)] * sm.pn1[tri_p(t, 1)] * sm.pn1[tri_p(t, 2)]
-                         : sm.pn1[tri_p(t, 0)] * sm.pn1[tri_p(t, 1)];
-        float m = fmaxf(sm.pmx[tri_p(t, 0)], sm.pmx[tri_p(t, 1)]);
-        if (D == 3) m = fmaxf(m, sm.pmx[tri_p(t, 2)]);
-        slot_write<D, S>(R, 0, px, py, pz, pw, d2, q * 1.000001f, m);
+        const uint32_t t = sm.tri[gl];
+        slot_from_planes(0, t);
         // adjacency of the initial polytope
         for (int e = 0; e < D; e++) {
             uint8_t nb = END;
@@ -666,6 +714,11 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
         if ((R.live >> s) & 1u) R2 = smax(R.d2[s], R2);
     R2 = group_butterfly_d<G>(R2, [](double a, double b) { return smax(a, b); });
 
+    // Row entries may be passed over without the conflict test only while
+    // every live vertex is good (vertex_good): nb_skip, per group.
+    SkipBounds win = {0.f, 0.f, 0.f};
+    bool nb_skip = true;
+
     // One clip of the cell by the bisector of neighbour z at (bx, by, bz)
     // (act: this group clips in this step; every lane of the wave calls it):
     // new plane, conflict test of every live vertex, cavity, consistency and
@@ -673,7 +726,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
     auto clip_step = [&](bool act, uint32_t z, double bx, double by, double bz) -> bool {
             // -- new half plane (cell.cpp:158-172)
             Plane e = {0, 0, 0, 0};
-            double ewm = 0.0;  // magnitude of e.w for the bounds (see plane_bounds)
+            double en1 = 0.0;  // 1-norm of e for the bounds (see plane_n1)
             bool plane_ok = false;
             int cur = 0;
             if (act) {
@@ -686,12 +739,13 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                     double ax = sx + bx, ay = sy + by, az = sz + bz;
                     double dot = ax * dx + ay * dy + az * dz;
                     e = {dx, dy, dz, -dot / 2.0};
-                    ewm = xmode ? 0.5 * (fabs(ax * dx) + fabs(ay * dy) + fabs(az * dz)) : fabs(e.w);
+                    const double ewm = xmode ? 0.5 * (fabs(ax * dx) + fabs(ay * dy) + fabs(az * dz)) : fabs(e.w);
+                    en1 = fabs(e.x) + fabs(e.y) + fabs(e.z) + ewm;
                     cur = nb_v;
                     plane_ok = true;
                     if (gl == 0) {
                         sm.plane[cur] = e;
-                        plane_bounds<D>(e, ewm, sm.pn1[cur], sm.pmx[cur]);
+                        sm.pn1[cur] = f2f_up(en1);
                         sm.pvid[cur] = (int32_t)z;
                     }
                     nb_v++;
@@ -701,19 +755,18 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
             uint32_t rem = 0;
             bool flag = false;
             if (act && plane_ok) {
-                const double en1 = (fabs(e.x) + fabs(e.y) + fabs(e.z) + ewm) * (1.0 + 1e-15);
-                const double emx = D == 2 ? fmax(fmax(fabs(e.x), fabs(e.y)), fabs(e.w))
-                                          : fmax(fmax(fabs(e.x), fabs(e.y)), fabs(e.z));
                 // per plane: the eps bound of its own components, and the
                 // rounding bound's factor (exact mode: below XTOL en1 q the
                 // rounding of the planes themselves may flip the sign, which
                 // the reference's eps does not bound; such tests go to the
                 // exact predicate)
-                const uint32_t e_eps = __float_as_uint(fmaxf(f2f_up(eps_bound<D>(emx)), 1.17549435e-38f));
-                const double c1 = (5.4e-15 + (xmode ? XTOL : 0.0)) * en1;
+                const uint32_t e_eps = __float_as_uint(eps_bound<D>(f2f_up(en1)));
+                const double en1s = en1 * (1.0 + 1e-15);
+                const double c1 = (5.4e-15 + (xmode ? XTOL : 0.0)) * en1s;
     #pragma unroll
                 for (int s = 0; s < S; s++) {
-                    if (!((R.live >> s) & 1u)) continue;
+                    const bool lv = (R.live >> s) & 1u;
+                    if (wave_ballot(lv) == 0ull || !lv) continue;  // levels no lane uses cost a branch
                     double t;
                     if (D == 3)
                         t = R.pw[s] * fma(e.x, R.px[s], fma(e.y, R.py[s], fma(e.z, R.pz[s], e.w)));
@@ -727,7 +780,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                     if (fabs(t) > bnd) {
                         c = t > 0.0;
                     } else {
-                        const double xb = xmode ? XTOL * en1 * (double)R.q[s] : 0.0;
+                        const double xb = xmode ? XTOL * en1s * (double)R.q[s] : 0.0;
                         uint32_t tt = sm.tri[s * G + gl];
                         const Plane p1 = sm.plane[tri_p(tt, 0)];
                         const Plane p2 = sm.plane[tri_p(tt, 1)];
@@ -749,9 +802,9 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                 }
             }
             // -- group masks
-            uint64_t Rm[NW], Lm[NW];
+            uint64_t Rm[NW];
     #pragma unroll
-            for (int w = 0; w < NW; w++) Rm[w] = Lm[w] = 0ull;
+            for (int w = 0; w < NW; w++) Rm[w] = 0ull;
     #pragma unroll
             for (int s = 0; s < S; s++) {
                 uint64_t b = (wave_ballot((rem >> s) & 1u) >> shift) & gmask;
@@ -824,13 +877,6 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                         j++;
                     }
                 }
-                // live mask of the group (after removal)
-    #pragma unroll
-                for (int s = 0; s < S; s++) {
-                    uint64_t b = (wave_ballot((R.live >> s) & 1u) >> shift) & gmask;
-                    int pos = s * G;
-                    Lm[pos >> 6] |= b << (pos & 63);
-                }
                 block_sync();
                 // -- consistency and capacity
                 bool ok = doclip;
@@ -881,10 +927,11 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                         }
                     }
                 }
-                bad = ((wave_ballot(bad) >> shift) & gmask) != 0ull;
+                const bool gbad = ((wave_ballot(bad) >> shift) & gmask) != 0ull;
+                bad = false;  // from here: a new vertex no skip can pass (see vertex_good)
                 if (doclip) {
                     const int nl_after = nlive - nb_r + Bt;
-                    if (bad) {
+                    if (gbad) {
                         status = INCONSISTENT_BOUNDARY;
                         ok = false;
                     } else if (nl_after >= max_t) {
@@ -896,43 +943,57 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                     }
                     nlive -= nb_r;
                 }
-                // -- slots of the new vertices: the j-th boundary edge takes the
-                //    j-th free slot (slot-id order)
+                // -- slots of the new vertices: round by round, each lane with a
+                //    free slot left offers its lowest one, and the boundary
+                //    edges take the offers lowest level first (one round, one
+                //    new vertex per lane, unless lanes are full); the edge of
+                //    a slot waits in its tri entry
                 uint32_t asg = 0;
-                if (ok) {
+                {
+                    uint32_t fr = ok ? ~R.live & ((1u << S) - 1u) : 0u;
+                    int base = 0;
+                    for (;;) {
+                        const int fl = fr ? __builtin_ctz(fr) : S;
+                        int r = base, tot = 0;
     #pragma unroll
-                    for (int s = 0; s < S; s++) {
-                        const int gs = s * G + gl;
-                        if ((R.live >> s) & 1u) continue;
-                        // free-slot rank = gs - (live slots below gs)
-                        int r = gs - mask_rank<NW>(Lm, gs);
-                        if (r < Bt) {
-                            sm.newslot[r] = (uint8_t)gs;
-                            asg |= 1u << s;
+                        for (int s = 0; s < S; s++) {
+                            const uint64_t b = (wave_ballot(fl == s) >> shift) & gmask;
+                            const int c = popc64(b);
+                            if (s < fl) r += c;
+                            else if (s == fl) r += popc64(b & ((1ull << gl) - 1ull));
+                            tot += c;
                         }
+                        if (fr && r < Bt) {
+                            const int gs = fl * G + gl;
+                            sm.newslot[r] = (uint8_t)gs;
+                            sm.tri[gs] = (uint32_t)r;
+                            asg |= 1u << fl;
+                        }
+                        fr &= fr - 1u;
+                        base += tot;
+                        if (wave_ballot(ok && base < Bt) == 0ull) break;
                     }
                 }
                 block_sync();
                 // -- new vertices (cell.cpp:346-364 orientation, :388-411 position)
                 if (ok) {
-                    float cn1, cmx;
-                    plane_bounds<D>(e, ewm, cn1, cmx);
+                    const float cn1 = f2f_up(en1);
                     while (asg) {
                         const int s = ffs64(asg);
                         asg &= asg - 1;
                         const int gs = s * G + gl;
-                        const int r = gs - mask_rank<NW>(Lm, gs);
+                        const int r = (int)sm.tri[gs];
                         const uint32_t ed = sm.edge[r];
                         uint32_t t;
                         Plane pa, pb;
-                        float q, m;
                         if (D == 3) {
                             const int a = ed & 0xff, b = (ed >> 8) & 0xff, K = (ed >> 16) & 0xff;
                             t = (uint32_t)cur | (uint32_t)a << 8 | (uint32_t)b << 16;
                             pa = sm.plane[a];
                             pb = sm.plane[b];
-                            q = cn1 * sm.pn1[a] * sm.pn1[b] * 1.000001f;
-                            m = fmaxf(cmx, fmaxf(sm.pmx[a], sm.pmx[b]));
+                            const float na = sm.pn1[a], nb = sm.pn1[b];
+                            const float q = cn1 * na * nb * 1.000001f;
+                            const float e5 = eps_bound<D>(fmaxf(cn1, fmaxf(na, nb)));
                             sm.tri[gs] = t;
                             sm.adj[0][gs] = sm.newslot[sm.by_end[a]];
                             sm.adj[1][gs] = (uint8_t)K;
@@ -942,7 +1003,8 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                                 if (tri_p(tk, f) == b && tri_p(tk, (f + 1) % 3) == a) sm.adj[f][K] = (uint8_t)gs;
                             double px, py, pz, pw, d2;
                             vertex_numerics<D>(e, pa, pb, sx, sy, sz, px, py, pz, pw, d2);
-                            slot_write<D, S>(R, s, px, py, pz, pw, d2, q, m);
+                            slot_write<D, S>(R, s, px, py, pz, pw, d2, q, e5);
+                            bad = bad || !vertex_good(win, pw, q, e5);
                         } else {
                             const int L = ed & 0xff, K = (ed >> 16) & 0xff;
                             pa = sm.plane[L];
@@ -956,60 +1018,136 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                             const uint32_t tk = sm.tri[K];
                             for (int f = 0; f < 2; f++)
                                 if (tri_p(tk, f) == L) sm.adj[f][K] = (uint8_t)gs;
-                            q = cn1 * sm.pn1[L] * 1.000001f;
-                            m = fmaxf(cmx, sm.pmx[L]);
+                            const float nL = sm.pn1[L];
+                            const float q = cn1 * nL * 1.000001f;
+                            const float e5 = eps_bound<D>(fmaxf(cn1, nL));
                             double px, py, pz, pw, d2;
                             if (swap)
                                 vertex_numerics<D>(pa, e, e, sx, sy, sz, px, py, pz, pw, d2);
                             else
                                 vertex_numerics<D>(e, pa, pa, sx, sy, sz, px, py, pz, pw, d2);
-                            slot_write<D, S>(R, s, px, py, pz, pw, d2, q, m);
+                            slot_write<D, S>(R, s, px, py, pz, pw, d2, q, e5);
+                            bad = bad || !vertex_good(win, pw, q, e5);
                         }
                     }
                     nlive += Bt;
                 }
+                if (((wave_ballot(bad) >> shift) & gmask) != 0ull) nb_skip = false;
                 block_sync();
             }
         return anyclip;
     };
 
     // --------------------------------------------------------- clip loop
-    // Seeds of a wave may start at different neighbours (resumed cells):
-    // the wave walks v from the smallest start, a group joins at its own.
-    int vstart = v0;
+    // The group walks its row in windows of G entries, one per lane.
+    // Every window entry that may cut the cell is clipped in row order; the
+    // others are passed over (window_filter).  Passing over an entry leaves
+    // the cell as it is, so the certificate of a passed entry is judged with
+    // the R2 of the last clip, all entries of the window at once.  Seeds of a
+    // wave walk their own windows: every step of the wave clips a candidate
+    // of each of its seeds.
+    const int cap_v = max_p < MAXP ? max_p : MAXP;
+    int wb = v0;                 // row entry of the window's lane 0
+    uint32_t pend = 0, cand = 0; // window entries ahead; of those, the ones to clip
+    double wd2 = 0.0;            // this lane's entry: squared distance, float offset
+    float wx = 0.f, wy = 0.f, wz = 0.f;
+    bool first = true;
+    int since = 0;
+    // entries of the window ahead whose bisector may cut the cell: the
+    // others keep every live vertex on the seed's side by a margin
+    auto window_filter = [&]() {
+        float mx = 0.f;  // largest offset . vertex of this lane's entry (the seed as origin)
+        bool vbad = false;
+        if constexpr (G == 16) {
+            // offsets (columns) times vertices (rows) of the wave's four
+            // seeds, one 16 x 16 block per seed and slot level, on the
+            // matrix cores: entry (i, j) of block b sits in register 4 b +
+            // i % 4 of lane 16 (i / 4) + j
+            // (maxima of at least 0 as signed integers: no NaN handling)
+            int m4[4] = {0, 0, 0, 0};
 #pragma unroll
-    for (int d = G; d < 64; d <<= 1) vstart = min(vstart, __shfl_xor(vstart, d, 64));
-    int cbase = -NB_CHUNK;  // first neighbour of the prefetched chunk
-    for (int v = vstart; v < k; v++) {
-        if (wave_ballot(!done) == 0ull) break;
-        const bool act = !done && v >= v0;
-        // the group prefetches the next NB_CHUNK neighbours and their
-        // positions into LDS, so the clip loop issues no dependent global loads
-        if (v >= cbase + NB_CHUNK) {
-            cbase = v;
-            for (int j = gl; j < NB_CHUNK; j += G) {
-                // a resumed group reads only its row from v0 on: the entries
-                // before are not written by a KNN launch that resumes too
-                if (!done && v + j < k && v + j >= v0) {
-                    const uint32_t zz = row[v + j];
-                    sm.nbi[j] = zz;
+            for (int s = 0; s < S; s++) {
+                const bool lv = (R.live >> s) & 1u;
+                if (wave_ballot(lv) == 0ull) continue;
+                vbad = vbad || (lv && !vertex_good(win, R.pw[s], R.q[s], R.e5[s]));
+                f32x16 c = {0.f};
+                c = __builtin_amdgcn_mfma_f32_16x16x1f32(lv ? (float)(R.px[s] - sx) : 0.f, wx, c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x1f32(lv ? (float)(R.py[s] - sy) : 0.f, wy, c, 0, 0, 0);
+                if (D == 3) c = __builtin_amdgcn_mfma_f32_16x16x1f32(lv ? (float)(R.pz[s] - sz) : 0.f, wz, c, 0, 0, 0);
 #pragma unroll
-                    for (int d = 0; d < D; d++) sm.nbp[j][d] = pts[(size_t)D * zz + d];
-                }
+                for (int b = 0; b < 4; b++)
+                    m4[b] = max(max(max(m4[b], __float_as_int(c[4 * b])), max(__float_as_int(c[4 * b + 1]), __float_as_int(c[4 * b + 2]))),
+                                __float_as_int(c[4 * b + 3]));
             }
-            block_sync();
+            mx = __int_as_float(rows_max_scatter(m4[0], m4[1], m4[2], m4[3]));
         }
-        // the step's neighbour: the prefetched row entry
+        const float h = wx * wx + wy * wy + wz * wz;
+        const float slack = 2e-6f * (fabsf(wx) + fabsf(wy) + fabsf(wz)) * __builtin_amdgcn_sqrtf((float)R2 * 1.001f);
+        const bool cut = !(mx < h * (0.5f - SKIP_MARGIN) - slack);
+        const uint32_t cm = (uint32_t)((wave_ballot(cut) >> shift) & gmask);
+        const bool gb = ((wave_ballot(vbad) >> shift) & gmask) != 0ull;
+        nb_skip = !gb;
+        cand = gb || nb_v >= cap_v ? pend : pend & cm;
+        since = 0;
+    };
+    for (;;) {
+        if (!BALL) {
+            const uint32_t cm = (uint32_t)((wave_ballot(wd2 > 4 * R2) >> shift) & gmask) & pend;
+            if (!done && cm != 0u && (cand == 0u || __builtin_ctz(cm) < __builtin_ctz(cand))) {
+                kc = wb + __builtin_ctz(cm) + 1;
+                done = true;
+            }
+        }
+        if (wave_ballot(!done && cand == 0u) != 0ull) {
+            // a seed has passed its window: every seed's next one
+            if (!done) {
+                if (!first) wb += cand != 0u ? __builtin_ctz(cand) : G;
+                if (wb >= k) done = true;
+            }
+            pend = done ? 0u : (uint32_t)((1ull << min(G, k - wb)) - 1ull);
+            cand = pend;
+            wd2 = 0.0;
+            wx = wy = wz = 0.f;
+            if ((pend >> gl) & 1u) {
+                const uint32_t zz = row[wb + gl];
+                double bp[3] = {0, 0, 0};
+                sm.nbi[gl] = zz;
+#pragma unroll
+                for (int d = 0; d < D; d++) sm.nbp[gl][d] = bp[d] = pts[(size_t)D * zz + d];
+                const double dx = bp[0] - sx, dy = bp[1] - sy, dz = D == 3 ? bp[2] - sz : 0.0;
+                wd2 = dx * dx + dy * dy + dz * dz;
+                wx = (float)dx;
+                wy = (float)dy;
+                wz = (float)dz;
+            }
+            win = window_bounds<D, G>(wd2, pend, sx, sy, sz);
+            block_sync();
+            if (wave_ballot(!done) == 0ull) break;
+            if (SKIP && !xmode && !first) window_filter();
+            first = false;
+            continue;
+        }
+        if (wave_ballot(!done) == 0ull) break;
+        if (SKIP && !xmode && since >= REFILTER) {
+            window_filter();
+            continue;
+        }
+        const bool act = !done;
+        // the step's neighbour
         uint32_t z = 0;
         double bx = 0, by = 0, bz = 0;
+        int j = 0;
         if (act) {
-            const int jj = v - cbase;
-            z = sm.nbi[jj];
-            bx = sm.nbp[jj][0];
-            by = sm.nbp[jj][1];
-            bz = D == 3 ? sm.nbp[jj][2] : 0.0;
+            j = __builtin_ctz(cand);
+            pend &= ~((2u << j) - 1u);
+            cand &= pend;
+            z = sm.nbi[j];
+            bx = sm.nbp[j][0];
+            by = sm.nbp[j][1];
+            bz = D == 3 ? sm.nbp[j][2] : 0.0;
         }
         const bool anyclip = clip_step(act, z, bx, by, bz);
+        since++;
         // -- certificate (cell.cpp:369-384) with the just-clipped neighbour;
         //    the largest seed-vertex distance only changes with a clip
         double mx = R2;
@@ -1028,11 +1166,12 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                 if (!EXACT && xmode && status == SUCCESS && !(dz2 > 4 * R2 * CERT_TIE)) {
                     status = NEEDS_EXACT_PREDICATES;  // a near tie: the exact kernel decides
                 } else {
-                    kc = v + 1;
+                    kc = wb + j + 1;
                     done = true;
                 }
             }
             if (status != SUCCESS) done = true;
+            if (!nb_skip || nb_v >= cap_v) cand = pend;
         }
     }
 
@@ -1159,7 +1298,6 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
             for (int p = gl; p < nb_v; p += G) {
                 out->plane[p] = sm.plane[p];
                 out->pn1[p] = sm.pn1[p];
-                out->pmx[p] = sm.pmx[p];
                 out->pvid[p] = sm.pvid[p];
             }
 #pragma unroll
