@@ -234,16 +234,7 @@ __global__ void __launch_bounds__(BLOCK)
 // item, read it again from the kernel-argument segment through a pointer
 // the compiler must treat as new each time: loop-invariant arguments would
 // otherwise be hoisted out of the item loop and stay live across it, and
-// the item's own registers would spill.  The struct is the kernel's only
-// explicit argument, so it starts the segment.
-template <class A>
-PG_DEV const __attribute__((address_space(4))) A* fresh_args() {
-    const __attribute__((address_space(4))) A* p =
-        (const __attribute__((address_space(4))) A*)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return p;
-}
-
+// the item's own registers would spill (fresh_args).
 struct BKnnArgs {
     const double* sorted;
     const uint32_t* perm;
@@ -299,53 +290,22 @@ __global__ void __launch_bounds__(64, (M <= 2 ? 6 : 5)) k_bknn_wave(BKnnArgs arg
 // across groups, and the clip's registers spill: it suits the short lists
 // of the certificate restarts, where capacity-sized grids would be mostly
 // empty blocks).
-struct BClipArgs {
-    const double* pts;
-    const uint32_t* seeds;
-    const int64_t* nq_dev;
-    const uint32_t* knn;
-    unsigned long long* ticket;
-    FaceArrays fa;
-    int k, max_p, max_t;
-};
-
-// a FaceArrays out of the argument segment, field by field
-PG_DEV FaceArrays face_arrays_of(const __attribute__((address_space(4))) FaceArrays& a) {
-    FaceArrays f;
-    f.stride = a.stride;
-    f.nbr = a.nbr;
-    f.area = a.area;
-    f.nrm = a.nrm;
-    f.cen = a.cen;
-    f.count = a.count;
-    f.vol = a.vol;
-    f.ccen = a.ccen;
-    f.status = a.status;
-    f.kcert = a.kcert;
-    f.cstate = a.cstate;
-    f.resume = a.resume;
-    f.lastnb = a.lastnb;
-    f.key = a.key;
-    f.nbr_cm = a.nbr_cm;
-    return f;
-}
-
 // FRESH: the arguments are re-read per group (3D: fewer spills); else they
 // stay in registers across groups (2D, whose clip has room for them).
 template <int DIM, int G, int S, bool FRESH>
-__global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_bvoronoi_loop(BClipArgs args) {
+__global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_bvoronoi_loop(ClipArgs args) {
     using C = VoroCfg<DIM, G, S>;
     __shared__ VoroSmem<DIM, G, S> sm[C::SPW];
     if constexpr (FRESH) {
         bool first = true;
         for (;;) {
-            const auto* A0 = fresh_args<BClipArgs>();
+            const auto* A0 = fresh_args<ClipArgs>();
             const int64_t nvb = (*A0->nq_dev + C::SPW - 1) / C::SPW;
             const int64_t vb = next_ticket(A0->ticket, 1, first);
             if (vb >= nvb) break;
-            const auto* A = fresh_args<BClipArgs>();
+            const auto* A = fresh_args<ClipArgs>();
             voronoi_group<DIM, G, S>(A->pts, INT64_MAX, A->seeds, *A->nq_dev, A->knn, A->k, A->max_p, A->max_t,
-                                     face_arrays_of(A->fa), sm, vb);
+                                     A->fa.resume, A->fa.cstate, A->fa.key, sm, vb);
             __syncthreads();
         }
     } else {
@@ -359,7 +319,7 @@ __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_bvoronoi_lo
             const int64_t b1 = b0 + chunk < nvb ? b0 + chunk : nvb;
             for (int64_t vb = b0; vb < b1; vb++) {
                 voronoi_group<DIM, G, S>(args.pts, INT64_MAX, args.seeds, nq, args.knn, args.k, args.max_p,
-                                         args.max_t, args.fa, sm, vb);
+                                         args.max_t, args.fa.resume, args.fa.cstate, args.fa.key, sm, vb);
                 __syncthreads();
             }
         }
@@ -368,15 +328,15 @@ __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_bvoronoi_lo
 
 template <int DIM, int G, int S>
 __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES))
-    k_bvoronoi(const double* __restrict__ pts, const uint32_t* __restrict__ seeds, const int64_t* __restrict__ nq_dev,
-               const uint32_t* __restrict__ knn, int k, int max_p, int max_t, FaceArrays fa) {
+    k_bvoronoi(ClipArgs args) {
     using C = VoroCfg<DIM, G, S>;
     __shared__ VoroSmem<DIM, G, S> sm[C::SPW];
-    const int64_t nq = *nq_dev;
+    const int64_t nq = *args.nq_dev;
     const int64_t vb = blockIdx.x;
     if (vb * C::SPW >= nq) return;  // whole block
     // no box holds k + 1 seeds or fewer: the exhaustive-row rule never applies
-    voronoi_group<DIM, G, S>(pts, INT64_MAX, seeds, nq, knn, k, max_p, max_t, fa, sm, vb);
+    voronoi_group<DIM, G, S>(args.pts, INT64_MAX, args.seeds, nq, args.knn, args.k, args.max_p, args.max_t,
+                             args.fa.resume, args.fa.cstate, args.fa.key, sm, vb);
 }
 
 // status == code (code < 0: != SUCCESS) among the listed seeds
@@ -638,18 +598,18 @@ void bclip(const double* pts, const uint32_t* seeds, const int64_t* nq_dev, int6
            int max_p, int max_t, FaceArrays fa, int blocks_per_cu, unsigned long long* ticket, bool loop,
            hipStream_t s) {
     using C = VoroCfg<DIM, G, S>;
+    const ClipArgs args{pts, INT64_MAX, seeds, 0, nq_dev, knn, ticket, fa, k, max_p, max_t};
     if (loop) {
         constexpr bool FRESH = DIM == 3;
         static const int occ = occupancy(k_bvoronoi_loop<DIM, G, S, FRESH>);
         const unsigned nb =
             (unsigned)std::min<int64_t>((cap + C::SPW - 1) / C::SPW, resident_blocks(occ, blocks_per_cu));
         k_fill<unsigned long long><<<1, TB, 0, s>>>(ticket, 1, 0ull);
-        const BClipArgs args{pts, seeds, nq_dev, knn, ticket, fa, k, max_p, max_t};
         k_bvoronoi_loop<DIM, G, S, FRESH><<<std::max(nb, 1u), 64, 0, s>>>(args);
         return;
     }
     const unsigned nb = (unsigned)std::max<int64_t>((cap + C::SPW - 1) / C::SPW, 1);
-    k_bvoronoi<DIM, G, S><<<nb, 64, 0, s>>>(pts, seeds, nq_dev, knn, k, max_p, max_t, fa);
+    k_bvoronoi<DIM, G, S><<<nb, 64, 0, s>>>(args);
 }
 }  // namespace
 

@@ -115,7 +115,7 @@ struct FaceArrays {
 constexpr int FACE_SLOTS = 64;
 
 // Saved clip state of one seed (64 planes, up to 64 vertex slots).
-constexpr int64_t CLIP_STATE_BYTES = 3328;
+constexpr int64_t CLIP_STATE_BYTES = 3104;
 
 // Clip + certify + extract the seeds listed in `seeds` (sorted ids; nullptr
 // = all n) with their neighbour rows knn[row q] (row q belongs to seeds[q]).

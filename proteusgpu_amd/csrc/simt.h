@@ -84,6 +84,20 @@ __device__ __forceinline__ double group_butterfly_d(double x, F op) {
     if constexpr (G >= 16) x = op(lane_xor_d<8>(x), x);
     return x;
 }
+// Maximum of non-negative floats over groups of G <= 16 lanes (as integers,
+// which order like them), every lane active.
+template <int G>
+__device__ __forceinline__ float group_max_f(float v) {
+    static_assert(G == 1 || G == 2 || G == 4 || G == 8 || G == 16, "group of 1..16 lanes");
+    int x = __builtin_bit_cast(int, v);
+    if constexpr (G >= 2) x = max(x, __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false));    // ^ 1
+    if constexpr (G >= 4) x = max(x, __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false));    // ^ 2
+    if constexpr (G >= 8) x = max(x, __builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, false));   // half row mirror
+    if constexpr (G >= 16) x = max(x, __builtin_amdgcn_mov_dpp(x, 0x140, 0xF, 0xF, false));  // row mirror
+    return __builtin_bit_cast(float, x);
+}
+// Sum of the four bytes.
+__device__ __forceinline__ uint32_t byte_sum(uint32_t x) { return __builtin_amdgcn_sad_u8(x, 0u, 0u); }
 // Inclusive prefix sum inside groups of G <= 16 lanes (gl = lane index in
 // its group), every lane active: row shifts by DPP, kept only where the
 // source lane lies in the same group.

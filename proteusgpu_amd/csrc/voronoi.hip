@@ -12,65 +12,47 @@ namespace {
 // wave.  Large kernel: 16 lanes x 8 slots = 128 slots, for seeds whose cell
 // outgrows 64 vertices before max_t (rare).
 template <int DIM, int G, int S>
-__global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_voronoi(const double* __restrict__ pts, int64_t n_total,
-                                                const uint32_t* __restrict__ seeds, int64_t nq,
-                                                const uint32_t* __restrict__ knn, int k, int max_p,
-                                                int max_t, FaceArrays fa) {
-    using C = VoroCfg<DIM, G, S>;
-    __shared__ VoroSmem<DIM, G, S> sm[C::SPW];
-    voronoi_group<DIM, G, S>(pts, n_total, seeds, nq, knn, k, max_p, max_t, fa, sm,
-                             xcd_block(blockIdx.x, gridDim.x));
+__global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_voronoi(ClipArgs a) {
+    __shared__ VoroSmem<DIM, G, S> sm[VoroCfg<DIM, G, S>::SPW];
+    voronoi_group<DIM, G, S>(a.pts, a.n_total, a.seeds, a.nq, a.knn, a.k, a.max_p, a.max_t, a.fa.resume, a.fa.cstate,
+                             a.fa.key, sm, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // The same kernel under its own name for certificate restarts, so that
 // profiles separate the first pass from the restarts.
 template <int DIM, int G, int S>
-__global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_voronoi_restart(const double* __restrict__ pts, int64_t n_total,
-                                                        const uint32_t* __restrict__ seeds, int64_t nq,
-                                                        const uint32_t* __restrict__ knn, int k, int max_p,
-                                                        int max_t, FaceArrays fa) {
-    using C = VoroCfg<DIM, G, S>;
-    __shared__ VoroSmem<DIM, G, S> sm[C::SPW];
-    voronoi_group<DIM, G, S>(pts, n_total, seeds, nq, knn, k, max_p, max_t, fa, sm,
-                             xcd_block(blockIdx.x, gridDim.x));
+__global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_voronoi_restart(ClipArgs a) {
+    __shared__ VoroSmem<DIM, G, S> sm[VoroCfg<DIM, G, S>::SPW];
+    voronoi_group<DIM, G, S>(a.pts, a.n_total, a.seeds, a.nq, a.knn, a.k, a.max_p, a.max_t, a.fa.resume, a.fa.cstate,
+                             a.fa.key, sm, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // Cells whose filtered predicate was degenerate, again with the exact
 // predicate (128 vertex slots).
 template <int DIM>
-__global__ void __launch_bounds__(64, 1) k_voronoi_exact(const double* __restrict__ pts, int64_t n_total,
-                                                         const uint32_t* __restrict__ seeds, int64_t nq,
-                                                         const uint32_t* __restrict__ knn, int k, int max_p,
-                                                         int max_t, FaceArrays fa) {
-    using C = VoroCfg<DIM, 16, 8>;
-    __shared__ VoroSmem<DIM, 16, 8> sm[C::SPW];
-    voronoi_group<DIM, 16, 8, true>(pts, n_total, seeds, nq, knn, k, max_p, max_t, fa, sm, blockIdx.x);
+__global__ void __launch_bounds__(64, 1) k_voronoi_exact(ClipArgs a) {
+    __shared__ VoroSmem<DIM, 16, 8> sm[VoroCfg<DIM, 16, 8>::SPW];
+    voronoi_group<DIM, 16, 8, true>(a.pts, a.n_total, a.seeds, a.nq, a.knn, a.k, a.max_p, a.max_t, a.fa.resume,
+                                    a.fa.cstate, a.fa.key, sm, blockIdx.x);
 }
 
 // Vertex-ball completion of seeds no row certifies (128 vertex slots).
 template <int DIM>
-__global__ void __launch_bounds__(64, 1) k_voronoi_ball(const double* __restrict__ pts, int64_t n_total,
-                                                        const uint32_t* __restrict__ seeds, int64_t nq,
-                                                        const uint32_t* __restrict__ knn, int k, int max_p,
-                                                        int max_t, FaceArrays fa, BallGrid bg) {
+__global__ void __launch_bounds__(64, 1) k_voronoi_ball(ClipArgs a, BallGrid bg) {
     using C = VoroCfg<DIM, 16, 8>;
     __shared__ VoroSmem<DIM, 16, 8> sm[C::SPW];
     __shared__ int32_t scr[C::SPW * (2 * 16 + 1)];
     bg.scr = scr;
-    voronoi_group<DIM, 16, 8, false, true>(pts, n_total, seeds, nq, knn, k, max_p, max_t, fa, sm, blockIdx.x, bg);
+    voronoi_group<DIM, 16, 8, false, true>(a.pts, a.n_total, a.seeds, a.nq, a.knn, a.k, a.max_p, a.max_t, a.fa.resume,
+                                           a.fa.cstate, a.fa.key, sm, blockIdx.x, bg);
 }
 
 template <int DIM, int G, int S>
-void run(const double* pts, int64_t n_total, const uint32_t* seeds, int64_t nq, const uint32_t* knn, int k,
-         int max_p, int max_t, FaceArrays fa, bool restart, hipStream_t s) {
+void run(const ClipArgs& a, bool restart, hipStream_t s) {
     using C = VoroCfg<DIM, G, S>;
-    int64_t nb = (nq + C::SPW - 1) / C::SPW;
-    if (restart)
-        k_voronoi_restart<DIM, G, S><<<dim3((unsigned)nb), dim3(64), 0, s>>>(pts, n_total, seeds, nq, knn, k,
-                                                                              max_p, max_t, fa);
-    else
-        k_voronoi<DIM, G, S><<<dim3((unsigned)nb), dim3(64), 0, s>>>(pts, n_total, seeds, nq, knn, k, max_p,
-                                                                      max_t, fa);
+    const unsigned nb = (unsigned)((a.nq + C::SPW - 1) / C::SPW);
+    if (restart) k_voronoi_restart<DIM, G, S><<<dim3(nb), dim3(64), 0, s>>>(a);
+    else k_voronoi<DIM, G, S><<<dim3(nb), dim3(64), 0, s>>>(a);
 }
 
 constexpr int TB = 256;
@@ -133,19 +115,15 @@ bool clip_resume() { return g_clip_resume; }
 void set_clip_resume(bool on) { g_clip_resume = on; }
 
 template <int DIM>
-void launch_dim(const double* sorted, int64_t n, const uint32_t* seeds, int64_t nq, const uint32_t* knn, int k,
-                int max_p, int max_t, int big, FaceArrays fa, hipStream_t s, bool restart, int lanes, int slots,
-                bool exact) {
+void launch_dim(const ClipArgs& a, int big, hipStream_t s, bool restart, int lanes, int slots, bool exact) {
     if (exact) {
         using C = VoroCfg<DIM, 16, 8>;
-        const int64_t nb = (nq + C::SPW - 1) / C::SPW;
-        k_voronoi_exact<DIM><<<dim3((unsigned)nb), dim3(64), 0, s>>>(sorted, n, seeds, nq, knn, k, max_p, max_t,
-                                                                      fa);
-    } else if (big) run<DIM, 16, 8>(sorted, n, seeds, nq, knn, k, max_p, max_t, fa, true, s);
-    else if (lanes == 8 && slots == 48) run<DIM, 8, 6>(sorted, n, seeds, nq, knn, k, max_p, max_t, fa, restart, s);
-    else if (lanes == 8) run<DIM, 8, 8>(sorted, n, seeds, nq, knn, k, max_p, max_t, fa, restart, s);
-    else if (slots == 48) run<DIM, 16, 3>(sorted, n, seeds, nq, knn, k, max_p, max_t, fa, restart, s);
-    else run<DIM, 16, 4>(sorted, n, seeds, nq, knn, k, max_p, max_t, fa, restart, s);
+        k_voronoi_exact<DIM><<<dim3((unsigned)((a.nq + C::SPW - 1) / C::SPW)), dim3(64), 0, s>>>(a);
+    } else if (big) run<DIM, 16, 8>(a, true, s);
+    else if (lanes == 8 && slots == 48) run<DIM, 8, 6>(a, restart, s);
+    else if (lanes == 8) run<DIM, 8, 8>(a, restart, s);
+    else if (slots == 48) run<DIM, 16, 3>(a, restart, s);
+    else run<DIM, 16, 4>(a, restart, s);
 }
 
 void launch_voronoi(int dim, const double* sorted, int64_t n, const uint32_t* seeds, int64_t nq,
@@ -153,10 +131,9 @@ void launch_voronoi(int dim, const double* sorted, int64_t n, const uint32_t* se
                     hipStream_t s, bool restart, bool exact) {
     if (nq <= 0) return;
     (void)g_clip_env;
-    if (dim == 2)
-        launch_dim<2>(sorted, n, seeds, nq, knn, k, max_p, max_t, big, fa, s, restart, lanes, slots, exact);
-    else
-        launch_dim<3>(sorted, n, seeds, nq, knn, k, max_p, max_t, big, fa, s, restart, lanes, slots, exact);
+    const ClipArgs a{sorted, n, seeds, nq, nullptr, knn, nullptr, fa, k, max_p, max_t};
+    if (dim == 2) launch_dim<2>(a, big, s, restart, lanes, slots, exact);
+    else launch_dim<3>(a, big, s, restart, lanes, slots, exact);
 }
 
 void launch_voronoi_ball(int dim, const double* sorted, int64_t n, const uint32_t* seeds, int64_t nq,
@@ -171,11 +148,10 @@ void launch_voronoi_ball(int dim, const double* sorted, int64_t n, const uint32_
     bg.perm = perm;
     bg.kmark = kmark;
     bg.sg = sg;
-    const int64_t nb = (nq + 3) / 4;  // 4 seeds per wave
-    if (dim == 2)
-        k_voronoi_ball<2><<<dim3((unsigned)nb), dim3(64), 0, s>>>(sorted, n, seeds, nq, knn, k, max_p, max_t, fa, bg);
-    else
-        k_voronoi_ball<3><<<dim3((unsigned)nb), dim3(64), 0, s>>>(sorted, n, seeds, nq, knn, k, max_p, max_t, fa, bg);
+    const unsigned nb = (unsigned)((nq + 3) / 4);  // 4 seeds per wave
+    const ClipArgs a{sorted, n, seeds, nq, nullptr, knn, nullptr, fa, k, max_p, max_t};
+    if (dim == 2) k_voronoi_ball<2><<<dim3(nb), dim3(64), 0, s>>>(a, bg);
+    else k_voronoi_ball<3><<<dim3(nb), dim3(64), 0, s>>>(a, bg);
 }
 
 void launch_collect_status(int64_t nq, const uint32_t* seeds, const int32_t* status, int code,

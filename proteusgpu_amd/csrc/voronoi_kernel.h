@@ -9,8 +9,9 @@
 // Layout on the GPU (differs from the reference, results do not):
 //   * a wave64 holds SPW = 64/G seeds, G lanes each; a lane owns S vertex
 //     slots, slot id gs = s*G + lane.  Per slot the lane keeps in registers
-//     the vertex position (px,py,pz), the Cramer denominator W, the squared
-//     seed distance d2 and two float bounds (q, m) used by the filter below.
+//     the vertex position, its squared seed distance and three float bounds
+//     used by the filter below; which slots are live, removed or on the
+//     cavity's rim are lane masks in scalar registers.
 //   * planes (FP64), plane->neighbour ids, vertex plane triples and the
 //     vertex adjacency (slot across each edge) live in LDS.
 //   * row entries are taken in windows of 16; the ones whose plane cannot
@@ -18,11 +19,12 @@
 //     making the 16 x vertices products of a window.
 //   * a clip tests every live vertex in parallel.  The reference decides
 //     with a 4x4 (3x3 in 2D) FP64 determinant per vertex; here
-//     det ~= W * (e . p + e.w) is evaluated from the cached vertex and used
-//     only when |det| exceeds a proven bound (48u |e|_1 q + eps bound, see
-//     conflict()); otherwise the reference determinant and its eps test are
-//     evaluated exactly as written.  Decisions and needs_exact_predicates
-//     flags are therefore identical to the reference.
+//     det ~= W * (e . p + e.w) is judged by its second factor, from the
+//     cached vertex, against the test's rounding and eps bound over |W|
+//     (SlotRegs, clip_step); a value below it goes to the reference
+//     determinant and its eps test, evaluated exactly as written.  Decisions
+//     and needs_exact_predicates flags are therefore identical to the
+//     reference.
 //   * the cavity boundary is found from the adjacency (an edge of a removed
 //     vertex whose neighbour is kept), in parallel over removed vertices,
 //     instead of the reference's serial walk; new vertices are the same
@@ -30,6 +32,15 @@
 //     positions and the certificate are bit-identical to the reference.
 //   * extraction walks each face's vertex cycle through the adjacency; face
 //     order is plane order as in the reference (box planes, then KNN order).
+//
+// What bounds it: VALU issue (87 % of the SIMD cycles at three waves per SIMD,
+// LDS 13.2 KB per wave).  At 1M uniform 3D seeds and k = 64 a wave of four
+// seeds takes 24 clip steps of about 500 VALU instructions, a fifth of them
+// the new vertices' Cramer rule, and 1.5k for the extraction: 16.0k in all,
+// 8.7 ms (k = 32: 7.4 ms).  With one conflict bound in double per test, slot
+// masks in vector registers, a loop per lane over its cavity edges, one
+// vector prefix per use and the extraction by plane index it was 19.9k
+// and 10.8 ms (9.3 ms).
 #pragma once
 
 #include "common.h"
@@ -71,8 +82,9 @@ struct SeedSmem {
     };
     float pn1[MAXP];        // |x|+|y|+|z|+|w| rounded up
     int32_t pvid[MAXP];     // neighbour (sorted id) of each plane, -1 = box
-    uint32_t tri[NS];       // planes of each vertex: a | b << 8 | c << 16
-    uint8_t adj[3][NS];     // neighbour slot across edge/line e
+    // per vertex x: its planes a | b << 8 | c << 16; y: the neighbour slots
+    // across its edges (lines in 2D), byte e across edge e
+    uint2 va[NS];
     union {
         struct {
             uint32_t edge[NS];        // boundary edges of the current clip
@@ -82,7 +94,10 @@ struct SeedSmem {
             uint32_t nbi[G];   // window of the neighbour row, one entry per lane
             double nbp[G][3];  // and the neighbours' positions
         };
-        uint32_t first[MAXP];  // extraction: vertex of each plane with the lowest plane key
+        struct {  // extraction
+            uint32_t first[MAXP];  // vertex of each plane with the lowest plane key
+            uint8_t plist[MAXP];   // planes holding a vertex, in plane order
+        };
     };
 };
 
@@ -96,6 +111,8 @@ PG_DEV float f2f_up(double d) {
     return f;
 }
 PG_DEV int tri_p(uint32_t t, int e) { return (int)((t >> (8 * e)) & 0xffu); }
+// write byte e of a vertex's adjacency
+PG_DEV void set_adj(uint2& v, int e, int slot) { reinterpret_cast<uint8_t*>(&v.y)[e] = (uint8_t)slot; }
 
 // Slot-independent identity of a vertex: its planes, sorted, packed in 24
 // bits (16 in 2D).
@@ -110,22 +127,11 @@ PG_DEV uint32_t vertex_key(uint32_t t) {
     return (a << 16) | (b << 8) | c;
 }
 
+// bit gs < 64 NW of a slot mask
 template <int NW>
 PG_DEV bool mask_has(const uint64_t (&m)[NW], int gs) {
-    if (gs >= 64 * NW) return false;
-    return (m[gs >> 6] >> (gs & 63)) & 1ull;
+    return (m[NW == 1 ? 0 : gs >> 6] >> (gs & 63)) & 1ull;
 }
-template <int NW>
-PG_DEV int mask_rank(const uint64_t (&m)[NW], int gs) {
-    int r = 0;
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-        if (w < (gs >> 6)) r += popc64(m[w]);
-        else if (w == (gs >> 6)) r += popc64(m[w] & ((1ull << (gs & 63)) - 1ull));
-    }
-    return r;
-}
-
 // Vertex of three planes (two lines in 2D) by the reference's Cramer rule
 // (cell.cpp:388-411), homogeneous part (X, Y, Z, W).
 template <int DIM>
@@ -175,15 +181,18 @@ PG_DEV bool conflict_exact(const Plane& p1, const Plane& p2, const Plane& p3, co
 // magnitude that bounds the rounding error of w, see XTOL)
 PG_DEV float plane_n1(const Plane& p, double wm) { return f2f_up(fabs(p.x) + fabs(p.y) + fabs(p.z) + wm); }
 
-// Per-seed register state of one lane.  Per slot: q bounds the product of
-// the vertex's plane 1-norms; e5 is the vertex's share of the reference's
-// eps (eps_bound of the largest 1-norm among its planes), made once with the
-// vertex instead of at every conflict test.
+// Per-seed register state of one lane.  Per slot: the vertex position, its
+// squared seed distance (float, +inf when not finite), and its share of the
+// conflict test's bound over |W|, W the vertex's Cramer denominator (floats
+// rounded up; see clip_step): qw = q / |W|, q bounding the product of the
+// planes' 1-norms, ew = eps / |W|, eps the eps_bound of the largest of them,
+// iw = 1 / |W|, made once with the vertex.  iw = +inf (every test of the vertex
+// is decided exactly) unless W is negative, as it is for a proper vertex.
 template <int S>
 struct SlotRegs {
-    double px[S], py[S], pz[S], pw[S], d2[S];
-    float q[S], e5[S];
-    uint32_t live;  // bit s = slot s holds a vertex
+    double px[S], py[S], pz[S];
+    float d2[S], qw[S], ew[S], iw[S];
+    bool live[S];  // slot s holds a vertex (lane masks in scalar registers)
 };
 
 // An upper bound (float, at least the smallest normal float) of 1.0000001e-14
@@ -205,48 +214,82 @@ PG_DEV float eps_bound(float m) {
 }
 
 template <int DIM, int S>
-PG_DEV void slot_write(SlotRegs<S>& r, int s, double px, double py, double pz, double pw, double d2,
-                       float q, float e5) {
+PG_DEV void slot_write(SlotRegs<S>& r, int s, double px, double py, double pz, float d2, float qw, float ew,
+                       float iw) {
 #pragma unroll
     for (int i = 0; i < S; i++) {
         if (i == s) {
             r.px[i] = px;
             r.py[i] = py;
             r.pz[i] = pz;
-            r.pw[i] = pw;
             r.d2[i] = d2;
-            r.q[i] = q;
-            r.e5[i] = e5;
+            r.qw[i] = qw;
+            r.ew[i] = ew;
+            r.iw[i] = iw;
+            r.live[i] = true;
         }
     }
-    r.live |= 1u << s;
 }
 
-// Build vertex numerics from its planes (reference arithmetic for position
-// and squared seed distance, cell.cpp:369-411).
-template <int DIM>
-PG_DEV void vertex_numerics(const Plane& a, const Plane& b, const Plane& c, double sx, double sy,
-                            double sz, double& px, double& py, double& pz, double& pw,
-                            double& d2) {
+// Squared seed distance of a vertex (cell.cpp:369-384's arithmetic).
+PG_DEV double vertex_d2(double px, double py, double pz, double sx, double sy, double sz) {
+    const double dx = px - sx, dy = py - sy, dz = pz - sz;
+    return dx * dx + dy * dy + dz * dz;
+}
+
+// A new vertex of planes a, b, c (reference arithmetic for the position,
+// cell.cpp:388-411) into slot s; na, nb, nc: the planes' 1-norms.
+template <int DIM, int S>
+PG_DEV void make_vertex(SlotRegs<S>& r, int s, const Plane& a, const Plane& b, const Plane& c, float na, float nb,
+                        float nc, double sx, double sy, double sz, float& qw, float& ew, float& iw) {
     double X, Y, Z, W;
     cramer<DIM>(a, b, c, X, Y, Z, W);
-    px = X / W;
-    py = Y / W;
-    pz = DIM == 3 ? Z / W : 0.0;
-    pw = W;
-    double dx = px - sx, dy = py - sy, dz = pz - sz;
-    d2 = dx * dx + dy * dy + dz * dz;
+    const double px = X / W, py = Y / W, pz = DIM == 3 ? Z / W : 0.0;
+    const float d = (float)vertex_d2(px, py, pz, sx, sy, sz);
+    // the bounds' products and v_rcp_f32 are each within 2^-22; 1.00001 covers them
+    const float aw = -(float)W;
+    iw = aw > 1e-37f ? __builtin_amdgcn_rcpf(aw) * 1.00001f : __builtin_inff();
+    qw = (DIM == 3 ? na * nb * nc : na * nb) * 1.000001f * iw;
+    ew = eps_bound<DIM>(fmaxf(fmaxf(na, nb), nc)) * iw;
+    slot_write<DIM, S>(r, s, px, py, pz, d <= 3e38f ? d : __builtin_inff(), qw, ew, iw);
+}
+
+// The initial box cell (cell.cpp:84-103): per vertex its planes, and the
+// vertices across its edges (edge e of a 3D vertex joins planes e, e + 1 mod
+// 3 and leads to the vertex holding them in the other order; line e of a 2D
+// vertex to the other vertex on it).
+template <int DIM>
+struct InitCell {
+    uint32_t tri[8], adj[8];
+};
+template <int DIM>
+constexpr InitCell<DIM> init_cell() {
+    InitCell<DIM> c{};
+    const uint32_t T3[8] = {2 | 5 << 8 | 0 << 16, 5 | 3 << 8 | 0 << 16, 1 | 5 << 8 | 2 << 16, 5 | 1 << 8 | 3 << 16,
+                            4 | 2 << 8 | 0 << 16, 4 | 0 << 8 | 3 << 16, 2 | 4 << 8 | 1 << 16, 4 | 3 << 8 | 1 << 16};
+    const uint32_t T2[4] = {2 | 0 << 8, 1 | 2 << 8, 3 | 1 << 8, 0 | 3 << 8};
+    const int n = DIM == 3 ? 8 : 4;
+    for (int i = 0; i < n; i++) c.tri[i] = DIM == 3 ? T3[i] : T2[i];
+    for (int i = 0; i < n; i++)
+        for (int e = 0; e < DIM; e++)
+            for (int j = 0; j < n; j++)
+                for (int f = 0; f < DIM; f++) {
+                    if (j == i) continue;
+                    const uint32_t ae = (c.tri[i] >> (8 * e)) & 0xff, be = (c.tri[i] >> (8 * ((e + 1) % DIM))) & 0xff;
+                    const uint32_t af = (c.tri[j] >> (8 * f)) & 0xff, bf = (c.tri[j] >> (8 * ((f + 1) % DIM))) & 0xff;
+                    if (DIM == 3 ? (af == be && bf == ae) : (af == ae)) c.adj[i] |= (uint32_t)j << (8 * e);
+                }
+    return c;
 }
 
 // Saved clip state (CLIP_STATE_BYTES per seed): planes, their bounds and
 // neighbour ids, then per vertex slot its planes (0xffffffff: empty slot)
-// and adjacency, then the plane and live-vertex counts.
+// and adjacency (as in LDS), then the plane and live-vertex counts.
 struct ClipState {
     Plane plane[64];
     float pn1[64];
     int32_t pvid[64];
-    uint32_t tri[64];
-    uint8_t adj[3][64];
+    uint2 va[64];
     int32_t nb_v, nlive;
 };
 static_assert(sizeof(ClipState) <= CLIP_STATE_BYTES, "clip state layout");
@@ -515,25 +558,26 @@ constexpr float SKIP_MARGIN = 1.0f / 32;
 constexpr float SKIP_F = 1.0f / 64;
 // clips after which the rest of a window is filtered again
 constexpr int REFILTER = 4;
+// 4 with the margin of the certificate's float compare
+constexpr float CERT_HI = 4.0f * (1.0f + 4e-7f), CERT_LO = 4.0f * (1.0f - 4e-7f);
 
 struct SkipBounds {
-    float g1, g2, g3;  // |W| SKIP_F > g1 q + g2 e5 + g3
+    float g1, g2, g3;  // SKIP_F > g1 qw + g2 ew + g3 iw
 };
-PG_DEV bool vertex_good(const SkipBounds& g, double pw, float q, float e5) {
-    return (float)pw * -SKIP_F > fmaf(g.g1, q, fmaf(g.g2, e5, g.g3));
+PG_DEV bool vertex_good(const SkipBounds& g, float qw, float ew, float iw) {
+    return fmaf(g.g1, qw, fmaf(g.g2, ew, g.g3 * iw)) < SKIP_F;
 }
-// wd2: squared distance of this lane's entry, ascending over the pend
+// wf: squared distance of this lane's entry, ascending over the pend
 // entries of the window (lanes 0 ..).
 template <int D, int G>
-PG_DEV SkipBounds window_bounds(double wd2, uint32_t pend, double sx, double sy, double sz) {
-    const float l2 = (float)wd2;
-    const float lo = shfl(l2, 0, G), hi = shfl(l2, pend ? 31 - __builtin_clz(pend) : 0, G);
-    const float E0 = __builtin_amdgcn_sqrtf(lo) * 0.999f, E1 = __builtin_amdgcn_sqrtf(hi) * 1.001f;
+PG_DEV SkipBounds window_bounds(float wf, uint32_t pend, double sx, double sy, double sz) {
+    const float lo = shfl(wf, 0, G), hi = shfl(wf, pend ? 31 - __builtin_clz(pend) : 0, G);
+    const float iE0 = __builtin_amdgcn_rsqf(lo) * 1.001f, E1 = __builtin_amdgcn_sqrtf(hi) * 1.001f;
     const float a = 1.75f + (float)(fabs(sx) + fabs(sy) + fabs(sz)) + 0.5f * E1;
     const float a2 = a * a;
     SkipBounds g;
-    g.g1 = 1.2e-14f * a / E0;
-    g.g2 = 2.1f / (E0 * E0);
+    g.g1 = 1.2e-14f * a * iE0;
+    g.g2 = 2.1f * (iE0 * iE0);
     g.g3 = D == 3 ? 2.1e-14f * a2 * a2 * a * E1 * E1 * E1 : 2.1e-14f * a2 * a2 * E1 * E1;
     return g;
 }
@@ -549,6 +593,53 @@ PG_DEV int rows_max_scatter(int m0, int m1, int m2, int m3) {
     return max((int)c[0], (int)c[1]);
 }
 
+// Arguments of the clip kernels: the first (explicit) kernel argument, so
+// that it starts the kernel-argument segment.  The output arrays are read
+// from the segment again when the outputs are written: as ordinary arguments
+// they would be loaded once and stay live across the clip, whose scalar
+// registers hold the lane masks of its slots and would spill.
+struct ClipArgs {
+    const double* pts;      // sorted points
+    int64_t n_total;        // seeds of the problem (exhaustive rows)
+    const uint32_t* seeds;  // sorted ids to clip (nullptr: all)
+    int64_t nq;             // their number,
+    const int64_t* nq_dev;  // or its device address (batches)
+    const uint32_t* knn;    // rows of length k
+    unsigned long long* ticket;
+    FaceArrays fa;
+    int k, max_p, max_t;
+};
+
+// The first argument of the running kernel, through a pointer the compiler
+// must treat as new.
+template <class A>
+PG_DEV const __attribute__((address_space(4))) A* fresh_args() {
+    const __attribute__((address_space(4))) A* p =
+        (const __attribute__((address_space(4))) A*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+// a FaceArrays out of the argument segment, field by field
+PG_DEV FaceArrays face_arrays_of(const __attribute__((address_space(4))) FaceArrays& a) {
+    FaceArrays f;
+    f.stride = a.stride;
+    f.nbr = a.nbr;
+    f.area = a.area;
+    f.nrm = a.nrm;
+    f.cen = a.cen;
+    f.count = a.count;
+    f.vol = a.vol;
+    f.ccen = a.ccen;
+    f.status = a.status;
+    f.kcert = a.kcert;
+    f.cstate = a.cstate;
+    f.resume = a.resume;
+    f.lastnb = a.lastnb;
+    f.key = a.key;
+    f.nbr_cm = a.nbr_cm;
+    return f;
+}
+
 // Exact mode (fa.key set, or EXACT): a conflict test is trusted in floating
 // point only above XTOL times the product of its rows' 1-norms (w measured
 // by the magnitude its rounding is relative to), a valid bound on how far the
@@ -562,15 +653,14 @@ PG_DEV int rows_max_scatter(int m0, int m1, int m2, int m3) {
 // BALL: the row is clipped whole, then the vertex-ball completion above
 // certifies the cell.
 template <int DIM, int G, int S, bool EXACT = false, bool BALL = false>
-__device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, const uint32_t* __restrict__ seeds,
-                              int64_t nq, const uint32_t* __restrict__ knn, int k, int max_p,
-                              int max_t, FaceArrays fa,
-                              VoroSmem<DIM, G, S>* smem,
-                              int64_t vblock, BallGrid bg = {}) {
+__device__ __forceinline__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, const uint32_t* __restrict__ seeds,
+                              int64_t nq, const uint32_t* __restrict__ knn, int k, int max_p, int max_t,
+                              const int32_t* resume, const uint8_t* cstate, const uint32_t* key,
+                              VoroSmem<DIM, G, S>* smem, int64_t vblock, BallGrid bg = {}) {
     using C = VoroCfg<DIM, G, S>;
     constexpr int NS = C::NS, NW = C::NW, MAXP = C::MAXP;
     constexpr int D = DIM;
-    constexpr bool SKIP = !EXACT && G == 16;  // row entries may be passed over
+    constexpr bool SKIP = !EXACT && (G == 16 || G == 8);  // row entries may be passed over
     const int tid = (int)threadIdx.x;
     const int grp = tid / G, gl = tid % G;
     const int shift = grp * G;
@@ -582,7 +672,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
     // exact mode (a build with the exact-predicate fallback): every test
     // whose sign the rounding of the planes could flip is decided exactly
     // (EXACT kernels) or flags the cell for them (the others)
-    const bool xmode = EXACT || fa.key != nullptr;
+    const bool xmode = EXACT || key != nullptr;
 
     const uint32_t sid = valid ? (seeds ? seeds[qi] : (uint32_t)qi) : 0u;
     const uint32_t* row = knn + (valid ? (size_t)qi * (size_t)k : 0);
@@ -596,11 +686,11 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
     // pass over the longer row from scratch.
     const int32_t shape_tag = (G << 24) | (S << 16);
     int v0 = 0;
-    if (valid && fa.resume != nullptr && NS <= 64) {
-        const int32_t r = fa.resume[sid];
+    if (valid && resume != nullptr && NS <= 64) {
+        const int32_t r = resume[sid];
         if (r > 0 && (r & 0x7fff0000) == shape_tag && (r & 0xffff) < k) v0 = r & 0xffff;
     }
-    const ClipState* cst = v0 ? reinterpret_cast<const ClipState*>(fa.cstate + (size_t)sid * CLIP_STATE_BYTES)
+    const ClipState* cst = v0 ? reinterpret_cast<const ClipState*>(cstate + (size_t)sid * CLIP_STATE_BYTES)
                               : nullptr;
     int nb_v0 = 2 * D, nlive0 = D == 3 ? 8 : 4;
     if (v0) {
@@ -614,9 +704,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
 #pragma unroll
         for (int i = 0; i < S; i++) {
             const int gs = i * G + gl;
-            sm.tri[gs] = cst->tri[gs];
-#pragma unroll
-            for (int e = 0; e < D; e++) sm.adj[e][gs] = cst->adj[e][gs];
+            sm.va[gs] = cst->va[gs];
         }
     }
     // Box planes (cell.cpp:44-82): eps = 1e-14 margin.
@@ -635,289 +723,288 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
         sm.pn1[gl] = plane_n1(p, fabs(p.w));
         sm.pvid[gl] = -1;
     }
-    // Initial vertices (cell.cpp:84-103).
+    // Initial vertices (cell.cpp:84-103): planes, and the vertices across
+    // their edges (edge e of a 3D vertex joins planes e and e + 1 mod 3).
     constexpr int NV0 = D == 3 ? 8 : 4;
     if (!v0 && gl < NV0) {
-        uint32_t t;
-        if (D == 3) {
-            const uint32_t T3[8] = {2 | 5 << 8 | 0 << 16, 5 | 3 << 8 | 0 << 16, 1 | 5 << 8 | 2 << 16,
-                                    5 | 1 << 8 | 3 << 16, 4 | 2 << 8 | 0 << 16, 4 | 0 << 8 | 3 << 16,
-                                    2 | 4 << 8 | 1 << 16, 4 | 3 << 8 | 1 << 16};
-            t = T3[gl];
-        } else {
-            const uint32_t T2[4] = {2 | 0 << 8, 1 | 2 << 8, 3 | 1 << 8, 0 | 3 << 8};
-            t = T2[gl];
-        }
-        sm.tri[gl] = t;
+        constexpr InitCell<D> T = init_cell<D>();
+        uint2 t = {0, 0};
+#pragma unroll
+        for (int i = 0; i < NV0; i++)
+            if (gl == i) t = make_uint2(T.tri[i], T.adj[i]);
+        sm.va[gl] = t;
     }
     block_sync();
     SlotRegs<S> R;
-    R.live = 0;
 #pragma unroll
     for (int s = 0; s < S; s++) {
-        R.px[s] = R.py[s] = R.pz[s] = R.pw[s] = R.d2[s] = 0.0;
-        R.q[s] = R.e5[s] = 0.f;
+        R.live[s] = false;
+        R.px[s] = R.py[s] = R.pz[s] = 0.0;
+        R.d2[s] = R.qw[s] = R.ew[s] = R.iw[s] = 0.f;
     }
-    // vertex numerics of slot i from its planes (of a resumed cell: with the
-    // same arithmetic and operand order as when the vertex was made)
-    auto slot_from_planes = [&](int i, uint32_t t) {
+    // vertex of slot i from its planes (of a resumed cell: with the same
+    // arithmetic and operand order as when it was made)
+    auto slot_from_planes = [&](int i, uint32_t t) __attribute__((always_inline)) {
         const int ia = tri_p(t, 0), ib = tri_p(t, 1), ic = D == 3 ? tri_p(t, 2) : tri_p(t, 1);
-        double px, py, pz, pw, d2;
-        vertex_numerics<D>(sm.plane[ia], sm.plane[ib], sm.plane[ic], sx, sy, sz, px, py, pz, pw, d2);
-        const float na = sm.pn1[ia], nb = sm.pn1[ib], nc = sm.pn1[ic];
-        const float q = (D == 3 ? na * nb * nc : na * nb) * 1.000001f;
-        slot_write<D, S>(R, i, px, py, pz, pw, d2, q, eps_bound<D>(fmaxf(fmaxf(na, nb), nc)));
+        float qw, ew, iw;
+        make_vertex<D, S>(R, i, sm.plane[ia], sm.plane[ib], sm.plane[ic], sm.pn1[ia], sm.pn1[ib], sm.pn1[ic], sx, sy,
+                          sz, qw, ew, iw);
     };
     if (v0) {
 #pragma unroll
         for (int i = 0; i < S; i++) {
-            const uint32_t t = sm.tri[i * G + gl];
+            const uint32_t t = sm.va[i * G + gl].x;
             if (t != 0xffffffffu) slot_from_planes(i, t);
         }
+    } else if (gl < NV0) {
+        slot_from_planes(0, sm.va[gl].x);  // NV0 <= G: vertex j lives in slot 0 of lane j
     }
-    // NV0 <= G: initial vertex j lives in slot 0 of lane j.
-    if (!v0 && gl < NV0) {
-        const uint32_t t = sm.tri[gl];
-        slot_from_planes(0, t);
-        // adjacency of the initial polytope
-        for (int e = 0; e < D; e++) {
-            uint8_t nb = END;
-            if (D == 3) {
-                int a0 = tri_p(t, e), b0 = tri_p(t, (e + 1) % 3);
-                for (int j = 0; j < NV0; j++) {
-                    if (j == gl) continue;
-                    uint32_t u = sm.tri[j];
-                    for (int f = 0; f < 3; f++)
-                        if (tri_p(u, f) == b0 && tri_p(u, (f + 1) % 3) == a0) nb = (uint8_t)j;
-                }
-            } else {
-                int L = tri_p(t, e);
-                for (int j = 0; j < NV0; j++) {
-                    if (j == gl) continue;
-                    uint32_t u = sm.tri[j];
-                    if (tri_p(u, 0) == L || tri_p(u, 1) == L) nb = (uint8_t)j;
-                }
-            }
-            sm.adj[e][gl] = nb;
-        }
-    }
-    block_sync();
 
     int nb_v = nb_v0;
     int nlive = nlive0;
     int status = SUCCESS;
     int kc = 0;
     bool done = !valid;
-    double R2 = 0.0;  // largest squared seed-vertex distance of the cell
+    // Largest squared seed-vertex distance of the cell: r2 in float for the
+    // certificate's clear decisions (a float compare against 4 r2 with a
+    // relative margin of 4e-7, several roundings), exact_R2 for the others.
+    auto exact_R2 = [&]() __attribute__((always_inline)) {
+        double m = 0.0;
 #pragma unroll
-    for (int s = 0; s < S; s++)
-        if ((R.live >> s) & 1u) R2 = smax(R.d2[s], R2);
-    R2 = group_butterfly_d<G>(R2, [](double a, double b) { return smax(a, b); });
+        for (int s = 0; s < S; s++)
+            if (R.live[s]) m = smax(vertex_d2(R.px[s], R.py[s], R.pz[s], sx, sy, sz), m);
+        return group_butterfly_d<G>(m, [](double a, double b) { return smax(a, b); });
+    };
+    auto group_r2 = [&]() __attribute__((always_inline)) {
+        float m = 0.f;
+#pragma unroll
+        for (int s = 0; s < S; s++) m = fmaxf(m, R.live[s] ? R.d2[s] : 0.f);
+        return group_max_f<G>(m);
+    };
+    float r2 = group_r2();
 
     // Row entries may be passed over without the conflict test only while
     // every live vertex is good (vertex_good): nb_skip, per group.
     SkipBounds win = {0.f, 0.f, 0.f};
     bool nb_skip = true;
+    const int cap_v = max_p < MAXP ? max_p : MAXP;  // planes the cell may have
 
     // One clip of the cell by the bisector of neighbour z at (bx, by, bz)
     // (act: this group clips in this step; every lane of the wave calls it):
     // new plane, conflict test of every live vertex, cavity, consistency and
     // new vertices.  Returns whether any seed of the wave clipped.
-    auto clip_step = [&](bool act, uint32_t z, double bx, double by, double bz) -> bool {
+    auto clip_step = [&](bool act, uint32_t z, double bx, double by, double bz) __attribute__((always_inline)) -> bool {
             // -- new half plane (cell.cpp:158-172)
-            Plane e = {0, 0, 0, 0};
-            double en1 = 0.0;  // 1-norm of e for the bounds (see plane_n1)
-            bool plane_ok = false;
-            int cur = 0;
-            if (act) {
-                if (nb_v >= max_p) {
-                    status = VERTEX_OVERFLOW;
-                } else if (nb_v >= MAXP) {
-                    status = SLOT_OVERFLOW;  // more planes than this kernel holds
-                } else {
-                    double dx = sx - bx, dy = sy - by, dz = sz - bz;
-                    double ax = sx + bx, ay = sy + by, az = sz + bz;
-                    double dot = ax * dx + ay * dy + az * dz;
-                    e = {dx, dy, dz, -dot / 2.0};
-                    const double ewm = xmode ? 0.5 * (fabs(ax * dx) + fabs(ay * dy) + fabs(az * dz)) : fabs(e.w);
-                    en1 = fabs(e.x) + fabs(e.y) + fabs(e.z) + ewm;
-                    cur = nb_v;
-                    plane_ok = true;
-                    if (gl == 0) {
-                        sm.plane[cur] = e;
-                        sm.pn1[cur] = f2f_up(en1);
-                        sm.pvid[cur] = (int32_t)z;
-                    }
-                    nb_v++;
-                }
+            if (wave_ballot(act && nb_v >= cap_v) != 0ull) {
+                // SLOT_OVERFLOW: more planes than this kernel holds
+                if (act && nb_v >= cap_v) status = nb_v >= max_p ? VERTEX_OVERFLOW : SLOT_OVERFLOW;
             }
-            // -- conflict test of every live vertex
-            uint32_t rem = 0;
-            bool flag = false;
-            if (act && plane_ok) {
-                // per plane: the eps bound of its own components, and the
-                // rounding bound's factor (exact mode: below XTOL en1 q the
-                // rounding of the planes themselves may flip the sign, which
-                // the reference's eps does not bound; such tests go to the
-                // exact predicate)
-                const uint32_t e_eps = __float_as_uint(eps_bound<D>(f2f_up(en1)));
-                const double en1s = en1 * (1.0 + 1e-15);
-                const double c1 = (5.4e-15 + (xmode ? XTOL : 0.0)) * en1s;
+            const bool go = act && nb_v < cap_v;
+            const int cur = nb_v;
+            const double ax = sx + bx, ay = sy + by, az = sz + bz;
+            Plane e = {sx - bx, sy - by, sz - bz, 0.0};
+            const double dot = ax * e.x + ay * e.y + az * e.z;
+            e.w = -dot / 2.0;
+            double ewm = fabs(e.w);
+            if (xmode) ewm = 0.5 * (fabs(ax * e.x) + fabs(ay * e.y) + fabs(az * e.z));
+            // 1-norm of e for the bounds (see plane_n1)
+            const double en1 = fabs(e.x) + fabs(e.y) + fabs(e.z) + ewm;
+            const float cn1 = f2f_up(en1);
+            if (go && gl == 0) {
+                sm.plane[cur] = e;
+                sm.pn1[cur] = cn1;
+                sm.pvid[cur] = (int32_t)z;
+            }
+            nb_v += go ? 1 : 0;
+            // -- conflict test of every live vertex.  The reference's
+            //    determinant is W f up to rounding, f = e . p + e.w >= 0 on the
+            //    seed's side and W < 0: the vertex goes when f < 0.  |W f|
+            //    above 5.4e-15 n1(e) q plus the eps bound of the four planes
+            //    decides as the reference does (48 u n1 q bounds the rounding of
+            //    both; exact mode: XTOL n1 q, below which the rounding of the
+            //    planes themselves may flip the sign, which the reference's eps
+            //    does not bound); here divided by |W| and compared in float
+            //    (1.00001: f's and the bound's float roundings).
+            const float c1 = (5.4e-15f + (xmode ? (float)XTOL : 0.f)) * 1.00001f * cn1;
+            const float e_eps = 1.00001f * eps_bound<D>(cn1);
+            bool rem[S];
+            uint32_t doubt = 0;  // slots to decide exactly
     #pragma unroll
-                for (int s = 0; s < S; s++) {
-                    const bool lv = (R.live >> s) & 1u;
-                    if (wave_ballot(lv) == 0ull || !lv) continue;  // levels no lane uses cost a branch
-                    double t;
-                    if (D == 3)
-                        t = R.pw[s] * fma(e.x, R.px[s], fma(e.y, R.py[s], fma(e.z, R.pz[s], e.w)));
-                    else
-                        t = R.pw[s] * fma(e.x, R.px[s], fma(e.y, R.py[s], e.w));
-                    // the larger of two non-negative floats by their bit
-                    // patterns (ordered like the values)
-                    const double epsu = (double)__uint_as_float(max(__float_as_uint(R.e5[s]), e_eps));
-                    const double bnd = fma(c1, (double)R.q[s], epsu);
-                    bool c;
-                    if (fabs(t) > bnd) {
-                        c = t > 0.0;
-                    } else {
-                        const double xb = xmode ? XTOL * en1s * (double)R.q[s] : 0.0;
-                        uint32_t tt = sm.tri[s * G + gl];
-                        const Plane p1 = sm.plane[tri_p(tt, 0)];
-                        const Plane p2 = sm.plane[tri_p(tt, 1)];
-                        const Plane p3 = sm.plane[D == 3 ? tri_p(tt, 2) : tri_p(tt, 1)];
-                        if (EXACT) {
-                            bool fl = false;
-                            c = conflict_exact<D>(p1, p2, p3, e, fl, xb);
-                            if (fl) {
-                                const double sp[3] = {sx, sy, sz}, bp[3] = {bx, by, bz};
-                                const int r = exact_conflict<D>(tt, sm, pts, sid, sp, z, bp, fa.key);
-                                if (r == 0) flag = true;  // outside the exact predicate's range
-                                else c = r > 0;
-                            }
-                        } else {
-                            c = conflict_exact<D>(p1, p2, p3, e, flag, xb);
-                        }
-                    }
-                    if (c) rem |= 1u << s;
-                }
+            for (int s = 0; s < S; s++) {
+                rem[s] = false;
+                const bool lv = go && R.live[s];
+                if (s > 0 && wave_ballot(lv) == 0ull) continue;  // levels no lane uses cost a branch
+                const double f = D == 3 ? fma(e.x, R.px[s], fma(e.y, R.py[s], fma(e.z, R.pz[s], e.w)))
+                                        : fma(e.x, R.px[s], fma(e.y, R.py[s], e.w));
+                const float ff = (float)f;
+                const float bnd = fmaf(c1, R.qw[s], fmaxf(R.ew[s], e_eps * R.iw[s]));
+                rem[s] = lv && ff < -bnd;
+                doubt |= lv && !(fabsf(ff) > bnd) ? 1u << s : 0u;
             }
-            // -- group masks
+            bool gflag = false;
+            if (wave_ballot(doubt != 0u) != 0ull) {
+                bool flag = false;
+                while (doubt) {
+                    const int s = __builtin_ctz(doubt);
+                    doubt &= doubt - 1u;
+                    const uint32_t tt = sm.va[s * G + gl].x;
+                    const int i1 = tri_p(tt, 0), i2 = tri_p(tt, 1), i3 = D == 3 ? tri_p(tt, 2) : i2;
+                    double xb = 0.0;
+                    if (xmode) {
+                        const float q = D == 3 ? sm.pn1[i1] * sm.pn1[i2] * sm.pn1[i3] : sm.pn1[i1] * sm.pn1[i2];
+                        xb = XTOL * (en1 * (1.0 + 1e-15)) * (double)(q * 1.000001f);
+                    }
+                    bool c;
+                    if (EXACT) {
+                        bool fl = false;
+                        c = conflict_exact<D>(sm.plane[i1], sm.plane[i2], sm.plane[i3], e, fl, xb);
+                        if (fl) {
+                            const double sp[3] = {sx, sy, sz}, bp[3] = {bx, by, bz};
+                            const int r = exact_conflict<D>(tt, sm, pts, sid, sp, z, bp, key);
+                            if (r == 0) flag = true;  // outside the exact predicate's range
+                            else c = r > 0;
+                        }
+                    } else {
+                        c = conflict_exact<D>(sm.plane[i1], sm.plane[i2], sm.plane[i3], e, flag, xb);
+                    }
+    #pragma unroll
+                    for (int i = 0; i < S; i++)
+                        if (i == s) rem[i] = c;
+                }
+                gflag = ((wave_ballot(flag) >> shift) & gmask) != 0ull;
+            }
+            // -- the group's removed slots
             uint64_t Rm[NW];
+            int nb_r = 0;
     #pragma unroll
             for (int w = 0; w < NW; w++) Rm[w] = 0ull;
     #pragma unroll
             for (int s = 0; s < S; s++) {
-                uint64_t b = (wave_ballot((rem >> s) & 1u) >> shift) & gmask;
-                int pos = s * G;
-                Rm[pos >> 6] |= b << (pos & 63);
+                Rm[(s * G) >> 6] |= ((wave_ballot(rem[s]) >> shift) & gmask) << ((s * G) & 63);
+                R.live[s] = R.live[s] && !rem[s];  // removed vertices leave the cell (also on failure)
             }
-            const bool gflag = ((wave_ballot(flag) >> shift) & gmask) != 0ull;
-            int nb_r = 0;
     #pragma unroll
             for (int w = 0; w < NW; w++) nb_r += popc64(Rm[w]);
-            bool doclip = false;
-            if (act && plane_ok) {
-                R.live &= ~rem;  // removed vertices leave the cell (also on failure)
-                if (gflag) {
-                    status = NEEDS_EXACT_PREDICATES;
-                } else if (nb_r == 0) {
-                    nb_v--;  // the plane clipped nothing (cell.cpp:132-136)
-                } else {
-                    doclip = true;
-                }
+            const bool doclip = go && !gflag && nb_r > 0;
+            if (go && !doclip) {
+                if (gflag) status = NEEDS_EXACT_PREDICATES;
+                else nb_v--;  // the plane clipped nothing (cell.cpp:132-136)
             }
-            // Most clip steps clip nothing (about 30 % of a uniform 3D seed's
-            // steps clip, and in half of a wave's steps none of its seeds does):
-            // the cavity, consistency and new-vertex machinery runs only when a
+            // The cavity, consistency and new-vertex machinery runs only when a
             // seed of the wave clips (a wave-uniform branch; a block is one wave).
             const bool anyclip = wave_ballot(doclip) != 0ull;
             if (anyclip) {
-                // -- cavity boundary: edges of removed vertices whose neighbour is
-                //    kept; bit 3 s + e of bm = edge e of my slot s (a lane walks only
-                //    its removed slots and then only its boundary edges)
-                uint32_t bm = 0;
-                if (doclip) {
-                    uint32_t rr = rem;
-                    while (rr) {
-                        const int s = __builtin_ctz(rr);
-                        rr &= rr - 1u;
-                        const int gs = s * G + gl;
+                // -- cavity boundary: edges of removed vertices whose neighbour
+                //    is kept
+                bool be[S][D];
+                uint2 va[S];
+                int mycnt = 0;
     #pragma unroll
-                        for (int ee = 0; ee < D; ee++)
-                            if (!mask_has<NW>(Rm, sm.adj[ee][gs])) bm |= 1u << (3 * s + ee);
+                for (int s = 0; s < S; s++) {
+    #pragma unroll
+                    for (int ee = 0; ee < D; ee++) be[s][ee] = false;
+                    va[s] = make_uint2(0u, 0u);
+                    const bool rm = doclip && rem[s];
+                    if (wave_ballot(rm) == 0ull) continue;
+                    if (rm) va[s] = sm.va[s * G + gl];
+    #pragma unroll
+                    for (int ee = 0; ee < D; ee++) {
+                        be[s][ee] = rm && !mask_has<NW>(Rm, tri_p(va[s].y, ee));
+                        mycnt += be[s][ee] ? 1 : 0;
                     }
                 }
-                const int mycnt = __builtin_popcount(bm);
-                const int incl = group_incl_sum<G>(mycnt, gl);
-                const int Bt = group_last<G>(incl);
-                int j = incl - mycnt;
-                if (doclip) {
-                    // in (slot, edge) order, as counted
-                    uint32_t b2 = bm;
-                    while (b2) {
-                        const int bit = __builtin_ctz(b2);
-                        b2 &= b2 - 1u;
-                        if (j >= NS) {  // more boundary edges than slots: overflow below
+                // -- slots for the new vertices: each lane with a free slot
+                //    offers its lowest one, and the boundary edges take the
+                //    offers lowest level first, so one new vertex per lane
+                //    unless lanes are full.  One prefix sum over the lanes for
+                //    both: the boundary edges in the high bits, one count of
+                //    offers per level (at most G = 16) in 5 bits each below
+                constexpr int FB = 5, EB = S <= 4 ? FB * S : 0;
+                int fl = S;
+    #pragma unroll
+                for (int s = S - 1; s >= 0; s--) fl = R.live[s] ? fl : s;
+                uint32_t in = (uint32_t)mycnt << EB;
+                if (S <= 4) in += fl < S ? 1u << (FB * fl) : 0u;
+                in = (uint32_t)group_incl_sum<G>((int)in, gl);
+                const uint32_t all = (uint32_t)group_last<G>((int)in);
+                const int Bt = (int)(all >> EB);
+                int j = (int)(in >> EB) - mycnt;
+                int offers = 0, rank = 0;  // of the group; of my offer
+                if (S <= 4) {
+    #pragma unroll
+                    for (int s = 0; s < S; s++) {
+                        const int c = (int)((all >> (FB * s)) & 31u);
+                        offers += c;
+                        rank += s < fl ? c : 0;
+                    }
+                    rank += (int)((in >> (FB * (fl & 3))) & 31u) - 1;
+                } else {
+    #pragma unroll
+                    for (int s = 0; s < S; s++) {
+                        const uint64_t b = (wave_ballot(fl == s) >> shift) & gmask;
+                        const int c = popc64(b);
+                        offers += c;
+                        rank += s < fl ? c : (s == fl ? popc64(b & ((1ull << gl) - 1ull)) : 0);
+                    }
+                }
+                // boundary edges in (slot, edge) order, as counted: plane a |
+                // plane b << 8 | kept neighbour << 16 (3D edge e joins planes e
+                // and e + 1 of the vertex; 2D: the line, 0, the neighbour)
+    #pragma unroll
+                for (int s = 0; s < S; s++) {
+                    if (s > 0 && wave_ballot(be[s][0] || be[s][1] || be[s][D - 1]) == 0ull) continue;
+    #pragma unroll
+                    for (int ee = 0; ee < D; ee++) {
+                        if (be[s][ee]) {
+                            const uint32_t sel = D == 3 ? (uint32_t)(ee | (ee + 1) % 3 << 8 | (4 + ee) << 16 | 0x0c << 24)
+                                                        : (uint32_t)(ee | 0x0c << 8 | (4 + ee) << 16 | 0x0c << 24);
+                            const uint32_t ed = __builtin_amdgcn_perm(va[s].y, va[s].x, sel);
+                            if (S > 3 || j < NS) {  // more boundary edges than slots: overflow below
+                                sm.edge[j < NS ? j : NS - 1] = ed;
+                                if (D == 3) {
+                                    sm.by_start[ed & 0xffu] = (uint8_t)j;
+                                    sm.by_end[(ed >> 8) & 0xffu] = (uint8_t)j;
+                                }
+                            }
                             j++;
-                            continue;
                         }
-                        const int s = bit / 3, ee = bit - 3 * s;
-                        const int gs = s * G + gl;
-                        const uint32_t t = sm.tri[gs];
-                        const int K = sm.adj[ee][gs];
-                        if (D == 3) {
-                            const int a = tri_p(t, ee), b = tri_p(t, ee == 2 ? 0 : ee + 1);
-                            sm.edge[j] = (uint32_t)a | (uint32_t)b << 8 | (uint32_t)K << 16;
-                            sm.by_start[a] = (uint8_t)j;
-                            sm.by_end[b] = (uint8_t)j;
-                        } else {
-                            const int L = tri_p(t, ee);
-                            sm.edge[j] = (uint32_t)L | (uint32_t)K << 16;
-                        }
-                        j++;
                     }
                 }
                 block_sync();
-                // -- consistency and capacity
+                // -- consistency and capacity.  3D: the boundary edges form one
+                //    cycle, each edge starting at the plane the one before it
+                //    ends at.  Around every plane the boundary edges that
+                //    start and end at it alternate, so when no two edges
+                //    start at one plane the successor map is a permutation.
                 bool ok = doclip;
                 bool bad = false;
-                int nxt = gl, lab = 0;  // 3D: successor edge and orbit label of edge gl
-                if (doclip) {
-                    if (D == 3) {
-                        // every boundary edge owns its start and end plane, and the
-                        // edge continuing it (the one starting at its end plane)
-                        // exists: the successor map is a permutation of the Bt edges
-                        for (int jj = gl; jj < Bt; jj += G) {
-                            uint32_t ed = sm.edge[jj];
-                            int a = ed & 0xff, b = (ed >> 8) & 0xff;
-                            if (sm.by_start[a] != jj || sm.by_end[b] != jj) bad = true;
-                            const int nx = sm.by_start[b];
-                            if (nx >= Bt || (int)(sm.edge[nx] & 0xffu) != b) bad = true;
-                        }
-                        if (Bt <= G && gl < Bt) {
-                            lab = gl;
-                            if (!bad) nxt = sm.by_start[(sm.edge[gl] >> 8) & 0xffu];
-                        }
-                    } else {
-                        bad = (Bt != 2);
-                    }
-                }
                 if (D == 3) {
-                    // ... and one cycle through all Bt edges: the smallest edge index
-                    // on each orbit, by pointer jumping over the group's lanes (all
-                    // groups of the wave take part; lanes without an edge point to
-                    // themselves), must be 0 everywhere
-                    if (nxt >= G) nxt = gl;  // only after a failed check above
+                    const int base = shift + gl;  // lane of the wave
+                    int nxt = base * 4, lab = gl;  // successor's lane (as a byte address), smallest edge seen
+                    if (doclip) {
+                        for (int jj = gl; jj < Bt && jj < NS; jj += G)
+                            if (sm.by_start[sm.edge[jj] & 0xffu] != jj) bad = true;
+                        if (Bt <= G && gl < Bt && !bad) {
+                            const int nx = sm.by_start[(sm.edge[gl] >> 8) & 0xffu];
+                            if (nx < Bt) nxt = (shift + nx) * 4;
+                            else bad = true;
+                        }
+                        if (gl >= Bt) lab = 0;
+                    }
+                    // the smallest edge index on each orbit, by pointer jumping
+                    // over the group's lanes (all groups of the wave take part;
+                    // lanes without an edge point to themselves), must be 0
+                    const int jmax = doclip && Bt <= G ? Bt : 0;
     #pragma unroll
                     for (int r = 1; r < 16 && r < G; r <<= 1) {
-                        const int l2 = shfl(lab, nxt, G);
-                        nxt = shfl(nxt, nxt, G);
-                        lab = min(lab, l2);
+                        if (wave_ballot(jmax > r) == 0ull) break;
+                        lab = min(lab, __builtin_amdgcn_ds_bpermute(nxt, lab));
+                        nxt = __builtin_amdgcn_ds_bpermute(nxt, nxt);
                     }
                     if (doclip) {
                         if (Bt <= G) {
                             if (lab != 0) bad = true;
-                        } else if (gl == 0 && !bad) {
+                        } else if (gl == 0 && !bad && Bt <= NS) {
                             int jj = 0, steps = 0;
                             do {
                                 jj = sm.by_start[(sm.edge[jj] >> 8) & 0xffu];
@@ -926,6 +1013,8 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                             if (steps != Bt || jj != 0) bad = true;
                         }
                     }
+                } else {
+                    bad = doclip && Bt != 2;
                 }
                 const bool gbad = ((wave_ballot(bad) >> shift) & gmask) != 0ull;
                 bad = false;  // from here: a new vertex no skip can pass (see vertex_good)
@@ -943,95 +1032,73 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                     }
                     nlive -= nb_r;
                 }
-                // -- slots of the new vertices: round by round, each lane with a
-                //    free slot left offers its lowest one, and the boundary
-                //    edges take the offers lowest level first (one round, one
-                //    new vertex per lane, unless lanes are full); the edge of
-                //    a slot waits in its tri entry
-                uint32_t asg = 0;
-                {
-                    uint32_t fr = ok ? ~R.live & ((1u << S) - 1u) : 0u;
-                    int base = 0;
-                    for (;;) {
-                        const int fl = fr ? __builtin_ctz(fr) : S;
-                        int r = base, tot = 0;
+                // the offers' slots, then, where lanes hold several new
+                // vertices, more rounds of offers (an edge past the first
+                // round waits in its slot's va entry)
+                uint32_t more = 0;
+                const bool mine = ok && fl < S && rank < Bt;
+                if (mine) sm.newslot[rank] = (uint8_t)(fl * G + gl);
+                if (wave_ballot(ok && offers < Bt) != 0ull) {
+                    uint32_t fr = 0;
     #pragma unroll
-                        for (int s = 0; s < S; s++) {
-                            const uint64_t b = (wave_ballot(fl == s) >> shift) & gmask;
-                            const int c = popc64(b);
-                            if (s < fl) r += c;
-                            else if (s == fl) r += popc64(b & ((1ull << gl) - 1ull));
-                            tot += c;
-                        }
+                    for (int s = 0; s < S; s++) fr |= ok && !R.live[s] && s != fl ? 1u << s : 0u;
+                    int base = offers;
+                    while (wave_ballot(ok && base < Bt) != 0ull) {
+                        const uint64_t b = (wave_ballot(fr != 0u) >> shift) & gmask;
+                        const int r = base + popc64(b & ((1ull << gl) - 1ull));
                         if (fr && r < Bt) {
-                            const int gs = fl * G + gl;
-                            sm.newslot[r] = (uint8_t)gs;
-                            sm.tri[gs] = (uint32_t)r;
-                            asg |= 1u << fl;
+                            const int s = __builtin_ctz(fr);
+                            sm.newslot[r] = (uint8_t)(s * G + gl);
+                            sm.va[s * G + gl].x = (uint32_t)r;
+                            more |= 1u << s;
                         }
                         fr &= fr - 1u;
-                        base += tot;
-                        if (wave_ballot(ok && base < Bt) == 0ull) break;
+                        base += popc64(b);
                     }
                 }
                 block_sync();
                 // -- new vertices (cell.cpp:346-364 orientation, :388-411 position)
-                if (ok) {
-                    const float cn1 = f2f_up(en1);
-                    while (asg) {
-                        const int s = ffs64(asg);
-                        asg &= asg - 1;
-                        const int gs = s * G + gl;
-                        const int r = (int)sm.tri[gs];
-                        const uint32_t ed = sm.edge[r];
-                        uint32_t t;
-                        Plane pa, pb;
-                        if (D == 3) {
-                            const int a = ed & 0xff, b = (ed >> 8) & 0xff, K = (ed >> 16) & 0xff;
-                            t = (uint32_t)cur | (uint32_t)a << 8 | (uint32_t)b << 16;
-                            pa = sm.plane[a];
-                            pb = sm.plane[b];
-                            const float na = sm.pn1[a], nb = sm.pn1[b];
-                            const float q = cn1 * na * nb * 1.000001f;
-                            const float e5 = eps_bound<D>(fmaxf(cn1, fmaxf(na, nb)));
-                            sm.tri[gs] = t;
-                            sm.adj[0][gs] = sm.newslot[sm.by_end[a]];
-                            sm.adj[1][gs] = (uint8_t)K;
-                            sm.adj[2][gs] = sm.newslot[sm.by_start[b]];
-                            const uint32_t tk = sm.tri[K];
-                            for (int f = 0; f < 3; f++)
-                                if (tri_p(tk, f) == b && tri_p(tk, (f + 1) % 3) == a) sm.adj[f][K] = (uint8_t)gs;
-                            double px, py, pz, pw, d2;
-                            vertex_numerics<D>(e, pa, pb, sx, sy, sz, px, py, pz, pw, d2);
-                            slot_write<D, S>(R, s, px, py, pz, pw, d2, q, e5);
-                            bad = bad || !vertex_good(win, pw, q, e5);
-                        } else {
-                            const int L = ed & 0xff, K = (ed >> 16) & 0xff;
-                            pa = sm.plane[L];
-                            const double rw = det2(e.x, e.y, pa.x, pa.y);
-                            const bool swap = rw > 0;
-                            t = swap ? ((uint32_t)L | (uint32_t)cur << 8) : ((uint32_t)cur | (uint32_t)L << 8);
-                            const uint8_t other = sm.newslot[1 - r];
-                            sm.tri[gs] = t;
-                            sm.adj[0][gs] = swap ? (uint8_t)K : other;
-                            sm.adj[1][gs] = swap ? other : (uint8_t)K;
-                            const uint32_t tk = sm.tri[K];
-                            for (int f = 0; f < 2; f++)
-                                if (tri_p(tk, f) == L) sm.adj[f][K] = (uint8_t)gs;
-                            const float nL = sm.pn1[L];
-                            const float q = cn1 * nL * 1.000001f;
-                            const float e5 = eps_bound<D>(fmaxf(cn1, nL));
-                            double px, py, pz, pw, d2;
-                            if (swap)
-                                vertex_numerics<D>(pa, e, e, sx, sy, sz, px, py, pz, pw, d2);
-                            else
-                                vertex_numerics<D>(e, pa, pa, sx, sy, sz, px, py, pz, pw, d2);
-                            slot_write<D, S>(R, s, px, py, pz, pw, d2, q, e5);
-                            bad = bad || !vertex_good(win, pw, q, e5);
-                        }
+                auto new_vertex = [&](int s, int r) __attribute__((always_inline)) {
+                    const int gs = s * G + gl;
+                    const uint32_t ed = sm.edge[r];
+                    const int K = (int)(ed >> 16);
+                    float qw, ew, iw;
+                    if (D == 3) {
+                        const int a = ed & 0xff, b = (ed >> 8) & 0xff;
+                        const uint32_t prev = sm.newslot[sm.by_end[a]], next = sm.newslot[sm.by_start[b]];
+                        const uint32_t tk = sm.va[K].x;
+                        make_vertex<D, S>(R, s, e, sm.plane[a], sm.plane[b], cn1, sm.pn1[a], sm.pn1[b], sx, sy, sz, qw, ew,
+                                          iw);
+                        sm.va[gs] = make_uint2((uint32_t)cur | (ed & 0xffffu) << 8, prev | (uint32_t)K << 8 | next << 16);
+                        // the kept neighbour's edge (b, a) now leads here
+                        const uint32_t rk = tk | tk << 24, ba = (uint32_t)(b | a << 8);
+                        const int f = (rk & 0xffffu) == ba ? 0 : (((rk >> 8) & 0xffffu) == ba ? 1 : 2);
+                        if (f < 2 || (rk >> 16) == ba) set_adj(sm.va[K], f, gs);
+                    } else {
+                        const int L = ed & 0xff;
+                        const Plane pa = sm.plane[L];
+                        const float nL = sm.pn1[L];
+                        const uint32_t other = sm.newslot[1 - r], tk = sm.va[K].x;
+                        const bool swap = det2(e.x, e.y, pa.x, pa.y) > 0;
+                        const Plane& p1 = swap ? pa : e;
+                        const Plane& p2 = swap ? e : pa;
+                        make_vertex<D, S>(R, s, p1, p2, p2, swap ? nL : cn1, swap ? cn1 : nL, swap ? cn1 : nL, sx, sy, sz,
+                                          qw, ew, iw);
+                        sm.va[gs] = swap ? make_uint2((uint32_t)L | (uint32_t)cur << 8, (uint32_t)K | other << 8)
+                                         : make_uint2((uint32_t)cur | (uint32_t)L << 8, other | (uint32_t)K << 8);
+                        set_adj(sm.va[K], tri_p(tk, 0) == L ? 0 : 1, gs);
                     }
-                    nlive += Bt;
+                    bad = bad || !vertex_good(win, qw, ew, iw);
+                };
+                if (mine) new_vertex(fl, rank);
+                if (wave_ballot(more != 0u) != 0ull) {
+                    while (more) {
+                        const int s = __builtin_ctz(more);
+                        more &= more - 1u;
+                        new_vertex(s, (int)sm.va[s * G + gl].x);
+                    }
                 }
+                if (ok) nlive += Bt;
                 if (((wave_ballot(bad) >> shift) & gmask) != 0ull) nb_skip = false;
                 block_sync();
             }
@@ -1046,19 +1113,17 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
     // the R2 of the last clip, all entries of the window at once.  Seeds of a
     // wave walk their own windows: every step of the wave clips a candidate
     // of each of its seeds.
-    const int cap_v = max_p < MAXP ? max_p : MAXP;
     int wb = v0;                 // row entry of the window's lane 0
     uint32_t pend = 0, cand = 0; // window entries ahead; of those, the ones to clip
-    double wd2 = 0.0;            // this lane's entry: squared distance, float offset
-    float wx = 0.f, wy = 0.f, wz = 0.f;
+    float wf = 0.f, wx = 0.f, wy = 0.f, wz = 0.f;  // this lane's entry: squared distance and offset
     bool first = true;
     int since = 0;
     // entries of the window ahead whose bisector may cut the cell: the
     // others keep every live vertex on the seed's side by a margin
-    auto window_filter = [&]() {
+    auto window_filter = [&]() __attribute__((always_inline)) {
         float mx = 0.f;  // largest offset . vertex of this lane's entry (the seed as origin)
         bool vbad = false;
-        if constexpr (G == 16) {
+        if constexpr (SKIP) {
             // offsets (columns) times vertices (rows) of the wave's four
             // seeds, one 16 x 16 block per seed and slot level, on the
             // matrix cores: entry (i, j) of block b sits in register 4 b +
@@ -1067,9 +1132,9 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
             int m4[4] = {0, 0, 0, 0};
 #pragma unroll
             for (int s = 0; s < S; s++) {
-                const bool lv = (R.live >> s) & 1u;
+                const bool lv = R.live[s];
                 if (wave_ballot(lv) == 0ull) continue;
-                vbad = vbad || (lv && !vertex_good(win, R.pw[s], R.q[s], R.e5[s]));
+                vbad = vbad || (lv && !vertex_good(win, R.qw[s], R.ew[s], R.iw[s]));
                 f32x16 c = {0.f};
                 c = __builtin_amdgcn_mfma_f32_16x16x1f32(lv ? (float)(R.px[s] - sx) : 0.f, wx, c, 0, 0, 0);
                 c = __builtin_amdgcn_mfma_f32_16x16x1f32(lv ? (float)(R.py[s] - sy) : 0.f, wy, c, 0, 0, 0);
@@ -1079,10 +1144,11 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                     m4[b] = max(max(max(m4[b], __float_as_int(c[4 * b])), max(__float_as_int(c[4 * b + 1]), __float_as_int(c[4 * b + 2]))),
                                 __float_as_int(c[4 * b + 3]));
             }
+            if (G == 8 && ((tid >> 5) & 1) != ((tid >> 3) & 1)) m4[0] = m4[1] = m4[2] = m4[3] = 0;
             mx = __int_as_float(rows_max_scatter(m4[0], m4[1], m4[2], m4[3]));
         }
         const float h = wx * wx + wy * wy + wz * wz;
-        const float slack = 2e-6f * (fabsf(wx) + fabsf(wy) + fabsf(wz)) * __builtin_amdgcn_sqrtf((float)R2 * 1.001f);
+        const float slack = 2e-6f * (fabsf(wx) + fabsf(wy) + fabsf(wz)) * __builtin_amdgcn_sqrtf(r2 * 1.001f);
         const bool cut = !(mx < h * (0.5f - SKIP_MARGIN) - slack);
         const uint32_t cm = (uint32_t)((wave_ballot(cut) >> shift) & gmask);
         const bool gb = ((wave_ballot(vbad) >> shift) & gmask) != 0ull;
@@ -1092,13 +1158,28 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
     };
     for (;;) {
         if (!BALL) {
-            const uint32_t cm = (uint32_t)((wave_ballot(wd2 > 4 * R2) >> shift) & gmask) & pend;
+            // passed entries the certificate holds at (a group's lanes act
+            // on their own entries; entries ascend, so a doubtful one can
+            // only precede the clear ones)
+            bool cert = wf > r2 * CERT_HI;
+            const bool ahead = !done && ((pend >> gl) & 1u);
+            if (wave_ballot(ahead && !cert && !(wf < r2 * CERT_LO)) != 0ull) {
+                const double R2 = exact_R2();
+                if (ahead) {
+                    const double dx = sm.nbp[gl][0] - sx, dy = sm.nbp[gl][1] - sy;
+                    const double dz = D == 3 ? sm.nbp[gl][2] - sz : 0.0;
+                    cert = dx * dx + dy * dy + dz * dz > 4 * R2;
+                }
+            }
+            const uint32_t cm = (uint32_t)((wave_ballot(cert) >> shift) & gmask) & pend;
             if (!done && cm != 0u && (cand == 0u || __builtin_ctz(cm) < __builtin_ctz(cand))) {
                 kc = wb + __builtin_ctz(cm) + 1;
                 done = true;
             }
         }
-        if (wave_ballot(!done && cand == 0u) != 0ull) {
+        const bool refill = wave_ballot(!done && cand == 0u) != 0ull;
+        bool filter = since >= REFILTER;
+        if (refill) {
             // a seed has passed its window: every seed's next one
             if (!done) {
                 if (!first) wb += cand != 0u ? __builtin_ctz(cand) : G;
@@ -1106,8 +1187,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
             }
             pend = done ? 0u : (uint32_t)((1ull << min(G, k - wb)) - 1ull);
             cand = pend;
-            wd2 = 0.0;
-            wx = wy = wz = 0.f;
+            wf = wx = wy = wz = 0.f;
             if ((pend >> gl) & 1u) {
                 const uint32_t zz = row[wb + gl];
                 double bp[3] = {0, 0, 0};
@@ -1115,23 +1195,20 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
 #pragma unroll
                 for (int d = 0; d < D; d++) sm.nbp[gl][d] = bp[d] = pts[(size_t)D * zz + d];
                 const double dx = bp[0] - sx, dy = bp[1] - sy, dz = D == 3 ? bp[2] - sz : 0.0;
-                wd2 = dx * dx + dy * dy + dz * dz;
+                wf = (float)(dx * dx + dy * dy + dz * dz);
                 wx = (float)dx;
                 wy = (float)dy;
                 wz = (float)dz;
             }
-            win = window_bounds<D, G>(wd2, pend, sx, sy, sz);
+            win = window_bounds<D, G>(wf, pend, sx, sy, sz);
             block_sync();
-            if (wave_ballot(!done) == 0ull) break;
-            if (SKIP && !xmode && !first) window_filter();
+            filter = !first;
             first = false;
-            continue;
         }
         if (wave_ballot(!done) == 0ull) break;
-        if (SKIP && !xmode && since >= REFILTER) {
-            window_filter();
-            continue;
-        }
+        filter = filter && SKIP && !xmode;
+        if (filter) window_filter();
+        if (refill || filter) continue;
         const bool act = !done;
         // the step's neighbour
         uint32_t z = 0;
@@ -1150,25 +1227,22 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
         since++;
         // -- certificate (cell.cpp:369-384) with the just-clipped neighbour;
         //    the largest seed-vertex distance only changes with a clip
-        double mx = R2;
-        if (anyclip) {
-            mx = 0.0;
-#pragma unroll
-            for (int s = 0; s < S; s++)
-                if ((R.live >> s) & 1u) mx = smax(R.d2[s], mx);
-            mx = group_butterfly_d<G>(mx, [](double a, double b) { return smax(a, b); });
+        if (anyclip) r2 = group_r2();
+        const double dx = bx - sx, dy = by - sy, dz = bz - sz;
+        const double dz2 = dx * dx + dy * dy + dz * dz;
+        bool cert = !BALL && (float)dz2 > r2 * CERT_HI;
+        if (!BALL && wave_ballot(act && (xmode || (!cert && !((float)dz2 < r2 * CERT_LO)))) != 0ull) {
+            const double R2 = exact_R2();
+            cert = dz2 > 4 * R2 * (EXACT ? CERT_TIE : 1.0);
+            if (!EXACT && xmode && act && cert && status == SUCCESS && !(dz2 > 4 * R2 * CERT_TIE)) {
+                status = NEEDS_EXACT_PREDICATES;  // a near tie: the exact kernel decides
+                cert = false;
+            }
         }
         if (act) {
-            R2 = mx;
-            const double dx = bx - sx, dy = by - sy, dz = bz - sz;
-            const double dz2 = dx * dx + dy * dy + dz * dz;
-            if (!BALL && dz2 > 4 * R2 * (EXACT ? CERT_TIE : 1.0)) {
-                if (!EXACT && xmode && status == SUCCESS && !(dz2 > 4 * R2 * CERT_TIE)) {
-                    status = NEEDS_EXACT_PREDICATES;  // a near tie: the exact kernel decides
-                } else {
-                    kc = wb + j + 1;
-                    done = true;
-                }
+            if (cert) {
+                kc = wb + j + 1;
+                done = true;
             }
             if (status != SUCCESS) done = true;
             if (!nb_skip || nb_v >= cap_v) cand = pend;
@@ -1199,15 +1273,15 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
             int32_t* const cpf = cst + G;
 #pragma unroll
             for (int s = 0; s < S; s++) {
-                const uint32_t t = sm.tri[s * G + gl];
-                const bool need = !bdone && ((R.live >> s) & 1u) && (!((known >> s) & 1u) || ctri[s] != t);
+                const uint32_t t = sm.va[s * G + gl].x;
+                const bool need = !bdone && R.live[s] && (!((known >> s) & 1u) || ctri[s] != t);
                 uint64_t m = (wave_ballot(need) >> shift) & gmask;
                 while (wave_ballot(m != 0ull) != 0ull) {
                     if (m == 0ull) continue;
                     const int src = ffs64(m);
                     m &= m - 1ull;
                     const double vv[3] = {shfl(R.px[s], src, G), shfl(R.py[s], src, G), shfl(R.pz[s], src, G)};
-                    const double r2v = shfl(R.d2[s], src, G);
+                    const double r2v = vertex_d2(vv[0], vv[1], vv[2], sx, sy, sz);
                     const int32_t cq =
                         ball_search_group<D, G>(bg, pts, vv, r2v, sid, sm.pvid, nb_v, gl, shift, gmask, cst, cpf);
                     if (gl == src) cand[s] = cq;
@@ -1220,7 +1294,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
             if (!bdone) {
 #pragma unroll
                 for (int s = 0; s < S; s++) {
-                    if (!((R.live >> s) & 1u)) continue;
+                    if (!R.live[s]) continue;
                     if (cand[s] == -2) far = true;
                     if (cand[s] < 0) continue;
                     const int32_t q = cand[s];
@@ -1274,6 +1348,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
     // at the same row length and applies this test itself)
     const int loop_status = status;
     const uint32_t zl = valid ? row[k - 1] : 0u;
+    const double R2 = BALL ? 0.0 : exact_R2();
     if (valid && !BALL) {
         const double dx = pts[(size_t)D * zl] - sx, dy = pts[(size_t)D * zl + 1] - sy;
         const double dz = D == 3 ? pts[(size_t)D * zl + 2] - sz : 0.0;
@@ -1289,6 +1364,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
         if (status != SUCCESS) kc = 0;
     }
 
+    const FaceArrays fa = face_arrays_of(fresh_args<ClipArgs>()->fa);
     // save an uncertified cell that ran through its whole row, for a resume
     // at a longer row
     if (fa.resume != nullptr && NS <= 64) {
@@ -1303,9 +1379,8 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
 #pragma unroll
             for (int i = 0; i < S; i++) {
                 const int gs = i * G + gl;
-                out->tri[gs] = ((R.live >> i) & 1u) ? sm.tri[gs] : 0xffffffffu;
-#pragma unroll
-                for (int e = 0; e < D; e++) out->adj[e][gs] = sm.adj[e][gs];
+                const uint2 v = sm.va[gs];
+                out->va[gs] = make_uint2(R.live[i] ? v.x : 0xffffffffu, v.y);
             }
             if (gl == 0) {
                 out->nb_v = nb_v;
@@ -1320,32 +1395,16 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
 
     // ---------------------------------------------------------- extraction
     const bool ext = valid && status == SUCCESS;
-    // normals and neighbour ids of my planes (cell.cpp:575-579, 646-669)
-    double nx[C::PPL], ny[C::PPL], nz[C::PPL];
-    int32_t pv[C::PPL];
 #pragma unroll
-    for (int i = 0; i < C::PPL; i++) {
-        const int p = gl + G * i;
-        nx[i] = ny[i] = nz[i] = 0.0;
-        pv[i] = -1;
-        if (ext && p < nb_v) {
-            const Plane pe = sm.plane[p];
-            const double nl = sqrt(pe.x * pe.x + pe.y * pe.y + pe.z * pe.z);
-            nx[i] = pe.x / nl;
-            ny[i] = pe.y / nl;
-            nz[i] = pe.z / nl;
-            pv[i] = sm.pvid[p];
-        }
-        if (p < MAXP) sm.first[p] = 0xffffffffu;
-    }
+    for (int i = 0; i < C::PPL; i++) sm.first[gl + G * i] = 0xffffffffu;
     block_sync();
-    // vertex positions to LDS (over the planes), lowest slot per plane
+    // lowest vertex per plane
     if (ext) {
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            if (!((R.live >> s) & 1u)) continue;
+            if (!R.live[s]) continue;
             const int gs = s * G + gl;
-            const uint32_t t = sm.tri[gs];
+            const uint32_t t = sm.va[gs].x;
             // a face's cycle starts at its vertex with the smallest sorted
             // plane tuple: the same vertex whatever slot it occupies, so the
             // fan sums round identically for every kernel shape
@@ -1355,10 +1414,44 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
         }
     }
     block_sync();
+    // the planes that hold a vertex, listed in plane order: face r is lane r %
+    // G's in pass r / G (of 26 planes of a cell some 16 are faces; by plane
+    // index the passes would take most lanes through planes without one)
+    bool has[C::PPL];
+    int nface = 0, fb_rank = 0;
+#pragma unroll
+    for (int i = 0; i < C::PPL; i++) {
+        const int p = gl + G * i;
+        has[i] = ext && p < nb_v && sm.first[p] != 0xffffffffu;
+        const uint64_t b = (wave_ballot(has[i]) >> shift) & gmask;
+        if (has[i]) sm.plist[nface + popc64(b & ((1ull << gl) - 1ull))] = (uint8_t)p;
+        nface += popc64(b);
+        if (BALL) fb_rank += popc64((wave_ballot(has[i] && p < first_ball) >> shift) & gmask);
+    }
+    block_sync();
+    // normals and neighbour ids of my faces (cell.cpp:575-579, 646-669)
+    double nx[C::PPL], ny[C::PPL], nz[C::PPL];
+    int fp[C::PPL];  // plane of my face (-1: none)
+#pragma unroll
+    for (int i = 0; i < C::PPL; i++) {
+        const int r = gl + G * i;
+        nx[i] = ny[i] = nz[i] = 0.0;
+        fp[i] = -1;
+        if (r < nface) {
+            fp[i] = sm.plist[r];
+            const Plane pe = sm.plane[fp[i]];
+            const double nl = sqrt(pe.x * pe.x + pe.y * pe.y + pe.z * pe.z);
+            nx[i] = pe.x / nl;
+            ny[i] = pe.y / nl;
+            nz[i] = pe.z / nl;
+        }
+    }
+    block_sync();
+    // vertex positions to LDS (over the planes)
     if (ext) {
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            if (!((R.live >> s) & 1u)) continue;
+            if (!R.live[s]) continue;
             const int gs = s * G + gl;
             sm.vpos[3 * gs] = R.px[s];
             sm.vpos[3 * gs + 1] = R.py[s];
@@ -1374,19 +1467,17 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
     const double* vpos = sm.vpos;
 #pragma unroll
     for (int i = 0; i < C::PPL; i++) {
-        const int p = gl + G * i;
         isface[i] = false;
         farea[i] = fcx[i] = fcy[i] = fcz[i] = 0.0;
         pvol[i] = pcx[i] = pcy[i] = pcz[i] = 0.0;
         double vol = 0.0, cxs = 0.0, cys = 0.0, czs = 0.0;
-        if (!(ext && p < nb_v)) continue;
-        if (sm.first[p] == 0xffffffffu) continue;
+        if (fp[i] < 0) continue;
+        const int p = fp[i];
         const uint32_t v0 = sm.first[p] & 0xffu;
         const double x0 = vpos[3 * v0], y0 = vpos[3 * v0 + 1], z0 = vpos[3 * v0 + 2];
         if (D == 2) {
-            const uint32_t t0 = sm.tri[v0];
-            const int ee = tri_p(t0, 0) == p ? 0 : 1;
-            const int v1 = sm.adj[ee][v0];
+            const uint2 t0 = sm.va[v0];
+            const int v1 = tri_p(t0.y, tri_p(t0.x, 0) == p ? 0 : 1);
             const double x1 = vpos[3 * v1], y1 = vpos[3 * v1 + 1];
             const double dx = x1 - x0, dy = y1 - y0;
             farea[i] = sqrt(dx * dx + dy * dy);
@@ -1437,9 +1528,9 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
                 pz = zz;
                 have_prev = true;
                 cnt++;
-                const uint32_t t = sm.tri[cv];
-                const int ee = tri_p(t, 0) == p ? 0 : (tri_p(t, 1) == p ? 1 : 2);
-                cv = sm.adj[ee][cv];
+                const uint2 t = sm.va[cv];
+                const int ee = tri_p(t.x, 0) == p ? 0 : (tri_p(t.x, 1) == p ? 1 : 2);
+                cv = (uint32_t)tri_p(t.y, ee);
             } while (cv != v0 && cnt <= NS);
             pvol[i] = vol;
             pcx[i] = cxs;
@@ -1457,7 +1548,7 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
         }
     }
     // face order = plane order among planes that form a face
-    uint64_t fm = 0;
+    uint64_t fm = 0;  // by rank in the list
 #pragma unroll
     for (int i = 0; i < C::PPL; i++) {
         uint64_t b = (wave_ballot(isface[i]) >> shift) & gmask;
@@ -1465,14 +1556,22 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
     }
     // cell volume and centroid moments: a pairwise sum over the plane index,
     // lowest bit first (lanes hold bits below log2 G, the planes of a lane
-    // the bits above), i.e. the same tree for every kernel shape
+    // the bits above), i.e. the same tree for every kernel shape; the faces'
+    // moments go back to their planes' lanes through LDS (over the positions)
+    block_sync();
+#pragma unroll
+    for (int i = 0; i < C::PPL; i++)
+        if (fp[i] >= 0) sm.plane[fp[i]] = {pvol[i], pcx[i], pcy[i], pcz[i]};
+    block_sync();
     const auto add = [](double theirs, double mine) { return mine + theirs; };
 #pragma unroll
     for (int i = 0; i < C::PPL; i++) {
-        pvol[i] = group_butterfly_d<G>(pvol[i], add);
-        pcx[i] = group_butterfly_d<G>(pcx[i], add);
-        pcy[i] = group_butterfly_d<G>(pcy[i], add);
-        pcz[i] = group_butterfly_d<G>(pcz[i], add);
+        Plane m = {0.0, 0.0, 0.0, 0.0};
+        if (has[i]) m = sm.plane[gl + G * i];
+        pvol[i] = group_butterfly_d<G>(m.x, add);
+        pcx[i] = group_butterfly_d<G>(m.y, add);
+        pcy[i] = group_butterfly_d<G>(m.z, add);
+        pcz[i] = group_butterfly_d<G>(m.w, add);
     }
 #pragma unroll
     for (int w = 1; w < C::PPL; w <<= 1)
@@ -1488,25 +1587,26 @@ __device__ void voronoi_group(const double* __restrict__ pts, int64_t n_total, c
         const int64_t st = fa.stride;
 #pragma unroll
         for (int i = 0; i < C::PPL; i++) {
-            const int p = gl + G * i;
             if (!isface[i]) continue;
-            int fi = popc64(fm & ((1ull << p) - 1ull));
-            if (BALL && p >= first_ball) {
+            const int r = gl + G * i;
+            const int32_t pv = sm.pvid[fp[i]];
+            int fi = popc64(fm & ((1ull << r) - 1ull));
+            if (BALL && r >= fb_rank) {
                 // faces of the completion's planes in (distance, input
                 // index) order, after the row's
-                const uint32_t zp = (uint32_t)sm.pvid[p];
+                const uint32_t zp = (uint32_t)pv;
                 const double kp = dist2<D>(pts + (size_t)D * zp, pts + (size_t)D * sid);
-                fi = popc64(first_ball >= 64 ? fm : (fm & ((1ull << first_ball) - 1ull)));
-                for (int q = first_ball; q < nb_v; q++) {
-                    if (q == p || !((fm >> q) & 1ull)) continue;
-                    const uint32_t zq = (uint32_t)sm.pvid[q];
+                fi = popc64(fb_rank >= 64 ? fm : (fm & ((1ull << fb_rank) - 1ull)));
+                for (int q = fb_rank; q < nface; q++) {
+                    if (q == r || !((fm >> q) & 1ull)) continue;
+                    const uint32_t zq = (uint32_t)sm.pvid[sm.plist[q]];
                     const double kq = dist2<D>(pts + (size_t)D * zq, pts + (size_t)D * sid);
                     if (kq < kp || (kq == kp && bg.perm[zq] < bg.perm[zp])) fi++;
                 }
             }
             const int64_t at = (int64_t)fi * st + sid;
-            fa.nbr[at] = pv[i];
-            if (fa.nbr_cm) fa.nbr_cm[(int64_t)sid * FACE_SLOTS + fi] = pv[i];
+            fa.nbr[at] = pv;
+            if (fa.nbr_cm) fa.nbr_cm[(int64_t)sid * FACE_SLOTS + fi] = pv;
             fa.area[at] = farea[i];
             const int64_t plane_stride = st * FACE_SLOTS;
             fa.nrm[at] = nx[i];
