@@ -253,8 +253,7 @@ struct BKnnArgs {
 
 template <int DIM, int M>
 __global__ void __launch_bounds__(64, (M <= 2 ? 6 : 5)) k_bknn_wave(BKnnArgs args) {
-    __shared__ int32_t c_start[64], c_pfx[65];
-    __shared__ KnnPend pend;
+    __shared__ KnnSmem<M> smem;
     const int64_t nq = *args.nq_dev;
     const int chunk = ticket_chunk(nq, KNN_CHUNK);
     bool first = true;
@@ -275,7 +274,7 @@ __global__ void __launch_bounds__(64, (M <= 2 ? 6 : 5)) k_bknn_wave(BKnnArgs arg
             uint32_t lo = 0;
             tail_of(tail, q, k, kp, lo);
             knn_wave_query<DIM, M>(A->sorted, A->perm, A->N[b], A->coff[b], A->starts, A->counts, q, k,
-                                   A->out + (size_t)qi * k, c_start, c_pfx, &pend, kp, lo);
+                                   A->out + (size_t)qi * k, smem, kp, lo);
             __syncthreads();
         }
     }
@@ -582,7 +581,7 @@ void bknn_dim(const double* sorted, const uint32_t* perm, const int32_t* sbox, c
               const int64_t* coff, const int32_t* starts, const int32_t* counts, const uint32_t* q,
               const int64_t* nq_dev, int64_t cap, int k, uint32_t* out, int wave_min_k, int blocks_per_cu,
               unsigned long long* ticket, hipStream_t s, KnnTail tail) {
-    if (k >= wave_min_k) {
+    if (k >= wave_min_k || knn_wave_faster(DIM, cap, k)) {
         if (k <= 64) bknn_wave<DIM, 1>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, s, tail);
         else if (k <= 128) bknn_wave<DIM, 2>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, s, tail);
         else if (k <= 192) bknn_wave<DIM, 3>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, s, tail);

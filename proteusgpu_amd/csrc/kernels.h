@@ -76,11 +76,24 @@ struct KnnTail {
     int32_t tag = 0;
 };
 
+// Whether the wave-per-query kernel beats the per-thread heap for nq queries
+// with rows of k < 20.  The heap is a chain of one thread's LDS updates
+// (2D k = 16: 170 us for 2,000 to 100,000 queries, wave 17 to 99 us) that full
+// launches of short rows hide: at 1.4M queries 2D k = 16 1150 us (wave 1138),
+// k = 12 769 (1081), k = 8 447 (1050); 3D k = 16 2481 (1442), k = 12 1637
+// (1369), k = 8 1095 (1348).
+inline bool knn_wave_faster(int dim, int64_t nq, int k) { return k >= (dim == 2 ? 16 : 12) || nq <= 400000; }
+
 // k nearest neighbours of queries (sorted ids; nullptr = all n points).
 // Rows ascending by (FP64 dist^2, original index); out row stride k.
 void launch_knn(int dim, const double* sorted, const uint32_t* perm, int64_t n, int N,
                 const int32_t* starts, const int32_t* counts, const uint32_t* queries, int64_t nq,
                 int k, uint32_t* out, hipStream_t s, KnnTail tail = {}, SubGrid sg = {});
+
+// launch_knn's rows of more than 256 (knn_long.hip).
+void launch_knn_long(int dim, const double* sorted, const uint32_t* perm, int N, const int32_t* starts,
+                     const int32_t* counts, const uint32_t* queries, int64_t nq, int k, uint32_t* out, KnnTail tail,
+                     SubGrid sg, hipStream_t s);
 
 // ------------------------------------------------------------- voronoi.hip
 struct FaceArrays {

@@ -12,7 +12,7 @@
 // neighbour set is the same.
 #include "common.h"
 #include "kernels.h"
-#include "knn_core.h"
+#include "knn_wave.h"
 
 namespace pg {
 namespace {
@@ -31,43 +31,6 @@ __global__ void __launch_bounds__(BLOCK)
     knn_heap_query<DIM, BLOCK>(sorted, perm, N, 0, starts, counts, q, k, out + (size_t)qi * k, hd, hi);
 }
 
-// waves per SIMD the register budget is sized for: 6 for rows up to 128,
-// 5 up to 256; the long restart rows (up to 1024) are rare
-template <int M>
-constexpr int knn_wave_occupancy() { return M <= 2 ? 6 : (M <= 4 ? 5 : 2); }
-
-// SUB: the grid has crowded cells with sub-grids (a separate instance, so
-// that the uniform case keeps its registers)
-template <int DIM, int M, bool SUB>
-__global__ void __launch_bounds__(64, knn_wave_occupancy<M>())
-    k_knn_wave(const double* __restrict__ sorted, const uint32_t* __restrict__ perm, int N,
-               const int32_t* __restrict__ starts, const int32_t* __restrict__ counts,
-               const uint32_t* __restrict__ queries, int64_t nq, int k, uint32_t* __restrict__ out,
-               KnnTail tail, SubGrid sg) {
-    __shared__ int32_t c_start[64], c_pfx[65];
-    __shared__ KnnPend pend;
-    const int64_t qi = xcd_block(blockIdx.x, gridDim.x);
-    if (qi >= nq) return;  // whole block
-    const uint32_t q = queries ? queries[qi] : (uint32_t)qi;
-    int kp = 0;
-    uint32_t lo = 0;
-    tail_of(tail, q, k, kp, lo);
-    knn_wave_query<DIM, M, SUB>(sorted, perm, N, 0, starts, counts, q, k, out + (size_t)qi * k, c_start, c_pfx,
-                                &pend, kp, lo, sg);
-}
-
-template <int DIM, int M>
-void run_wave(const double* sorted, const uint32_t* perm, int N, const int32_t* starts,
-              const int32_t* counts, const uint32_t* queries, int64_t nq, int k, uint32_t* out,
-              KnnTail tail, SubGrid sg, hipStream_t s) {
-    if (sg.m != nullptr)
-        k_knn_wave<DIM, M, true><<<(unsigned)nq, 64, 0, s>>>(sorted, perm, N, starts, counts, queries, nq, k, out,
-                                                             tail, sg);
-    else
-        k_knn_wave<DIM, M, false><<<(unsigned)nq, 64, 0, s>>>(sorted, perm, N, starts, counts, queries, nq, k, out,
-                                                              tail, sg);
-}
-
 template <int DIM>
 void dispatch_wave(const double* sorted, const uint32_t* perm, int N, const int32_t* starts,
                    const int32_t* counts, const uint32_t* queries, int64_t nq, int k, uint32_t* out,
@@ -78,8 +41,7 @@ void dispatch_wave(const double* sorted, const uint32_t* perm, int N, const int3
     else if (k <= 128) run_wave<DIM, 2>(sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
     else if (k <= 192) run_wave<DIM, 3>(sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
     else if (k <= 256) run_wave<DIM, 4>(sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
-    else if (k <= 512) run_wave<DIM, 8>(sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
-    else run_wave<DIM, 16>(sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
+    else launch_knn_long(DIM, sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
 }
 
 template <int DIM, int BLOCK>
@@ -101,15 +63,15 @@ void launch_knn(int dim, const double* sorted, const uint32_t* perm, int64_t n, 
                 int k, uint32_t* out, hipStream_t s, KnnTail tail, SubGrid sg) {
     (void)n;
     if (nq <= 0) return;
-    // Long rows (and short query lists) go to the wave-per-query kernel; the
-    // threshold can be moved with PGPU_KNN_WAVE_MIN_K for tuning runs.
+    // Long rows and short query lists go to the wave-per-query kernel; the row
+    // length can be moved with PGPU_KNN_WAVE_MIN_K for tuning runs.
     static const int wave_min_k = [] {
         const char* e = getenv("PGPU_KNN_WAVE_MIN_K");
         return e ? atoi(e) : 20;
     }();
     // the LDS heap holds at most 256 entries per query, and only the wave
     // kernel takes crowded cells through their sub-grids
-    if (k >= wave_min_k || k > 256 || sg.m != nullptr) {
+    if (k >= wave_min_k || k > 256 || sg.m != nullptr || knn_wave_faster(dim, nq, k)) {
         if (dim == 2) dispatch_wave<2>(sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
         else dispatch_wave<3>(sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
         return;

@@ -175,9 +175,7 @@ PG_DEV void knn_heap_query(const double* __restrict__ sorted, const uint32_t* __
 // by a bitonic network and merged into the kept list, one 64-entry slot at
 // a time (lower half of slot + reversed batch stays, the upper half carries
 // into the next slot).
-// Same rows and same total order as k_knn, no LDS heap, full waves: used
-// for rows of 20 and more, where the per-thread heap would leave the CUs
-// nearly empty.
+// Same rows and same total order as k_knn, no LDS heap, full waves.
 
 PG_DEV bool cand_less(double da, uint32_t oa, double db, uint32_t ob) {
     return da < db || (da == db && oa < ob);
@@ -254,6 +252,28 @@ struct KnnPend {
     uint32_t s[128];
 };
 
+// Candidates of the row search (knn_rows_query): key and sorted id, up to CAP.
+template <int M>
+struct KnnRows {
+    static constexpr int BITS = M <= 2 ? 8 : 9;  // bits of a candidate's position in its key
+    static constexpr int CAP = 1 << BITS;
+    uint32_t key[CAP], id[CAP];
+    int32_t shift[64];  // per row of cells: first sorted id minus the row's first candidate index
+    uint32_t mark[64];  // rows starting in the current 64 candidates
+};
+
+// LDS of one wave query.
+template <int M>
+struct KnnSmem {
+    union {
+        struct {
+            int32_t c_start[64], c_pfx[65];
+            KnnPend pend;
+        };
+        KnnRows<M> rows;
+    };
+};
+
 // Merge 64 candidates (one per lane, unsorted, +inf padded) into the kept
 // list (slot-major, ascending): sort them across the wave (bitonic), then,
 // slot by slot, the lower half of (slot, batch) stays and the upper half
@@ -321,8 +341,250 @@ PG_DEV double knn_guess_r2(const double (&p)[3], int N, int cnt, int nin, float 
     return (double)R * (double)R;
 }
 
-// One query by the 64 lanes of a one-wave block; c_start / c_pfx are the
-// block's LDS tables (64 and 65 entries), pend its candidate buffer.  Grid
+// ---- 32-bit keys across the wave (ascending with the lane index)
+//
+// Compare-exchange with lane l ^ X: the lane whose bit B is clear keeps the
+// smaller key of the pair.
+template <int X, int B>
+PG_DEV void key_cx(uint32_t& a, int l) {
+    const uint32_t b = lane_xor<X>(a);
+    const uint32_t lo = min(a, b), hi = max(a, b);
+    a = (l & B) ? hi : lo;
+}
+template <int J>
+PG_DEV void key_half_clean(uint32_t& a, int l) {
+    if constexpr (J >= 1) {
+        key_cx<J, J>(a, l);
+        key_half_clean<J / 2>(a, l);
+    }
+}
+template <int K>
+PG_DEV void key_sort_phase(uint32_t& a, int l) {
+    key_cx<K - 1, K / 2>(a, l);
+    key_half_clean<K / 4>(a, l);
+    if constexpr (K < 64) key_sort_phase<2 * K>(a, l);
+}
+// Merge 64 unsorted keys into the M x 64 smallest kept (slot-major,
+// ascending; padding ~0); out: the smallest key this lane saw leave the list.
+template <int M>
+PG_DEV void key_merge_batch(uint32_t (&kk)[M], uint32_t& out, uint32_t a, int l, bool first) {
+    key_sort_phase<2>(a, l);
+    if (first) {
+        kk[0] = a;
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        const uint32_t r = lane_xor<63>(a);
+        const uint32_t hi = max(kk[j], r);
+        kk[j] = min(kk[j], r);
+        key_half_clean<32>(kk[j], l);
+        if (j + 1 < M) {
+            a = hi;
+            key_half_clean<32>(a, l);
+        } else {
+            out = min(out, hi);
+        }
+    }
+}
+
+// One query by rows of grid cells.  The cells of a row (consecutive along
+// x) hold consecutive sorted points, so the ball of squared radius r2 around
+// the query is covered by one run of points per row it reaches: a lane takes
+// a row, bounds its run by the ball's half width there, and the runs'
+// points are spread over the lanes (a mark at every run's first candidate
+// and a max-scan give each lane its row).  The points inside the ball wait in
+// LDS under a 32-bit key, their squared distance quantized (monotone) above
+// their position in the buffer; the keys are sorted across the wave with
+// integer min / max.  Equal quantized distances among the kept ranks are put in
+// the exact (d^2, input index) order afterwards.
+//
+// false: nothing was written, and the ring walk has to answer: fewer than k
+// points after a second, wider ball, more than the buffer or the row limit
+// holds, a candidate below its ring's distance bound (the argument of
+// knn_wave_query), or ties that reach past the kept keys.  With the ball's k
+// first in order the row is the ring walk's by the same argument: the rows
+// skip only points outside the ball (the float bounds carry a slack of
+// several float roundings of N), so every point of the ball is seen.
+//
+// What bounds it: VALU issue (810 instructions per query, k = 32 and its 64
+// tails; the ring walk with FP64 sorts took 1.75k).  1M uniform 3D queries:
+// k = 32 2.4 -> 1.18 ms, k = 64 3.25 -> 1.50 ms.  One run of points per row
+// of cells replaces 27 and then 98 cells looked at one by one, the mark scan a
+// binary search per candidate, and an exchange of the sort takes three
+// integer instructions instead of a dozen.
+template <int DIM, int M>
+PG_DEV bool knn_rows_query(const double* __restrict__ sorted, const uint32_t* __restrict__ perm, int N, int64_t cbase,
+                           const int32_t* __restrict__ starts, const int32_t* __restrict__ counts, uint32_t q, int k,
+                           uint32_t* __restrict__ o, KnnRows<M>& sm, const double (&p)[3], const double (&P)[3],
+                           double r2, float lam, int kp, double lo_d, uint32_t lo_s) {
+    const int l = threadIdx.x;
+    constexpr int BITS = KnnRows<M>::BITS, CAP = KnnRows<M>::CAP, QB = 32 - BITS;
+    const float Px = (float)P[0], Py = (float)P[1], Pz = (float)P[2];
+    const float slack = 1e-4f + 4e-7f * (float)N;
+    int n = 0;
+    bool odd = false;
+    for (int pass = 0;; pass++) {
+        const float Rc = __builtin_amdgcn_sqrtf((float)r2) * 1.00001f * (float)N + slack;  // in cells
+        const int jlo = max(0, min(N - 1, (int)floorf(Py - Rc))), jhi = max(0, min(N - 1, (int)floorf(Py + Rc)));
+        const int klo = DIM == 3 ? max(0, min(N - 1, (int)floorf(Pz - Rc))) : 0;
+        const int khi = DIM == 3 ? max(0, min(N - 1, (int)floorf(Pz + Rc))) : 0;
+        const int nj = jhi - jlo + 1, nrows = nj * (khi - klo + 1);
+        if (nrows > 256) return false;
+        const float rnj = 1.0f / (float)nj;
+        const float rr2 = Rc * Rc;
+        // the smallest quantum that keeps every d^2 <= r2 below 2^QB
+        const double base_d = kp > 0 ? lo_d : 0.0;
+        const double qs = (double)(1u << (QB - 1)) * 1.999 / (r2 - base_d);
+        n = 0;
+        odd = false;
+        for (int rb = 0; rb < nrows; rb += 64) {
+            const int t = rb + l;
+            const int dk = DIM == 3 ? idiv_small(t, nj, rnj) : 0;
+            const int j = jlo + t - dk * nj, kk = klo + dk;
+            float w2 = rr2;
+            {
+                // cells on the grid's border are open outwards
+                const float g = fmaxf(fmaxf(j == 0 ? 0.f : (float)j - Py, j == N - 1 ? 0.f : Py - (float)(j + 1)), 0.f);
+                w2 -= g * g;
+            }
+            if (DIM == 3) {
+                const float g =
+                    fmaxf(fmaxf(kk == 0 ? 0.f : (float)kk - Pz, kk == N - 1 ? 0.f : Pz - (float)(kk + 1)), 0.f);
+                w2 -= g * g;
+            }
+            int st = 0, cnt = 0;
+            if (t < nrows && w2 >= 0.f) {
+                const float hx = __builtin_amdgcn_sqrtf(w2) * 1.00001f + slack;
+                const int ilo = max(0, min(N - 1, (int)floorf(Px - hx)));
+                const int ihi = max(0, min(N - 1, (int)floorf(Px + hx)));
+                const int64_t c = cbase + (int64_t)j * N + (int64_t)kk * N * N;
+                st = starts[c + ilo];
+                cnt = starts[c + ihi] + counts[c + ihi] - st;
+            }
+            const int incl = wave_incl_sum(cnt);
+            const int total = (int)read_lane((uint32_t)incl, 63);
+            const int first = incl - cnt;
+            sm.shift[l] = st - first;
+            uint32_t row = 0;  // 1 + the row of the last candidate so far
+            for (int cb = 0; cb < total; cb += 64) {
+                sm.mark[l] = 0u;
+                __syncthreads();
+                if (cnt > 0 && first >= cb && first < cb + 64) sm.mark[first - cb] = (uint32_t)l + 1u;
+                __syncthreads();
+                const uint32_t rw = max(wave_incl_max(sm.mark[l]), row);
+                row = read_lane(rw, 63);
+                const int cj = cb + l;
+                bool take = false, near = false;
+                double d = 0.0;
+                uint32_t cs = 0;
+                if (cj < total) {
+                    cs = (uint32_t)(sm.shift[rw - 1u] + cj);
+                    double pc[3] = {0, 0, 0};
+#pragma unroll
+                    for (int e = 0; e < DIM; e++) pc[e] = sorted[(size_t)DIM * cs + e];
+                    d = dist2<DIM>(p, pc);
+                    take = d <= r2 && cs != q;
+                    if (kp > 0) take = take && (d > lo_d || (d == lo_d && ent_less(perm, lo_d, lo_s, d, cs)));
+                    // within rounding of a ring's edge: checked exactly below
+                    const float u = __builtin_amdgcn_sqrtf((float)d) * (float)N;
+                    near = take && fabsf(u - rintf(u)) < 2e-6f * fmaxf(u, 1.0f);
+                }
+                if (__ballot(near) != 0ull) {
+                    if (near) {
+                        double pc[3] = {0, 0, 0};
+#pragma unroll
+                        for (int e = 0; e < DIM; e++) pc[e] = sorted[(size_t)DIM * cs + e];
+                        const int a = grid_cell<DIM>(p, N), b = grid_cell<DIM>(pc, N);
+                        int ring = max(abs(a % N - b % N), abs((a / N) % N - (b / N) % N));
+                        if (DIM == 3) ring = max(ring, abs(a / (N * N) - b / (N * N)));
+                        const double md = (double)(ring - 1) / (double)N;
+                        odd = odd || (ring >= 2 && d < md * md);
+                    }
+                }
+                const uint64_t surv = (uint64_t)__ballot(take);
+                const int ns = __popcll((unsigned long long)surv);
+                if (n + ns > CAP) return false;
+                if (take) {
+                    const int at = n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(surv >> 32),
+                                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)surv, 0u));
+                    sm.key[at] = (uint32_t)((d - base_d) * qs) << BITS | (uint32_t)at;
+                    sm.id[at] = cs;
+                }
+                n += ns;
+            }
+            __syncthreads();
+        }
+        if (__ballot(odd) != 0ull) return false;
+        if (n >= k) break;
+        if (pass >= 1) return false;
+        // fewer than k points in the ball: a wider one
+        const float g = __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(lam / ((float)(kp + n) + 1.0f)) * (2.0f / DIM));
+        r2 *= (double)fminf(fmaxf(g, 1.5f), 16.0f);
+    }
+    uint32_t kk[M], out = ~0u;
+#pragma unroll
+    for (int j = 0; j < M; j++) kk[j] = ~0u;
+    for (int b = 0; b < n; b += 64) key_merge_batch<M>(kk, out, b + l < n ? sm.key[b + l] : ~0u, l, b == 0);
+    if (n > 64 * M) {
+        // a key that left the list ties with the last kept rank
+        uint32_t kth = 0;
+#pragma unroll
+        for (int j = 0; j < M; j++)
+            if (j == (k - 1) >> 6) kth = read_lane(kk[j], (k - 1) & 63);
+        if (__ballot((out >> BITS) <= (kth >> BITS)) != 0ull) return false;
+    }
+    // equal quantized distances at neighbouring ranks, up to rank k
+    bool tie = false;
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        uint32_t nx = (uint32_t)__shfl_down((int)kk[j], 1, 64);
+        if (j + 1 < M) {
+            const uint32_t h = read_lane(kk[j + 1 < M ? j + 1 : j], 0);
+            if (l == 63) nx = h;
+        } else if (l == 63) {
+            nx = ~kk[j];
+        }
+        const int r = 64 * j + l;
+        tie = tie || (r < k && r + 1 < n && (nx >> BITS) == (kk[j] >> BITS));
+    }
+    uint32_t id[M];
+#pragma unroll
+    for (int j = 0; j < M; j++) id[j] = 64 * j + l < n ? sm.id[kk[j] & (CAP - 1)] : 0xffffffffu;
+    if (__ballot(tie) != 0ull) {
+        if (M > 1) return false;  // ties in longer rows: the ring walk's
+        double d = __builtin_inf();
+        if (l < n) {
+            double pc[3] = {0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < DIM; e++) pc[e] = sorted[(size_t)DIM * id[0] + e];
+            d = dist2<DIM>(p, pc);
+        }
+        // odd-even transpositions in the exact order (already in order but
+        // for the ties) until nothing moves
+        for (int still = 0, ph = 0; still < 2; ph ^= 1) {
+            const int pl = ((l + ph) ^ 1) - ph;
+            const int src = pl < 0 || pl > 63 ? l : pl;
+            const double pd = __shfl(d, src, 64);
+            const uint32_t pi = (uint32_t)__shfl((int)id[0], src, 64);
+            const bool up = src > l;
+            const bool swap = src != l && src < n && l < n && (up ? ent_less(perm, pd, pi, d, id[0]) : ent_less(perm, d, id[0], pd, pi));
+            if (swap) {
+                d = pd;
+                id[0] = pi;
+            }
+            still = __ballot(swap) != 0ull ? 0 : still + 1;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < M; j++)
+        if (64 * j + l < k) o[64 * j + l] = id[j];
+    return true;
+}
+
+// One query by the 64 lanes of a one-wave block.  Without sub-grids and for
+// rows of up to 256 the search by rows (knn_rows_query) answers nearly all
+// queries; the ring walk below the others.  Grid
 // cells of the query's box are cbase + i + j N + k N^2.  kp > 0: the first
 // kp neighbours are known, lo_s (sorted id) the last of them; only
 // neighbours kp..k-1 are found (candidates up to lo_s in the order are
@@ -352,9 +614,11 @@ template <int DIM, int M, bool SUB = false>
 PG_DEV void knn_wave_query(const double* __restrict__ sorted, const uint32_t* __restrict__ perm, int N,
                            int64_t cbase, const int32_t* __restrict__ starts,
                            const int32_t* __restrict__ counts, uint32_t q, int k, uint32_t* __restrict__ o,
-                           int32_t* c_start, int32_t* c_pfx, KnnPend* pend, int kp = 0, uint32_t lo_s = 0,
-                           SubGrid sg = {}) {
+                           KnnSmem<M>& smem, int kp = 0, uint32_t lo_s = 0, SubGrid sg = {}) {
     const int l = threadIdx.x;
+    int32_t* const c_start = smem.c_start;
+    int32_t* const c_pfx = smem.c_pfx;
+    KnnPend* const pend = &smem.pend;
     double p[3] = {0, 0, 0};
 #pragma unroll
     for (int d = 0; d < DIM; d++) p[d] = sorted[(size_t)DIM * q + d];
@@ -423,6 +687,12 @@ PG_DEV void knn_wave_query(const double* __restrict__ sorted, const uint32_t* __
         }
         const int tot = (int)read_lane((uint32_t)wave_incl_sum(cnt), 63);
         r2 = knn_guess_r2<DIM>(p, N, tot, __popcll((unsigned long long)__ballot(in)), lam);
+    }
+    if (!SUB && M <= 4) {
+        if (knn_rows_query<DIM, M>(sorted, perm, N, cbase, starts, counts, q, k, o, smem.rows, p, P, r2, lam, kp, lo_d,
+                                   lo_s))
+            return;
+        __syncthreads();
     }
     bool odd_l = false;  // a kept candidate below its ring's distance bound
     // Candidates 0 .. total-1 of the cells (or sub-cells) in c_start / c_pfx

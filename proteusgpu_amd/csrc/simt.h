@@ -73,6 +73,19 @@ __device__ __forceinline__ int wave_incl_sum(int x) {
     return x;
 }
 
+// Inclusive prefix maximum over the 64 lanes, every lane active (as
+// wave_incl_sum).
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v) {
+    uint32_t x = v;
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false));
+    return x;
+}
+
 // Butterfly over groups of G <= 16 lanes (DPP), every lane active: x is
 // combined with lane l ^ 1, then l ^ 2, .. l ^ G/2, as op(theirs, mine).
 template <int G, class F>
