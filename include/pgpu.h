@@ -105,7 +105,8 @@ int pg_knn_solve_noalloc(pg_ctx* ctx, int dim, const double* pts, int64_t n, int
  * read once at the start of each build
  * (no reference counterpart; results never depend on it): lanes per seed
  * (8 or 16) and vertex slots per seed (48 or 64; seeds that outgrow them
- * are recomputed by a 128-slot kernel).  Default 16 x 64, or PGPU_CLIP_CFG. */
+ * are recomputed by a 128-slot kernel).  Default 16 x 64, or PGPU_CLIP_CFG.
+ * 3D: 2D clips have one shape, 8 lanes x 16 slots. */
 int pg_set_clip_config(int lanes, int slots);
 int pg_get_clip_config(int* lanes, int* slots);
 
@@ -392,8 +393,8 @@ int pg_mesh_compute_k(pg_ctx* ctx, const pg_mesh_params* params, const pg_kmodel
  * point and state arrays; coordinates of every box lie in its own unit box.
  * Every box needs more than max(k, k_max) + 1 points. */
 typedef struct {
-    int clip_lanes;      /* lanes per seed of the fast clip kernel: 8 or 16         */
-    int clip_slots;      /* vertex slots per seed of the fast clip kernel: 48 or 64 */
+    int clip_lanes;      /* lanes per seed of the fast 3D clip kernel: 8 or 16         */
+    int clip_slots;      /* vertex slots per seed of the fast 3D clip kernel: 48 or 64 */
     int knn_wave_min_k;  /* rows at least this long always use the wave-per-query
                           * KNN (shorter ones where it is the faster one)        */
     int blocks_per_cu;   /* resident blocks per CU of the persistent KNN and clip

@@ -277,13 +277,19 @@ int64_t collect_list(pg_mesh* m, const uint32_t* seeds, int64_t nq, int code, ui
 }
 
 // The shape tag under which the fast clip kernel saves and resumes cells.
-int32_t clip_shape_tag(int lanes, int slots) { return (lanes << 24) | ((slots / lanes) << 16); }
+int32_t clip_shape_tag(int dim, int lanes, int slots) {
+    if (dim == 2) {
+        lanes = pg::CLIP2D_LANES;
+        slots = pg::CLIP2D_SLOTS;
+    }
+    return (lanes << 24) | ((slots / lanes) << 16);
+}
 
 void run_list(pg_mesh* m, const uint32_t* list, int64_t nq, int k, int big, hipStream_t s, bool exact = false) {
     uint32_t* rows = m->rows.get<uint32_t>((size_t)nq * k);
     pg::KnnTail tail;  // seeds that resume need only the rest of their row
     if (m->use_resume && !big && !exact)
-        tail = {m->resume.as<int32_t>(), m->lastnb.as<uint32_t>(), clip_shape_tag(m->lanes, m->slots)};
+        tail = {m->resume.as<int32_t>(), m->lastnb.as<uint32_t>(), clip_shape_tag(m->prm.dim, m->lanes, m->slots)};
     pg::launch_knn(m->prm.dim, m->g.sorted.as<double>(), m->g.perm.as<uint32_t>(), m->n_seeds, m->g.N,
                    m->g.starts.as<int32_t>(), m->g.counts.as<int32_t>(), list, nq, k, rows, s, tail, m->g.sub());
     pg::FaceArrays fa = m->faces();
@@ -1926,19 +1932,18 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
     auto knn = [&](const uint32_t* q, const int64_t* nq, int k, bool big) {
         pg::KnnTail tail;  // seeds that resume need only the rest of their row
         if (B->resume.p && !big)
-            tail = {B->resume.as<int32_t>(), B->lastnb.as<uint32_t>(), clip_shape_tag(B->lanes, B->slots)};
+            tail = {B->resume.as<int32_t>(), B->lastnb.as<uint32_t>(), clip_shape_tag(dim, B->lanes, B->slots)};
         pg::launch_bknn(dim, B->sorted.as<double>(), B->perm.as<uint32_t>(), B->sorted_box.as<int32_t>(),
                         B->N.as<int32_t>(), B->coff.as<int64_t>(), B->starts.as<int32_t>(), B->counts.as<int32_t>(),
                         q, nq, cap, k, B->knn.as<uint32_t>(), B->wave_min_k, B->bpc,
                         B->ticket.as<unsigned long long>(), s, tail);
     };
-    // 3D first pass and learned buckets: one block per seed group (the 3D
-    // clip spills in a persistent loop); the short restart lists, and every
-    // 2D list (whose clip does not spill): persistent blocks
+    // first pass and learned buckets: one block per seed group (the clip
+    // spills in a persistent loop); the short restart lists: persistent blocks
     auto clip = [&](const uint32_t* q, const int64_t* nq, int k, int big, bool restart_list) {
         pg::launch_bvoronoi(dim, B->sorted.as<double>(), q, nq, cap, B->knn.as<uint32_t>(), k, p.max_p, p.max_t, big,
                             B->lanes, B->slots, B->faces(), B->bpc, B->ticket.as<unsigned long long>(),
-                            restart_list || dim == 2, s);
+                            restart_list, s);
     };
     auto collect = [&](const uint32_t* L, const int64_t* nL, int code, uint32_t* out, int64_t* nout) {
         pg::launch_bcollect(nL, cap, L, B->status.as<int32_t>(), code, out, B->flags.as<int32_t>(),

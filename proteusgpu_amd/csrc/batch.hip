@@ -189,7 +189,6 @@ PG_DEV int ticket_chunk(int64_t items, int most) {
     return (int)(c < 1 ? 1 : (c > most ? most : c));
 }
 constexpr int KNN_CHUNK = 16;  // queries per ticket, at most
-constexpr int CLIP_CHUNK = 2;  // seed groups per ticket, at most
 
 // Resident one-wave blocks of a kernel on the device (its occupancy per CU,
 // capped at blocks_per_cu, times the CUs).
@@ -289,39 +288,21 @@ __global__ void __launch_bounds__(64, (M <= 2 ? 6 : 5)) k_bknn_wave(BKnnArgs arg
 // across groups, and the clip's registers spill: it suits the short lists
 // of the certificate restarts, where capacity-sized grids would be mostly
 // empty blocks).
-// FRESH: the arguments are re-read per group (3D: fewer spills); else they
-// stay in registers across groups (2D, whose clip has room for them).
-template <int DIM, int G, int S, bool FRESH>
+// The arguments are re-read per group (fewer spills).
+template <int DIM, int G, int S>
 __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_bvoronoi_loop(ClipArgs args) {
     using C = VoroCfg<DIM, G, S>;
     __shared__ VoroSmem<DIM, G, S> sm[C::SPW];
-    if constexpr (FRESH) {
-        bool first = true;
-        for (;;) {
-            const auto* A0 = fresh_args<ClipArgs>();
-            const int64_t nvb = (*A0->nq_dev + C::SPW - 1) / C::SPW;
-            const int64_t vb = next_ticket(A0->ticket, 1, first);
-            if (vb >= nvb) break;
-            const auto* A = fresh_args<ClipArgs>();
-            voronoi_group<DIM, G, S>(A->pts, INT64_MAX, A->seeds, *A->nq_dev, A->knn, A->k, A->max_p, A->max_t,
-                                     A->fa.resume, A->fa.cstate, A->fa.key, sm, vb);
-            __syncthreads();
-        }
-    } else {
-        const int64_t nq = *args.nq_dev;
-        const int64_t nvb = (nq + C::SPW - 1) / C::SPW;
-        const int chunk = ticket_chunk(nvb, CLIP_CHUNK);
-        bool first = true;
-        for (;;) {
-            const int64_t b0 = next_ticket(args.ticket, chunk, first);
-            if (b0 >= nvb) break;
-            const int64_t b1 = b0 + chunk < nvb ? b0 + chunk : nvb;
-            for (int64_t vb = b0; vb < b1; vb++) {
-                voronoi_group<DIM, G, S>(args.pts, INT64_MAX, args.seeds, nq, args.knn, args.k, args.max_p,
-                                         args.max_t, args.fa.resume, args.fa.cstate, args.fa.key, sm, vb);
-                __syncthreads();
-            }
-        }
+    bool first = true;
+    for (;;) {
+        const auto* A0 = fresh_args<ClipArgs>();
+        const int64_t nvb = (*A0->nq_dev + C::SPW - 1) / C::SPW;
+        const int64_t vb = next_ticket(A0->ticket, 1, first);
+        if (vb >= nvb) break;
+        const auto* A = fresh_args<ClipArgs>();
+        voronoi_group<DIM, G, S>(A->pts, INT64_MAX, A->seeds, *A->nq_dev, A->knn, A->k, A->max_p, A->max_t,
+                                 A->fa.resume, A->fa.cstate, A->fa.key, sm, vb);
+        __syncthreads();
     }
 }
 
@@ -599,12 +580,11 @@ void bclip(const double* pts, const uint32_t* seeds, const int64_t* nq_dev, int6
     using C = VoroCfg<DIM, G, S>;
     const ClipArgs args{pts, INT64_MAX, seeds, 0, nq_dev, knn, ticket, fa, k, max_p, max_t};
     if (loop) {
-        constexpr bool FRESH = DIM == 3;
-        static const int occ = occupancy(k_bvoronoi_loop<DIM, G, S, FRESH>);
+        static const int occ = occupancy(k_bvoronoi_loop<DIM, G, S>);
         const unsigned nb =
             (unsigned)std::min<int64_t>((cap + C::SPW - 1) / C::SPW, resident_blocks(occ, blocks_per_cu));
         k_fill<unsigned long long><<<1, TB, 0, s>>>(ticket, 1, 0ull);
-        k_bvoronoi_loop<DIM, G, S, FRESH><<<std::max(nb, 1u), 64, 0, s>>>(args);
+        k_bvoronoi_loop<DIM, G, S><<<std::max(nb, 1u), 64, 0, s>>>(args);
         return;
     }
     const unsigned nb = (unsigned)std::max<int64_t>((cap + C::SPW - 1) / C::SPW, 1);
@@ -630,6 +610,7 @@ void launch_bvoronoi(int dim, const double* sorted, const uint32_t* seeds, const
     auto go = [&](auto dimc) {
         constexpr int D = decltype(dimc)::value;
         if (big) bclip<D, 16, 8>(sorted, seeds, nq_dev, cap, knn, k, max_p, max_t, fa, blocks_per_cu, ticket, loop, s);
+        else if constexpr (D == 2) bclip<2, CLIP2D_LANES, CLIP2D_SLOTS / CLIP2D_LANES>(sorted, seeds, nq_dev, cap, knn, k, max_p, max_t, fa, blocks_per_cu, ticket, loop, s);
         else if (lanes == 8 && slots == 48) bclip<D, 8, 6>(sorted, seeds, nq_dev, cap, knn, k, max_p, max_t, fa, blocks_per_cu, ticket, loop, s);
         else if (lanes == 8) bclip<D, 8, 8>(sorted, seeds, nq_dev, cap, knn, k, max_p, max_t, fa, blocks_per_cu, ticket, loop, s);
         else if (slots == 48) bclip<D, 16, 3>(sorted, seeds, nq_dev, cap, knn, k, max_p, max_t, fa, blocks_per_cu, ticket, loop, s);

@@ -152,7 +152,9 @@ void launch_voronoi_ball(int dim, const double* sorted, int64_t n, const uint32_
                          const int32_t* starts, const int32_t* counts, const uint32_t* perm, int kmark,
                          hipStream_t s, SubGrid sg = {});
 
-// Process-wide default shape of the fast clip kernel for the following
+// The fast 2D clip kernel's shape, whatever the configuration below.
+constexpr int CLIP2D_LANES = 8, CLIP2D_SLOTS = 16;
+// Process-wide default shape of the fast 3D clip kernel for the following
 // builds: lanes per seed (8 or 16) and vertex slots per seed (48 or 64).
 bool valid_clip_config(int lanes, int slots);
 void set_clip_config(int lanes, int slots);

@@ -76,15 +76,12 @@ __global__ void __launch_bounds__(TB) k_compact(int64_t nq, const uint32_t* seed
 
 }  // namespace
 
-// Vertex slots of the fast kernel per seed: 16 lanes x 4 (64 slots) or
-// 16 lanes x 3 (48 slots; less work per clip, more seeds overflow into the
-// 128-slot kernel).  Chosen by the autotuner or PGPU_CLIP_SLOTS.
-// Fast-kernel shape: lanes per seed x vertex slots per lane.  16 x 4 (64
+// Fast-kernel shape in 3D: lanes per seed x vertex slots per lane.  16 x 4 (64
 // slots, 4 seeds per wave), 16 x 3 (48 slots; less work per clip, a few
 // more seeds overflow into the 128-slot kernel), 8 x 6 and 8 x 8 (8 seeds
 // per wave: the group-wide work of a clip is shared by twice as many seeds,
 // at twice the LDS per wave).  Chosen by the autotuner or PGPU_CLIP_CFG
-// ("16x4", "16x3", "8x6", "8x8").
+// ("16x4", "16x3", "8x6", "8x8").  2D clips have one shape (CLIP2D_LANES).
 static std::atomic<int> g_clip_lanes{16}, g_clip_slots{64};
 static const bool g_clip_env = [] {
     const char* e = getenv("PGPU_CLIP_CFG");
@@ -120,6 +117,7 @@ void launch_dim(const ClipArgs& a, int big, hipStream_t s, bool restart, int lan
         using C = VoroCfg<DIM, 16, 8>;
         k_voronoi_exact<DIM><<<dim3((unsigned)((a.nq + C::SPW - 1) / C::SPW)), dim3(64), 0, s>>>(a);
     } else if (big) run<DIM, 16, 8>(a, true, s);
+    else if constexpr (DIM == 2) run<2, CLIP2D_LANES, CLIP2D_SLOTS / CLIP2D_LANES>(a, restart, s);
     else if (lanes == 8 && slots == 48) run<DIM, 8, 6>(a, restart, s);
     else if (lanes == 8) run<DIM, 8, 8>(a, restart, s);
     else if (slots == 48) run<DIM, 16, 3>(a, restart, s);

@@ -55,29 +55,46 @@ struct Plane {
     double x, y, z, w;
 };
 
-// Fast kernels (at most 64 vertex slots) hold 48 planes per seed, which
-// keeps a seed's LDS below 3.3 KB (three waves per SIMD); a seed that needs
-// more planes before max_p, or more vertex slots, is redone by the 128-slot
-// kernel, which holds the full 64 planes.
+// Fast kernels (at most 64 vertex slots) hold 48 planes per seed in 3D, which
+// keeps a seed's LDS below 3.4 KB (three waves per SIMD), and 24 in 2D; a
+// seed that needs more planes before max_p, or more vertex slots, is redone
+// by the 128-slot kernel, which holds the full 64 planes.  2D cells have six
+// vertices and a clip makes two: 8 lanes x 2 slots per seed, 8 seeds per
+// wave.  At 16 x 4, 4 seeds per wave, as in 3D, three lanes of four had
+// nothing to do: 1M uniform seeds at k = 16 2.66 -> 1.06 ms.
 template <int DIM, int G, int S>
 struct VoroCfg {
     static constexpr int NS = G * S;               // vertex slots per seed
     static constexpr int SPW = 64 / G;             // seeds per wave (= block)
-    static constexpr int MAXP = NS > 64 ? 64 : 48; // plane slots per seed
+    static constexpr int MAXP = NS > 64 ? 64 : (DIM == 3 ? 48 : 24);  // plane slots per seed
     static constexpr int NW = (NS + 63) / 64;      // 64-bit words of a slot mask
     static constexpr int PPL = MAXP / G;           // planes per lane at extraction
     // waves per SIMD the register budget is sized for: the 16-lane fast
-    // kernels fit three in LDS (under 3.4 KB per seed)
-    static constexpr int WAVES = (G == 16 && NS <= 64) ? 3 : 1;
+    // kernels fit three in LDS (under 3.4 KB per seed), the 2D one four
+    static constexpr int WAVES = NS > 64 ? 1 : (DIM == 2 ? 4 : (G == 16 ? 3 : 1));
     static_assert(NS <= 128, "slot ids are bytes below 255");
     static_assert(G <= 64 && 64 % G == 0, "groups tile the wave");
     static_assert(MAXP % G == 0, "planes tile the group");
 };
 
-template <int NS, int MAXP, int G>
+// A plane in LDS (2D: without z).
+template <int DIM>
+struct alignas(DIM == 3 ? 16 : 8) PlaneMem {
+    double v[DIM + 1];
+    PG_DEV PlaneMem& operator=(const Plane& p) {
+        v[0] = p.x;
+        v[1] = p.y;
+        if (DIM == 3) v[2] = p.z;
+        v[DIM] = p.w;
+        return *this;
+    }
+    PG_DEV operator Plane() const { return Plane{v[0], v[1], DIM == 3 ? v[2] : 0.0, v[DIM]}; }
+};
+
+template <int DIM, int NS, int MAXP, int G>
 struct SeedSmem {
     union {
-        Plane plane[MAXP];      // planes while clipping
+        PlaneMem<DIM> plane[MAXP];  // planes while clipping
         double vpos[3 * NS];    // vertex positions during extraction
     };
     float pn1[MAXP];        // |x|+|y|+|z|+|w| rounded up
@@ -89,10 +106,10 @@ struct SeedSmem {
         struct {
             uint32_t edge[NS];        // boundary edges of the current clip
             uint8_t newslot[NS];      // slot of the j-th new vertex
-            uint8_t by_start[MAXP];   // 3D: boundary edge starting at a plane
-            uint8_t by_end[MAXP];     // 3D: boundary edge ending at a plane
+            uint8_t by_start[DIM == 3 ? MAXP : 1];  // 3D: boundary edge starting at a plane
+            uint8_t by_end[DIM == 3 ? MAXP : 1];    // 3D: boundary edge ending at a plane
             uint32_t nbi[G];   // window of the neighbour row, one entry per lane
-            double nbp[G][3];  // and the neighbours' positions
+            double nbp[G][DIM];  // and the neighbours' positions
         };
         struct {  // extraction
             uint32_t first[MAXP];  // vertex of each plane with the lowest plane key
@@ -102,7 +119,7 @@ struct SeedSmem {
 };
 
 template <int DIM, int G, int S>
-using VoroSmem = SeedSmem<VoroCfg<DIM, G, S>::NS, VoroCfg<DIM, G, S>::MAXP, G>;
+using VoroSmem = SeedSmem<DIM, VoroCfg<DIM, G, S>::NS, VoroCfg<DIM, G, S>::MAXP, G>;
 
 // Round a non-negative double up to float (next float above on inexact).
 PG_DEV float f2f_up(double d) {
@@ -1167,7 +1184,7 @@ __device__ __forceinline__ void voronoi_group(const double* __restrict__ pts, in
                 const double R2 = exact_R2();
                 if (ahead) {
                     const double dx = sm.nbp[gl][0] - sx, dy = sm.nbp[gl][1] - sy;
-                    const double dz = D == 3 ? sm.nbp[gl][2] - sz : 0.0;
+                    const double dz = D == 3 ? sm.nbp[gl][D - 1] - sz : 0.0;
                     cert = dx * dx + dy * dy + dz * dz > 4 * R2;
                 }
             }
@@ -1221,7 +1238,7 @@ __device__ __forceinline__ void voronoi_group(const double* __restrict__ pts, in
             z = sm.nbi[j];
             bx = sm.nbp[j][0];
             by = sm.nbp[j][1];
-            bz = D == 3 ? sm.nbp[j][2] : 0.0;
+            bz = D == 3 ? sm.nbp[j][D - 1] : 0.0;
         }
         const bool anyclip = clip_step(act, z, bx, by, bz);
         since++;
@@ -1561,7 +1578,7 @@ __device__ __forceinline__ void voronoi_group(const double* __restrict__ pts, in
     block_sync();
 #pragma unroll
     for (int i = 0; i < C::PPL; i++)
-        if (fp[i] >= 0) sm.plane[fp[i]] = {pvol[i], pcx[i], pcy[i], pcz[i]};
+        if (fp[i] >= 0) sm.plane[fp[i]] = Plane{pvol[i], pcx[i], pcz[i], pcy[i]};
     block_sync();
     const auto add = [](double theirs, double mine) { return mine + theirs; };
 #pragma unroll
@@ -1570,8 +1587,8 @@ __device__ __forceinline__ void voronoi_group(const double* __restrict__ pts, in
         if (has[i]) m = sm.plane[gl + G * i];
         pvol[i] = group_butterfly_d<G>(m.x, add);
         pcx[i] = group_butterfly_d<G>(m.y, add);
-        pcy[i] = group_butterfly_d<G>(m.z, add);
-        pcz[i] = group_butterfly_d<G>(m.w, add);
+        pcy[i] = group_butterfly_d<G>(m.w, add);
+        pcz[i] = group_butterfly_d<G>(m.z, add);
     }
 #pragma unroll
     for (int w = 1; w < C::PPL; w <<= 1)

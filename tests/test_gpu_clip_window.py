@@ -45,3 +45,19 @@ def test_nearly_degenerate_lattices(ctx, dim, amp):
 def test_clusters_far_below_the_box(ctx, scale):
     pts = np.concatenate([scale * (uniform_points(4000, 3, 5) - 0.5) + 0.5, uniform_points(12000, 3, 6)])
     _same(ctx, pts, boundary="reflective", k=32, restart=True, k_max=128)
+
+
+@pytest.mark.parametrize("faces", [12, 15, 16, 17, 20, 21, 30, 60])
+def test_2d_cells_of_many_faces(ctx, faces):
+    """Rings of points around a seed: cells around the 16 vertex slots and 24
+    planes (20 besides the box) of the fast 2D kernel, and beyond them (60 and
+    the box's 4 fill max_p: the next row entry overflows the cell)."""
+    a = 2 * np.pi * (np.arange(faces) + 0.25) / faces
+    rings = [np.concatenate([[[cx, cy]], np.stack([cx + 0.04 * np.cos(a), cy + 0.04 * np.sin(a)], 1)])
+             for cx, cy in ((0.31, 0.42), (0.68, 0.27), (0.5, 0.8))]
+    base = uniform_points(3000, 2, 91)
+    keep = np.all([np.hypot(*(base - r[0]).T) > 0.09 for r in rings], axis=0)
+    pts = np.concatenate([base[keep]] + rings)
+    for k in (16, 32):
+        out = _same(ctx, pts, boundary="reflective", k=k, restart=True)
+        assert faces == 60 or out["face_counts"].max() >= faces
