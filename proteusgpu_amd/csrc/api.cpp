@@ -206,7 +206,8 @@ struct pg_mesh {
     DBuf ovals;  // seeds in clip order
     uint32_t* out_order() { return sorted_space ? iperm.as<uint32_t>() : g.perm.as<uint32_t>(); }
     // hydro tables
-    DBuf hid, area_u, vol_u, o2s, bad;
+    DBuf vol_u, o2s, bad;
+    DBuf srec;  // static-mesh update: states by sorted seed
     // owner-computes-once update: hydro code per sorted seed, twin code per
     // face slot, and scratch for the sorted cell records and the per-slot
     // face fluxes
@@ -251,7 +252,7 @@ struct pg_kmodel {
 struct pg_state {
     int dim = 3;
     int64_t n = 0;
-    DBuf rho[2], vel[2], E[2];
+    DBuf rho[2], vel[2], E[2], dt;
     int cur = 0;
 };
 
@@ -688,15 +689,12 @@ void mesh_finalize(pg_ctx* c, pg_mesh* m) {
     hipStream_t s = c->stream;
     const size_t ns = (size_t)m->n_seeds;
     const double sc = m->scale();
-    const double as = m->prm.dim == 2 ? sc : sc * sc;
     const double vs = m->prm.dim == 2 ? sc * sc : sc * sc * sc;
     int32_t* bad = m->bad.get<int32_t>(2);
     HIPCHK(hipMemsetAsync(bad, 0, 2 * sizeof(int32_t), s));
     const int64_t* gsrc = m->prm.boundary == PG_BOUNDARY_PERIODIC ? m->gsrc.as<int64_t>() : nullptr;
-    pg::launch_finalize(m->n_seeds, m->n_hydro, m->n_seeds, m->out_order(), gsrc,
-                        m->count.as<uint8_t>(), m->nbr.as<int32_t>(), m->area.as<double>(),
-                        m->vol.as<double>(), as, vs, m->hid.get<int32_t>(ns * MAXP),
-                        m->area_u.get<double>(ns * MAXP), m->vol_u.get<double>(ns),
+    pg::launch_finalize(m->n_seeds, m->n_hydro, m->n_seeds, m->out_order(), gsrc, m->count.as<uint8_t>(),
+                        m->nbr.as<int32_t>(), m->vol.as<double>(), vs, m->vol_u.get<double>(ns),
                         m->o2s.get<int32_t>(std::max<int64_t>(m->n_hydro, 1)), m->hcode.get<int32_t>(ns), bad, s);
     HIPCHK(hipGetLastError());
     // faces over all cells (VMesh.num_faces), read with the error counters:
@@ -1218,8 +1216,7 @@ int pg_dt_cfl(pg_ctx* c, const pg_mesh* mc, const pg_state* st, double gamma, do
         pg_mesh* m = const_cast<pg_mesh*>(mc);
         argchk(st->n == m->n_hydro && st->dim == m->prm.dim, "state does not match mesh");
         mesh_finalize(c, m);
-        DBuf out;
-        unsigned long long* d = out.get<unsigned long long>(1);
+        unsigned long long* d = const_cast<pg_state*>(st)->dt.get<unsigned long long>(1);
         double init = 1e100;  // finite_volume_solver.cpp:153
         HIPCHK(hipMemcpyAsync(d, &init, sizeof(double), hipMemcpyHostToDevice, c->stream));
         const int b = st->cur;
@@ -1241,12 +1238,13 @@ int pg_hydro_step(pg_ctx* c, const pg_mesh* mc, pg_state* st, double gamma, doub
         argchk(st->n == m->n_hydro && st->dim == m->prm.dim, "state does not match mesh");
         mesh_finalize(c, m);
         const int b = st->cur, nb = 1 - b;
-        pg::launch_hll_static(st->dim, m->n_seeds, m->n_hydro, m->n_seeds, m->n_seeds * MAXP,
-                              m->out_order(), m->count.as<uint8_t>(), m->hid.as<int32_t>(),
-                              m->nrm.as<double>(), m->area_u.as<double>(), m->vol_u.as<double>(), gamma, dt,
-                              flux_mode, st->rho[b].as<double>(), st->vel[b].as<double>(),
-                              st->E[b].as<double>(), st->rho[nb].as<double>(), st->vel[nb].as<double>(),
-                              st->E[nb].as<double>(), c->stream);
+        const double sc = m->scale();
+        pg::launch_hll_static(st->dim, m->n_seeds, m->n_seeds, m->n_seeds * MAXP, m->hcode.as<int32_t>(),
+                              m->count.as<uint8_t>(), m->nbr.as<int32_t>(), m->nrm.as<double>(), m->area.as<double>(),
+                              st->dim == 2 ? sc : sc * sc, m->vol_u.as<double>(), gamma, dt, flux_mode,
+                              st->rho[b].as<double>(), st->vel[b].as<double>(), st->E[b].as<double>(),
+                              m->srec.get<double>((size_t)m->n_seeds * pg::static_rec_doubles(st->dim)),
+                              st->rho[nb].as<double>(), st->vel[nb].as<double>(), st->E[nb].as<double>(), c->stream);
         HIPCHK(hipGetLastError());
         st->cur = nb;
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -1414,7 +1412,8 @@ void sim_hydro(pg_ctx* c, pg_sim* S, double dt_max, bool moving) {
     u.solve = m.solve.as<uint64_t>();
     u.nbr = m.nbr.as<int32_t>();
     u.nrm = m.nrm.as<double>();
-    u.area_u = m.area_u.as<double>();
+    u.area = m.area.as<double>();
+    u.ascale = dim == 2 ? sc : sc * sc;
     u.cen = m.cen.as<double>();
     u.sorted = m.g.sorted.as<double>();
     u.scale = sc;
@@ -1860,7 +1859,7 @@ struct pg_batch {
     DBuf nbr, area, nrm, cen, count, vol, ccen, status, kcert;
     DBuf cstate, resume, lastnb;  // saved cells of uncertified seeds (restarts resume them)
     DBuf ticket;          // work-queue counter of the persistent kernels
-    DBuf hid, area_u, vol_u, o2s, hsorted, tot;
+    DBuf vol_u, o2s, tot;
     DBuf hcode, nbr_cm, twin, solve, frec, fbuf;  // owner-computes-once update
     hipGraphExec_t exec = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -2012,11 +2011,10 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
     }
     if (!big_done) big_pass(kb);
     const double sc = B->scale();
-    const double as = dim == 2 ? sc : sc * sc, vs = dim == 2 ? sc * sc : sc * sc * sc;
+    const double vs = dim == 2 ? sc * sc : sc * sc * sc;
     pg::launch_bfinalize(n_dev, cap, cap, B->perm.as<uint32_t>(), B->orig_h.as<int32_t>(), B->count.as<uint8_t>(),
-                         B->nbr.as<int32_t>(), B->area.as<double>(), B->vol.as<double>(), as, vs, B->periodic ? 1 : 0,
-                         B->hid.as<int32_t>(), B->area_u.as<double>(), B->vol_u.as<double>(), B->o2s.as<int32_t>(),
-                         B->hsorted.as<int32_t>(), B->hcode.as<int32_t>(), B->st() + 1, s);
+                         B->nbr.as<int32_t>(), B->vol.as<double>(), vs, B->periodic ? 1 : 0, B->vol_u.as<double>(),
+                         B->o2s.as<int32_t>(), B->hcode.as<int32_t>(), B->st() + 1, s);
     pg::launch_face_twins(n_dev, cap, cap, B->hcode.as<int32_t>(), B->count.as<uint8_t>(), B->nbr_cm.as<int32_t>(),
                           B->twin.as<uint8_t>(), B->solve.as<uint64_t>(), s);
     pg::launch_bcount_failed(n_dev, cap, B->status.as<int32_t>(), B->st() + 3, s);
@@ -2055,7 +2053,8 @@ void batch_hydro(pg_batch* B, hipStream_t s) {
     u.solve = B->solve.as<uint64_t>();
     u.nbr = B->nbr.as<int32_t>();
     u.nrm = B->nrm.as<double>();
-    u.area_u = B->area_u.as<double>();
+    u.area = B->area.as<double>();
+    u.ascale = dim == 2 ? B->scale() : B->scale() * B->scale();
     u.cen = B->cen.as<double>();
     u.sorted = B->sorted.as<double>();
     u.scale = B->scale();
@@ -2269,11 +2268,8 @@ int pg_batch_create(pg_ctx* c, const pg_sim_params* prm, int nbox, const int64_t
                 B->lastnb.get<uint32_t>(cs);
                 B->resume.get<int32_t>(cs);
             }
-            B->hid.get<int32_t>(cs * MAXP);
-            B->area_u.get<double>(cs * MAXP);
             B->vol_u.get<double>(cs);
             B->o2s.get<int32_t>(n);
-            B->hsorted.get<int32_t>(cs);
             B->hcode.get<int32_t>(cs);
             B->nbr_cm.get<int32_t>(cs * MAXP);
             B->twin.get<uint8_t>(cs * MAXP);

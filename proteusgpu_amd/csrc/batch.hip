@@ -351,32 +351,20 @@ __global__ void __launch_bounds__(TB)
 __global__ void __launch_bounds__(TB)
     k_bfinalize(const int64_t* __restrict__ n_dev, int64_t stride, const uint32_t* __restrict__ perm,
                 const int32_t* __restrict__ orig_h, const uint8_t* __restrict__ count, const int32_t* __restrict__ nbr,
-                const double* __restrict__ area, const double* __restrict__ vol, double ascale, double vscale,
-                int periodic, int32_t* __restrict__ hid, double* __restrict__ area_u, double* __restrict__ vol_u,
-                int32_t* __restrict__ o2s, int32_t* __restrict__ hsorted, int32_t* __restrict__ hcode, int32_t* bad) {
+                const double* __restrict__ vol, double vscale, int periodic, double* __restrict__ vol_u,
+                int32_t* __restrict__ o2s, int32_t* __restrict__ hcode, int32_t* bad) {
     const int64_t n = *n_dev;
     for (int64_t s = (int64_t)blockIdx.x * TB + threadIdx.x; s < n; s += (int64_t)gridDim.x * TB) {
         const int32_t h = orig_h[perm[s]];
-        hsorted[s] = h;
         hcode[s] = h;  // ghosts: -1 - source, as orig_h
         if (h < 0) continue;
         o2s[h] = (int32_t)s;
         vol_u[s] = vscale * vol[s];
         const int c = count[s];
         if (c == 0) atomicAdd(bad, 1);
-        for (int f = 0; f < c; f++) {
-            const int64_t at = (int64_t)f * stride + s;
-            const int32_t j = nbr[at];
-            int32_t hj = -1;
-            if (j >= 0) {
-                const int32_t oj = orig_h[perm[j]];
-                hj = oj >= 0 ? oj : -1 - oj;
-            } else if (periodic) {
-                atomicAdd(bad + 1, 1);
-            }
-            hid[at] = hj;
-            area_u[at] = ascale * area[at];
-        }
+        if (periodic)
+            for (int f = 0; f < c; f++)
+                if (nbr[(int64_t)f * stride + s] < 0) atomicAdd(bad + 1, 1);
     }
 }
 
@@ -630,12 +618,10 @@ void launch_bcollect(const int64_t* nq_dev, int64_t cap, const uint32_t* seeds, 
 }
 
 void launch_bfinalize(const int64_t* n_dev, int64_t cap, int64_t stride, const uint32_t* perm, const int32_t* orig_h,
-                      const uint8_t* count, const int32_t* nbr, const double* area, const double* vol, double ascale,
-                      double vscale, int periodic, int32_t* hid, double* area_u, double* vol_u, int32_t* o2s,
-                      int32_t* hsorted, int32_t* hcode, int32_t* bad, hipStream_t s) {
-    k_bfinalize<<<std::min<unsigned>(nblk(cap), 2048), TB, 0, s>>>(n_dev, stride, perm, orig_h, count, nbr, area, vol,
-                                                                   ascale, vscale, periodic, hid, area_u, vol_u, o2s,
-                                                                   hsorted, hcode, bad);
+                      const uint8_t* count, const int32_t* nbr, const double* vol, double vscale, int periodic,
+                      double* vol_u, int32_t* o2s, int32_t* hcode, int32_t* bad, hipStream_t s) {
+    k_bfinalize<<<std::min<unsigned>(nblk(cap), 2048), TB, 0, s>>>(n_dev, stride, perm, orig_h, count, nbr, vol, vscale,
+                                                                   periodic, vol_u, o2s, hcode, bad);
 }
 
 void launch_bdt(int dim, int64_t n_h, int nbox, const int32_t* hbox, const int32_t* o2s, const double* vol_u,

@@ -51,7 +51,8 @@ struct OwnedUpdate {
     const uint8_t* twin = nullptr;  // launch_face_twins of the same mesh
     const uint64_t* solve = nullptr;
     const int32_t* nbr = nullptr;
-    const double *nrm = nullptr, *area_u = nullptr, *cen = nullptr, *sorted = nullptr;
+    const double *nrm = nullptr, *area = nullptr, *cen = nullptr, *sorted = nullptr;
+    double ascale = 1.0;  // of the stored areas
     double scale = 1.0, gam = 1.4;
     int flux_mode = 1, move = 1;
     // time step: *dt_dev capped at dt_max > 0, or per box dt_box[hbox[i]]
@@ -79,16 +80,15 @@ int64_t totals_blocks(int64_t n);
 void launch_totals(int dim, SimView sv, double* part, hipStream_t s);
 
 void launch_finalize(int64_t n, int64_t n_hydro, int64_t stride, const uint32_t* perm,
-                     const int64_t* gsrc, const uint8_t* count, const int32_t* nbr,
-                     const double* area, const double* vol, double ascale, double vscale,
-                     int32_t* hid, double* area_u, double* vol_u, int32_t* o2s, int32_t* hcode, int32_t* bad,
-                     hipStream_t s);
+                     const int64_t* gsrc, const uint8_t* count, const int32_t* nbr, const double* vol, double vscale,
+                     double* vol_u, int32_t* o2s, int32_t* hcode, int32_t* bad, hipStream_t s);
 
-void launch_hll_static(int dim, int64_t n, int64_t n_hydro, int64_t stride, int64_t nplane,
-                       const uint32_t* perm, const uint8_t* count, const int32_t* hid,
-                       const double* nrm, const double* area_u, const double* vol_u, double gam,
-                       double dt, int flux_mode, const double* rho, const double* vel,
-                       const double* E, double* rho2, double* vel2, double* E2, hipStream_t s);
+// rec: scratch, static_rec_doubles(dim) per seed.
+int64_t static_rec_doubles(int dim);
+void launch_hll_static(int dim, int64_t n, int64_t stride, int64_t nplane, const int32_t* hcode, const uint8_t* count,
+                       const int32_t* nbr, const double* nrm, const double* area, double ascale, const double* vol_u,
+                       double gam, double dt, int flux_mode, const double* rho, const double* vel, const double* E,
+                       double* rec, double* rho2, double* vel2, double* E2, hipStream_t s);
 
 void launch_dt_cfl(int dim, int64_t n_hydro, const int32_t* o2s, const double* vol_u, double gam,
                    double cfl, const double* rho, const double* vel, const double* E,
@@ -111,9 +111,8 @@ void launch_cells_orig(int64_t n, int64_t stride, int dim, const uint32_t* perm,
 
 // batched boxes (batch.hip)
 void launch_bfinalize(const int64_t* n_dev, int64_t cap, int64_t stride, const uint32_t* perm, const int32_t* orig_h,
-                      const uint8_t* count, const int32_t* nbr, const double* area, const double* vol, double ascale,
-                      double vscale, int periodic, int32_t* hid, double* area_u, double* vol_u, int32_t* o2s,
-                      int32_t* hsorted, int32_t* hcode, int32_t* bad, hipStream_t s);
+                      const uint8_t* count, const int32_t* nbr, const double* vol, double vscale, int periodic,
+                      double* vol_u, int32_t* o2s, int32_t* hcode, int32_t* bad, hipStream_t s);
 void launch_bdt(int dim, int64_t n_h, int nbox, const int32_t* hbox, const int32_t* o2s, const double* vol_u,
                 double gam, double cfl, const double* rho, const double* vel, const double* E, double* dt_box,
                 hipStream_t s, const double* wgen = nullptr, CflMesh cm = {});

@@ -20,14 +20,15 @@ constexpr int TB = 256;
 inline unsigned nblk(int64_t n) { return (unsigned)((n + TB - 1) / TB); }
 inline unsigned nblk_dt(int64_t n) { return (unsigned)((n + (int64_t)TB * DT_CELLS - 1) / ((int64_t)TB * DT_CELLS)); }
 
-// Per sorted cell: hydro id of every face's neighbour (-1 = box plane,
-// which is a reflective wall), unscaled area and cell volume.
+// Per sorted cell: its hydro code and unscaled volume, and the error counters
+// (bad[0] hydro cells without faces, bad[1] faces of periodic hydro cells on
+// the box plane, which means that the ghost layer is thinner than the cell;
+// finite_volume_solver.cpp:130-136 would read out of bounds there).
 __global__ void __launch_bounds__(TB) k_finalize(int64_t n, int64_t n_hydro, int64_t stride,
                                                  const uint32_t* perm, const int64_t* gsrc,
-                                                 const uint8_t* count, const int32_t* nbr,
-                                                 const double* area, const double* vol, double ascale,
-                                                 double vscale, int32_t* hid, double* area_u,
-                                                 double* vol_u, int32_t* o2s, int32_t* hcode, int32_t* bad) {
+                                                 const uint8_t* count, const int32_t* nbr, const double* vol,
+                                                 double vscale, double* vol_u, int32_t* o2s, int32_t* hcode,
+                                                 int32_t* bad) {
     int64_t s = (int64_t)blockIdx.x * TB + threadIdx.x;
     if (s >= n) return;
     const uint32_t o = perm[s];
@@ -38,64 +39,79 @@ __global__ void __launch_bounds__(TB) k_finalize(int64_t n, int64_t n_hydro, int
     vol_u[s] = vscale * vol[s];
     const int c = count[s];
     if (c == 0) atomicAdd(bad, 1);
-    for (int f = 0; f < c; f++) {
-        const int64_t at = (int64_t)f * stride + s;
-        const int32_t j = nbr[at];
-        int32_t h = -1;
-        if (j >= 0) {
-            const uint32_t oj = perm[j];
-            h = oj < n_hydro ? (int32_t)oj : (int32_t)gsrc[oj - n_hydro];
-        } else if (gsrc) {
-            // periodic mesh: a hydro cell reaching the box plane means the
-            // ghost layer is thinner than the cell (finite_volume_solver.cpp:130-136
-            // would read out of bounds here)
-            atomicAdd(bad + 1, 1);
-        }
-        hid[at] = h;
-        area_u[at] = ascale * area[at];
-    }
+    if (gsrc)
+        for (int f = 0; f < c; f++)
+            if (nbr[(int64_t)f * stride + s] < 0) atomicAdd(bad + 1, 1);
+}
+
+// State of a static-mesh update by sorted seed: rho, v[DIM], E in rows of
+// whole 16-byte words (ghosts take their source cell's).
+template <int DIM>
+constexpr int STATIC_REC = DIM == 3 ? 6 : 4;
+template <int DIM>
+__global__ void __launch_bounds__(TB)
+    k_static_records(int64_t n, const int32_t* __restrict__ hcode, const double* __restrict__ rho,
+                     const double* __restrict__ vel, const double* __restrict__ E, double* __restrict__ rec) {
+    const int64_t s = (int64_t)blockIdx.x * TB + threadIdx.x;
+    if (s >= n) return;
+    const int32_t c = hcode[s];
+    const int64_t h = c >= 0 ? c : -1 - (int64_t)c;
+    double* r = rec + s * STATIC_REC<DIM>;
+    r[0] = rho[h];
+#pragma unroll
+    for (int d = 0; d < DIM; d++) r[1 + d] = vel[(size_t)DIM * h + d];
+    r[1 + DIM] = E[h];
 }
 
 // One static-mesh HLL update per hydro cell (finite_volume_solver.cpp:53-106):
 // every cell sums the fluxes through its own faces, exactly as the
 // reference, and writes the new primitives to the second buffer.
+//
+// What bounds it: the neighbours' states.  Read from the state arrays in input
+// order they were five scattered lines per face (1M cells: 830 us a step);
+// from records in sorted order, with the blocks of an XCD on consecutive
+// cells, they come from its L2: 450 us and 67 for the records.
 template <int DIM>
 __global__ void __launch_bounds__(TB)
-    k_hll_static(int64_t n, int64_t n_hydro, int64_t stride, int64_t nplane,
-                 const uint32_t* __restrict__ perm, const uint8_t* __restrict__ count,
-                 const int32_t* __restrict__ hid, const double* __restrict__ nrm,
-                 const double* __restrict__ area_u, const double* __restrict__ vol_u, double gam,
-                 double dt, int flux_mode, const double* __restrict__ rho,
-                 const double* __restrict__ vel, const double* __restrict__ E,
-                 double* __restrict__ rho2, double* __restrict__ vel2, double* __restrict__ E2) {
-    int64_t s = (int64_t)blockIdx.x * TB + threadIdx.x;
+    k_hll_static(int64_t n, int64_t stride, int64_t nplane, const int32_t* __restrict__ hcode,
+                 const uint8_t* __restrict__ count, const int32_t* __restrict__ nbr, const double* __restrict__ nrm,
+                 const double* __restrict__ area, double ascale, const double* __restrict__ vol_u, double gam,
+                 double dt, int flux_mode, const double* __restrict__ rec, double* __restrict__ rho2,
+                 double* __restrict__ vel2, double* __restrict__ E2) {
+    const int64_t s = xcd_block(blockIdx.x, gridDim.x) * TB + threadIdx.x;
     if (s >= n) return;
-    const uint32_t i = perm[s];
-    if (i >= n_hydro) return;
-    Prim si;
-    si.rho = rho[i];
-    si.E = E[i];
-    si.v[2] = 0.0;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) si.v[d] = vel[(size_t)DIM * i + d];
+    const int32_t i = hcode[s];
+    if (i < 0) return;
+    auto state_of = [&](int64_t t) {
+        const double2* r = reinterpret_cast<const double2*>(rec + t * STATIC_REC<DIM>);
+        const double2 a = r[0], b = r[1];
+        Prim p;
+        p.rho = a.x;
+        p.v[0] = a.y;
+        p.v[1] = b.x;
+        p.v[2] = 0.0;
+        if (DIM == 3) {
+            p.v[2] = b.y;
+            p.E = r[DIM - 1].x;
+        } else {
+            p.E = b.y;
+        }
+        return p;
+    };
+    const Prim si = state_of(s);
     Prim tot = {0.0, {0.0, 0.0, 0.0}, 0.0};
     const int c = count[s];
     const double sgn = flux_mode == 1 ? -1.0 : 1.0;
+    int32_t j = c > 0 ? nbr[s] : -1;
     for (int f = 0; f < c; f++) {
         const int64_t at = (int64_t)f * stride + s;
-        const int32_t j = hid[at];
         const bool wall = j < 0;
-        Prim sj = si;
-        if (!wall) {
-            sj.rho = rho[j];
-            sj.E = E[j];
-#pragma unroll
-            for (int d = 0; d < DIM; d++) sj.v[d] = vel[(size_t)DIM * j + d];
-        }
+        const Prim sj = wall ? si : state_of(j);
+        if (f + 1 < c) j = nbr[at + stride];
         // flux_mode 1 negates the stored (inward) normal exactly
         const Geom g = geom_of(sgn * nrm[at], sgn * nrm[nplane + at], sgn * nrm[2 * nplane + at]);
         const Prim F = hll<DIM>(gam, si, sj, g, wall);
-        const double a = area_u[at];
+        const double a = ascale * area[at];
         tot.rho += F.rho * a;
 #pragma unroll
         for (int d = 0; d < DIM; d++) tot.v[d] += F.v[d] * a;
@@ -298,7 +314,7 @@ template <int DIM>
 __global__ void __launch_bounds__(TB)
     k_face_flux(const int64_t* n_dev, int64_t n_host, int64_t stride, int64_t nplane, const int32_t* __restrict__ hcode,
                 const uint64_t* __restrict__ solve, const int32_t* __restrict__ nbr,
-                const double* __restrict__ nrm, const double* __restrict__ area_u, const double* __restrict__ cen,
+                const double* __restrict__ nrm, const double* __restrict__ area, double ascale, const double* __restrict__ cen,
                 const double* __restrict__ sorted, double scale, double gam, int flux_mode, int move,
                 const CellRec* __restrict__ rec, double* __restrict__ fbuf) {
     const int64_t n = seed_count(n_dev, n_host);
@@ -348,7 +364,7 @@ __global__ void __launch_bounds__(TB)
             double Fm, Fp[3], Fe;
             ale_face<DIM>(gam, sgn, move, si, ri, gi, sj, rj, gj, wall, nrm[at], nrm[nplane + at],
                           nrm[2 * nplane + at], fc, Fm, Fp, Fe);
-            const double a = area_u[at];
+            const double a = ascale * area[at];
             double* fo = fbuf + at * (DIM + 2);
             fo[0] = Fm * a;
 #pragma unroll
@@ -570,30 +586,29 @@ __global__ void __launch_bounds__(TB)
 
 }  // namespace
 
-void launch_finalize(int64_t n, int64_t n_hydro, int64_t stride, const uint32_t* perm,
-                     const int64_t* gsrc, const uint8_t* count, const int32_t* nbr,
-                     const double* area, const double* vol, double ascale, double vscale,
-                     int32_t* hid, double* area_u, double* vol_u, int32_t* o2s, int32_t* hcode, int32_t* bad,
-                     hipStream_t s) {
+void launch_finalize(int64_t n, int64_t n_hydro, int64_t stride, const uint32_t* perm, const int64_t* gsrc,
+                     const uint8_t* count, const int32_t* nbr, const double* vol, double vscale, double* vol_u,
+                     int32_t* o2s, int32_t* hcode, int32_t* bad, hipStream_t s) {
     if (n <= 0) return;
-    k_finalize<<<nblk(n), TB, 0, s>>>(n, n_hydro, stride, perm, gsrc, count, nbr, area, vol, ascale,
-                                      vscale, hid, area_u, vol_u, o2s, hcode, bad);
+    k_finalize<<<nblk(n), TB, 0, s>>>(n, n_hydro, stride, perm, gsrc, count, nbr, vol, vscale, vol_u, o2s, hcode, bad);
 }
 
-void launch_hll_static(int dim, int64_t n, int64_t n_hydro, int64_t stride, int64_t nplane,
-                       const uint32_t* perm, const uint8_t* count, const int32_t* hid,
-                       const double* nrm, const double* area_u, const double* vol_u, double gam,
-                       double dt, int flux_mode, const double* rho, const double* vel,
-                       const double* E, double* rho2, double* vel2, double* E2, hipStream_t s) {
+int64_t static_rec_doubles(int dim) { return dim == 3 ? STATIC_REC<3> : STATIC_REC<2>; }
+
+void launch_hll_static(int dim, int64_t n, int64_t stride, int64_t nplane, const int32_t* hcode, const uint8_t* count,
+                       const int32_t* nbr, const double* nrm, const double* area, double ascale, const double* vol_u,
+                       double gam, double dt, int flux_mode, const double* rho, const double* vel, const double* E,
+                       double* rec, double* rho2, double* vel2, double* E2, hipStream_t s) {
     if (n <= 0) return;
-    if (dim == 2)
-        k_hll_static<2><<<nblk(n), TB, 0, s>>>(n, n_hydro, stride, nplane, perm, count, hid, nrm,
-                                               area_u, vol_u, gam, dt, flux_mode, rho, vel, E, rho2,
-                                               vel2, E2);
-    else
-        k_hll_static<3><<<nblk(n), TB, 0, s>>>(n, n_hydro, stride, nplane, perm, count, hid, nrm,
-                                               area_u, vol_u, gam, dt, flux_mode, rho, vel, E, rho2,
-                                               vel2, E2);
+    if (dim == 2) {
+        k_static_records<2><<<nblk(n), TB, 0, s>>>(n, hcode, rho, vel, E, rec);
+        k_hll_static<2><<<nblk(n), TB, 0, s>>>(n, stride, nplane, hcode, count, nbr, nrm, area, ascale, vol_u, gam, dt,
+                                               flux_mode, rec, rho2, vel2, E2);
+    } else {
+        k_static_records<3><<<nblk(n), TB, 0, s>>>(n, hcode, rho, vel, E, rec);
+        k_hll_static<3><<<nblk(n), TB, 0, s>>>(n, stride, nplane, hcode, count, nbr, nrm, area, ascale, vol_u, gam, dt,
+                                               flux_mode, rec, rho2, vel2, E2);
+    }
 }
 
 void launch_dt_cfl(int dim, int64_t n_hydro, const int32_t* o2s, const double* vol_u, double gam,
@@ -645,14 +660,14 @@ void launch_hll_owned(int dim, OwnedUpdate u, hipStream_t s) {
     if (dim == 2) {
         k_cell_records<2><<<gb, TB, 0, s>>>(u.n_dev, u.n, u.hcode, u.sv, u.wgen, u.rec);
         k_face_flux<2><<<gf, TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.solve, u.nbr, u.nrm,
-                                         u.area_u, u.cen, u.sorted, u.scale, u.gam, u.flux_mode, u.move, u.rec,
+                                         u.area, u.ascale, u.cen, u.sorted, u.scale, u.gam, u.flux_mode, u.move, u.rec,
                                          u.fbuf);
         k_face_sum<2><<<gb, TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.count, u.twin, u.nbr, u.fbuf,
                                         u.dt_dev, u.dt_max, u.dt_box, u.hbox, u.sv);
     } else {
         k_cell_records<3><<<gb, TB, 0, s>>>(u.n_dev, u.n, u.hcode, u.sv, u.wgen, u.rec);
         k_face_flux<3><<<gf, TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.solve, u.nbr, u.nrm,
-                                         u.area_u, u.cen, u.sorted, u.scale, u.gam, u.flux_mode, u.move, u.rec,
+                                         u.area, u.ascale, u.cen, u.sorted, u.scale, u.gam, u.flux_mode, u.move, u.rec,
                                          u.fbuf);
         k_face_sum<3><<<gb, TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.count, u.twin, u.nbr, u.fbuf,
                                         u.dt_dev, u.dt_max, u.dt_box, u.hbox, u.sv);
