@@ -130,7 +130,9 @@ PG_DEV double cfl_length(double V, int32_t s, const CflMesh& cm) {
     if (cm.count == nullptr) return R;
     const int c = cm.count[s];
     double dmin = 1e300;
-    for (int f = 0; f < c; f++) {
+    // faces lie in row order, by distance: the first generator's is nearest
+    // (2M cells: 106 us; with all their faces looked at 850 us)
+    for (int f = 0; f < c && dmin == 1e300; f++) {
         const int32_t js = cm.nbr[(int64_t)f * cm.stride + s];
         if (js < 0) continue;
         double dd = 0.0;
