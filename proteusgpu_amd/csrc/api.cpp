@@ -123,21 +123,20 @@ struct Grid {
         int32_t* st = starts.get<int32_t>(ncell);
         int32_t* fl = fill.get<int32_t>(ncell);
         int32_t* tp = tmp.get<int32_t>(pg::scan_tmp_elems(std::max(ncell, n)));
-        HIPCHK(hipMemsetAsync(cnt, 0, sizeof(int32_t) * ncell, s));
-        HIPCHK(hipMemsetAsync(fl, 0, sizeof(int32_t) * ncell, s));
+        int32_t* bg = big.get<int32_t>(ncell + 1);
+        pg::launch_grid_clear(ncell, cnt, fl, bg, s, sub_m.get<int32_t>(ncell), sub_alloc.get<int32_t>(1));
         pg::launch_cell_count(dim, pts.as<double>(), n, N, cell.get<int32_t>(n), cnt, s);
         pg::scan_exclusive_i32(cnt, st, ncell, tp, total.get<int32_t>(1), s);
         uint32_t* pm = perm.get<uint32_t>(n);
         pg::launch_cell_scatter(n, cell.as<int32_t>(), st, fl, pm, s);
-        int32_t* bg = big.get<int32_t>(ncell + 1);
         pg::launch_cell_sort(ncell, st, cnt, pm, bg + 1, bg, s);
         pg::launch_gather_points(dim, n, pm, pts.as<double>(), sorted.get<double>((size_t)n * dim), s);
         // a sub-cell table holds at most n / 3 + 64 entries (about 3 points
         // per sub-cell, at least 8 (2D: 9) sub-cells per cell of over 32)
         const int64_t cap = n / 2 + 1024;
-        pg::launch_subgrid(dim, sorted.as<double>(), n, N, ncell, st, cnt, bg + 1, bg, sub_m.get<int32_t>(ncell),
+        pg::launch_subgrid(dim, sorted.as<double>(), n, N, ncell, st, cnt, bg + 1, bg, sub_m.as<int32_t>(),
                            sub_ptr.get<int32_t>(ncell), sub_start.get<int32_t>(cap), sub_cnt.get<int32_t>(cap), cap,
-                           sub_idx.get<uint32_t>(n), sub_alloc.get<int32_t>(1), s);
+                           sub_idx.get<uint32_t>(n), sub_alloc.as<int32_t>(), s);
         has_sub = true;
         crowded = -1;
         HIPCHK(hipGetLastError());
@@ -206,7 +205,22 @@ struct pg_mesh {
     DBuf ovals;  // seeds in clip order
     uint32_t* out_order() { return sorted_space ? iperm.as<uint32_t>() : g.perm.as<uint32_t>(); }
     // hydro tables
-    DBuf vol_u, o2s, bad;
+    DBuf vol_u, o2s;
+    // tallies of a build's collects, zeroed together at its start
+    static constexpr int TALLIES = 32;
+    DBuf tallies;
+    int tally_next = 0;
+    void new_tallies(hipStream_t s) {
+        pg::launch_fill_u64(tallies.get<unsigned long long>(3 * TALLIES), 3 * TALLIES, 0ull, s);
+        tally_next = 0;
+    }
+    // error counters of finalisation (2) and the face total
+    DBuf bad;
+    int32_t* new_bad(hipStream_t s) {
+        int32_t* b = bad.get<int32_t>(3);
+        pg::launch_fill_i32(b, 3, 0, s);
+        return b;
+    }
     DBuf srec;  // static-mesh update: states by sorted seed
     // owner-computes-once update: hydro code per sorted seed, twin code per
     // face slot, and scratch for the sorted cell records and the per-slot
@@ -265,16 +279,32 @@ int32_t read_i32(const int32_t* d, hipStream_t s) {
     return h;
 }
 
-// Seeds of `seeds` (nullptr: all) whose status equals code, into out.
-int64_t collect_list(pg_mesh* m, const uint32_t* seeds, int64_t nq, int code, uint32_t* out,
-                     hipStream_t s) {
-    int32_t* fl = m->flags.get<int32_t>(m->n_seeds);
-    int32_t* of = m->offs.get<int32_t>(m->n_seeds);
-    int32_t* tp = m->g.tmp.get<int32_t>(pg::scan_tmp_elems(std::max(m->n_seeds, m->g.ncell)));
-    int32_t* c = m->cnt1.get<int32_t>(1);
-    pg::launch_collect_status(nq, seeds, m->status.as<int32_t>(), code, out, fl, of, tp, c, s);
+// Statuses of a list of seeds, from one collect.
+struct Tally {
+    int64_t match = 0;     // seeds with the code asked for
+    int64_t overflow = 0;  // seeds that outgrew the fast kernel's slots
+    int64_t other = 0;     // seeds with any other status but SUCCESS
+};
+
+// Seeds of `seeds` (nullptr: all) whose status equals code, into out, and
+// their tally.
+Tally collect(pg_mesh* m, const uint32_t* seeds, int64_t nq, int code, uint32_t* out, hipStream_t s) {
+    Tally t;
+    if (nq <= 0) return t;
+    unsigned long long h[3] = {0, 0, 0};
+    if (m->tally_next == pg_mesh::TALLIES) m->new_tallies(s);
+    unsigned long long* d = m->tallies.as<unsigned long long>() + 3 * m->tally_next++;
+    pg::launch_collect(nq, nullptr, seeds, m->status.as<int32_t>(), code, out, d, true, s);
     HIPCHK(hipGetLastError());
-    return read_i32(c, s);
+    HIPCHK(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    t.match = (int64_t)h[0];
+    t.overflow = (int64_t)h[1];
+    t.other = (int64_t)h[2];
+    return t;
+}
+int64_t collect_list(pg_mesh* m, const uint32_t* seeds, int64_t nq, int code, uint32_t* out, hipStream_t s) {
+    return collect(m, seeds, nq, code, out, s).match;
 }
 
 // The shape tag under which the fast clip kernel saves and resumes cells.
@@ -333,15 +363,25 @@ int next_k(int k, int cap) {
 constexpr int BIG_ROW = 256;
 int big_row(int k, int cap, bool restart) { return restart ? std::max(k, std::min(cap, BIG_ROW)) : k; }
 
+// What a restart chain knows of the statuses it leaves (of all its seeds):
+// nothing when !known.
+struct ChainEnd {
+    bool known = false;
+    int64_t uncertified = 0, overflow = 0, other = 0;
+    bool clean() const { return known && uncertified == 0 && overflow == 0 && other == 0; }
+};
+
 // Seeds cur[0..nq) (nullptr: all) were just clipped with rows of length k;
 // uncertified seeds go on at the next k, until all pass or k reaches its
 // cap.  Seeds that outgrow the fast kernel's vertex slots keep that status
 // through the chain, and the 128-slot kernel clips all of them once, at
 // big_row(k), when the chain's k would pass that row (or the chain ends);
 // after every longer step it runs again, and the next step's list is then
-// taken over all of cur, so that its uncertified seeds continue too.
-// Returns the largest k used.
-int restart_chain(pg_mesh* m, const uint32_t* cur, int64_t nq, int k, hipStream_t s) {
+// taken over all of cur, so that its uncertified seeds continue too.  One
+// collect (and one synchronisation) per step tells both what goes on and
+// whether anything overflowed or failed, so a chain that leaves neither needs
+// no further look at the statuses.  Returns the largest k used.
+int restart_chain(pg_mesh* m, const uint32_t* cur, int64_t nq, int k, hipStream_t s, ChainEnd* end = nullptr) {
     const pg_mesh_params& p = m->prm;
     const size_t ns = (size_t)m->n_seeds;
     uint32_t* buf[2] = {m->list.get<uint32_t>(ns), m->list2.get<uint32_t>(ns)};
@@ -349,48 +389,58 @@ int restart_chain(pg_mesh* m, const uint32_t* cur, int64_t nq, int k, hipStream_
     const int cap = (int)std::min<int64_t>(std::min(std::max(p.k_max, k), KNN_MAX_K), m->n_seeds - 1);
     const bool restart = p.restart != 0;
     const int kb = big_row(k, cap, restart);
-    const uint32_t* L = cur;
-    int64_t nL = nq;
     int kmax = k;
     bool big_done = false;
-    auto big_pass = [&](int kk) -> int64_t {
+    ChainEnd st;
+    uint32_t* L = buf[0];  // the uncertified seeds (st.uncertified of them)
+    auto look_all = [&] {
+        const Tally t = collect(m, cur, nq, PG_SECURITY_RADIUS_NOT_REACHED, L, s);
+        st = {true, t.match, t.overflow, t.other};
+    };
+    auto big_pass = [&](int kk) {
         const int64_t no = collect_list(m, cur, nq, pg::SLOT_OVERFLOW, ov, s);
-        if (no > 0) {
-            run_list(m, ov, no, kk, 1, s);
-            m->info.n_restarted += no;
-            kmax = std::max(kmax, kk);
-            L = cur;
-            nL = nq;
-        }
+        run_list(m, ov, no, kk, 1, s);
+        m->info.n_restarted += no;
+        kmax = std::max(kmax, kk);
         return no;
     };
-    while (restart && nL > 0) {
+    look_all();
+    while (restart) {
         const int kn = next_k(k, cap);
         if (kn < 0) break;
         if (!big_done && kn > kb) {
-            big_pass(kb);
             big_done = true;
+            if (st.overflow > 0) {
+                big_pass(kb);
+                look_all();
+            }
         }
-        uint32_t* dst = (L == buf[0]) ? buf[1] : buf[0];
-        const int64_t nr = collect_list(m, L, nL, PG_SECURITY_RADIUS_NOT_REACHED, dst, s);
-        if (nr == 0) break;
+        if (st.uncertified == 0) break;
         k = kn;
-        run_list(m, dst, nr, k, 0, s);
-        m->info.n_restarted += nr;
+        run_list(m, L, st.uncertified, k, 0, s);
+        m->info.n_restarted += st.uncertified;
         kmax = std::max(kmax, k);
+        uint32_t* dst = L == buf[0] ? buf[1] : buf[0];
+        const Tally t = collect(m, L, st.uncertified, PG_SECURITY_RADIUS_NOT_REACHED, dst, s);
         L = dst;
-        nL = nr;
-        if (big_done) big_pass(k);
+        st.uncertified = t.match;
+        st.overflow += t.overflow;
+        st.other += t.other;
+        if (big_done && st.overflow > 0) {
+            big_pass(k);
+            look_all();
+        }
     }
-    if (!big_done) {
+    if (!big_done && st.overflow > 0) {
         const int64_t no = big_pass(kb);
+        st.known = false;
         // a 128-slot pass below the cap may leave seeds that longer rows
         // certify: they continue in a chain from kb (the only uncertified
         // seeds of cur at this point)
-        if (restart && no > 0 && kb < cap &&
-            collect_list(m, ov, no, PG_SECURITY_RADIUS_NOT_REACHED, buf[0], s) > 0)
-            kmax = std::max(kmax, restart_chain(m, cur, nq, kb, s));
+        if (restart && kb < cap && collect_list(m, ov, no, PG_SECURITY_RADIUS_NOT_REACHED, buf[0], s) > 0)
+            kmax = std::max(kmax, restart_chain(m, cur, nq, kb, s, &st));
     }
+    if (end) *end = st;
     return kmax;
 }
 
@@ -537,14 +587,16 @@ void mesh_build_once(pg_ctx* c, pg_mesh* m, const double* pts, int64_t n, bool o
     m->lanes = pg::clip_lanes();
     m->slots = pg::clip_slots();
     if (m->use_resume) {
+        // the first pass sets every seed's resume entry: no restart resumes a
+        // cell of an earlier build (or of recycled memory)
         m->cstate.get<uint8_t>(ns * pg::CLIP_STATE_BYTES);
         m->lastnb.get<uint32_t>(ns);
-        // saved cells belong to this build only: no pass may resume a cell
-        // of an earlier build (or of recycled memory)
-        pg::launch_fill_i32(m->resume.get<int32_t>(ns), (int64_t)ns, 0, s);
+        m->resume.get<int32_t>(ns);
     }
     m->finalized = false;
+    m->new_tallies(s);
 
+    ChainEnd end;
     m->info = pg_mesh_info_t{};
     m->learned_rows = km != nullptr;
     int k_used = p.k;
@@ -564,7 +616,7 @@ void mesh_build_once(pg_ctx* c, pg_mesh* m, const double* pts, int64_t n, bool o
         HIPCHK(hipGetLastError());
         m->info.row_entries += nseeds * k;
         if (mk) mk->mark(MK_CLIP, s);
-        k_used = restart_chain(m, nullptr, nseeds, k, s);
+        k_used = restart_chain(m, nullptr, nseeds, k, s, &end);
     } else {
         // learned first pass: features -> bucket per seed -> seeds grouped by
         // bucket (ascending id inside a bucket) -> KNN + clip per bucket
@@ -625,17 +677,18 @@ void mesh_build_once(pg_ctx* c, pg_mesh* m, const double* pts, int64_t n, bool o
         // a seed recomputed at a row length at least its certified k gives
         // the same cell whatever its first bucket, so the chain may start at
         // 64 (overflowed seeds at 64, uncertified ones at 128, then 256)
-        k_used = std::max(restart_chain(m, nullptr, nseeds, std::min<int64_t>(64, nseeds - 1), s),
+        k_used = std::max(restart_chain(m, nullptr, nseeds, std::min<int64_t>(64, nseeds - 1), s, &end),
                           *std::max_element(bk, bk + pg::LK_NCLASS));
     }
-    if (p.restart) ball_pass(m, s);
-    if (p.exact) k_used = std::max(k_used, exact_chain(m, s));
+    // a chain that left every cell certified has nothing to complete or count
+    if (p.restart && !(end.known && end.uncertified == 0)) ball_pass(m, s);
+    if (p.exact && !end.clean()) k_used = std::max(k_used, exact_chain(m, s));
     if (mk) mk->mark(MK_RESTART, s);
     m->info.n_seeds = nseeds;
     m->info.n_hydro = m->n_hydro;
     m->info.N_grid = m->g.N;
     m->info.k_used = k_used;
-    m->info.n_failed = collect_list(m, nullptr, nseeds, -1, m->list.get<uint32_t>(ns), s);
+    if (!end.clean()) m->info.n_failed = collect_list(m, nullptr, nseeds, -1, m->list.get<uint32_t>(ns), s);
     if (count) count_faces(m, s);
 }
 
@@ -674,14 +727,9 @@ void mesh_build(pg_ctx* c, pg_mesh* m, const double* pts, int64_t n, bool on_dev
 
 // Total faces over all cells (VMesh.num_faces).
 void count_faces(pg_mesh* m, hipStream_t s) {
-    const size_t ns = (size_t)m->n_seeds;
-    const int64_t nseeds = m->n_seeds;
-    int32_t* co = m->flags.get<int32_t>(ns);
-    int32_t* po = m->offs.get<int32_t>(ns);
-    int32_t* tp = m->g.tmp.get<int32_t>(pg::scan_tmp_elems(std::max<int64_t>(nseeds, m->g.ncell)));
-    pg::launch_counts_orig(nseeds, m->out_order(), m->count.as<uint8_t>(), co, s);
-    pg::scan_exclusive_i32(co, po, nseeds, tp, m->cnt1.get<int32_t>(1), s);
-    m->info.num_faces = read_i32(m->cnt1.as<int32_t>(), s);
+    int32_t* total = m->new_bad(s) + 2;
+    pg::launch_face_total(m->n_seeds, m->count.as<uint8_t>(), total, s);
+    m->info.num_faces = read_i32(total, s);
 }
 
 void mesh_finalize(pg_ctx* c, pg_mesh* m) {
@@ -690,8 +738,7 @@ void mesh_finalize(pg_ctx* c, pg_mesh* m) {
     const size_t ns = (size_t)m->n_seeds;
     const double sc = m->scale();
     const double vs = m->prm.dim == 2 ? sc * sc : sc * sc * sc;
-    int32_t* bad = m->bad.get<int32_t>(2);
-    HIPCHK(hipMemsetAsync(bad, 0, 2 * sizeof(int32_t), s));
+    int32_t* bad = m->new_bad(s);
     const int64_t* gsrc = m->prm.boundary == PG_BOUNDARY_PERIODIC ? m->gsrc.as<int64_t>() : nullptr;
     pg::launch_finalize(m->n_seeds, m->n_hydro, m->n_seeds, m->out_order(), gsrc, m->count.as<uint8_t>(),
                         m->nbr.as<int32_t>(), m->vol.as<double>(), vs, m->vol_u.get<double>(ns),
@@ -699,17 +746,12 @@ void mesh_finalize(pg_ctx* c, pg_mesh* m) {
     HIPCHK(hipGetLastError());
     // faces over all cells (VMesh.num_faces), read with the error counters:
     // meshes built on the device (simulations) learn their face count here
-    int32_t* co = m->flags.get<int32_t>(ns);
-    int32_t* po = m->offs.get<int32_t>(ns);
-    int32_t* tp = m->g.tmp.get<int32_t>(pg::scan_tmp_elems(std::max<int64_t>(m->n_seeds, m->g.ncell)));
-    pg::launch_counts_orig(m->n_seeds, m->out_order(), m->count.as<uint8_t>(), co, s);
-    pg::scan_exclusive_i32(co, po, m->n_seeds, tp, m->cnt1.get<int32_t>(1), s);
+    pg::launch_face_total(m->n_seeds, m->count.as<uint8_t>(), bad + 2, s);
     HIPCHK(hipGetLastError());
-    int32_t hb[2] = {0, 0}, nf = 0;
+    int32_t hb[3] = {0, 0, 0};
     HIPCHK(hipMemcpyAsync(hb, bad, sizeof(hb), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(&nf, m->cnt1.as<int32_t>(), sizeof(nf), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
-    m->info.num_faces = nf;
+    m->info.num_faces = hb[2];
     if (hb[0] != 0) throw Error{PG_ERR_CELLS, "hydro cells without faces (uncertified cells)"};
     if (hb[1] != 0)
         throw Error{PG_ERR_CELLS, std::to_string(hb[1]) +
@@ -1049,6 +1091,7 @@ int pg_voronoi_compute(pg_ctx* c, const pg_knn* kc, int max_p, int max_t, pg_mes
             m->lanes = pg::clip_lanes();
             m->slots = pg::clip_slots();
             m->finalized = false;
+            m->new_tallies(s);
             m->info = pg_mesh_info_t{};
             pg::launch_voronoi(dim, g.sorted.as<double>(), n, nullptr, n, rows, k, max_p, max_t, 0, m->faces(),
                                m->lanes, m->slots, s);
@@ -1385,10 +1428,8 @@ void sim_hydro(pg_ctx* c, pg_sim* S, double dt_max, bool moving) {
     pg_mesh& m = S->mesh;
     const int dim = S->prm.mesh.dim;
     const double sc = m.scale();
-    pg::launch_prim_from_q(dim, S->view(), m.o2s.as<int32_t>(), m.vol_u.as<double>(), s);
     unsigned long long* d = S->dt.get<unsigned long long>(1);
-    const double init = 1e100;
-    HIPCHK(hipMemcpyAsync(d, &init, sizeof(double), hipMemcpyHostToDevice, s));
+    pg::launch_prim_from_q(dim, S->view(), m.o2s.as<int32_t>(), m.vol_u.as<double>(), s, (double*)d);
     const double* w = nullptr;  // steered generator velocities (regularised motion)
     if (moving && S->prm.move_mesh == PG_MOVE_REGULARIZED) {
         double* wg = S->wgen.get<double>((size_t)S->n * dim);
@@ -1515,7 +1556,7 @@ int pg_sim_step(pg_ctx* c, pg_sim* S, double dt_max, double* dt_used) {
             sim_rebuild(c, S, &mk);
         }
         mk.mark(MK_END, s);
-        HIPCHK(hipStreamSynchronize(s));
+        double dt = sim_read_dt(c, S, dt_max);  // ends with the step's synchronisation
         auto el = [&](int a, int b) {
             float ms = 0;
             HIPCHK(hipEventElapsedTime(&ms, mk.ev[a], mk.ev[b]));
@@ -1534,7 +1575,6 @@ int pg_sim_step(pg_ctx* c, pg_sim* S, double dt_max, double* dt_used) {
         t.total_ms = el(MK_START, MK_END);
         t.n_restarted = S->mesh.info.n_restarted;
         t.k_used = S->mesh.info.k_used;
-        double dt = sim_read_dt(c, S, dt_max);
         if (dt_used) *dt_used = dt;
         });
     });
@@ -1909,8 +1949,6 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
     const pg_mesh_params& p = B->prm.mesh;
     const int64_t cap = B->cap;
     pg::launch_fill_i32(B->st(), 4, 0, s);
-    // saved cells belong to this rebuild only
-    if (B->resume.p) pg::launch_fill_i32(B->resume.as<int32_t>(), cap, 0, s);
     const int32_t* goff = nullptr;
     if (B->periodic) {
         pg::launch_ghost_count(dim, B->x.as<double>(), B->n_h, p.buff, B->gcnt.as<int32_t>(), s);
@@ -1945,8 +1983,8 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
                             restart_list, s);
     };
     auto collect = [&](const uint32_t* L, const int64_t* nL, int code, uint32_t* out, int64_t* nout) {
-        pg::launch_bcollect(nL, cap, L, B->status.as<int32_t>(), code, out, B->flags.as<int32_t>(),
-                            B->offs.as<int32_t>(), B->tmp.as<int32_t>(), B->total.as<int32_t>(), nout, s);
+        pg::launch_fill_u64((unsigned long long*)nout, 1, 0ull, s);
+        pg::launch_collect(cap, nL, L, B->status.as<int32_t>(), code, out, (unsigned long long*)nout, false, s);
     };
     // first pass: every seed at the fixed k, or every bucket of the learned
     // k at its own k; then the restart chain of the single-box build

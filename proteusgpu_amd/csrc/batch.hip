@@ -315,33 +315,9 @@ __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES))
     const int64_t vb = blockIdx.x;
     if (vb * C::SPW >= nq) return;  // whole block
     // no box holds k + 1 seeds or fewer: the exhaustive-row rule never applies
-    voronoi_group<DIM, G, S>(args.pts, INT64_MAX, args.seeds, nq, args.knn, args.k, args.max_p, args.max_t,
-                             args.fa.resume, args.fa.cstate, args.fa.key, sm, vb);
-}
-
-// status == code (code < 0: != SUCCESS) among the listed seeds
-__global__ void __launch_bounds__(TB)
-    k_bflag(const int64_t* __restrict__ nq_dev, int64_t cap, const uint32_t* __restrict__ seeds,
-            const int32_t* __restrict__ status, int code, int32_t* __restrict__ flags) {
-    const int64_t nq = *nq_dev;
-    for (int64_t i = (int64_t)blockIdx.x * TB + threadIdx.x; i < cap; i += (int64_t)gridDim.x * TB) {
-        int f = 0;
-        if (i < nq) {
-            const int st = status[seeds ? seeds[i] : (uint32_t)i];
-            f = code < 0 ? (st != SUCCESS) : (st == code);
-        }
-        flags[i] = f;
-    }
-}
-
-__global__ void __launch_bounds__(TB)
-    k_bcompact(const int64_t* __restrict__ nq_dev, const uint32_t* __restrict__ seeds,
-               const int32_t* __restrict__ flags, const int32_t* __restrict__ offs, const int32_t* __restrict__ total,
-               uint32_t* __restrict__ list, int64_t* __restrict__ nout) {
-    const int64_t nq = *nq_dev;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *nout = *total;
-    for (int64_t i = (int64_t)blockIdx.x * TB + threadIdx.x; i < nq; i += (int64_t)gridDim.x * TB)
-        if (flags[i]) list[offs[i]] = seeds ? seeds[i] : (uint32_t)i;
+    // a first pass resumes nothing, and sets every seed's resume entry
+    voronoi_group<DIM, G, S>(args.pts, INT64_MAX, args.seeds, nq, args.knn, args.k, args.max_p, args.max_t, nullptr,
+                             nullptr, args.fa.key, sm, vb);
 }
 
 // ------------------------------------------------------------------ hydro
@@ -504,9 +480,7 @@ void launch_bgrid(int dim, const double* pts, const int64_t* n_dev, int64_t cap,
                   int32_t* starts, int32_t* fill, int32_t* tmp, int32_t* total, uint32_t* perm, double* sorted,
                   int32_t* sorted_box, int32_t* big, hipStream_t s) {
     const unsigned gb = std::min<unsigned>(nblk(cap), 2048);
-    const unsigned gc = std::min<unsigned>(nblk(cell_cap), 2048);
-    k_fill<int32_t><<<gc, TB, 0, s>>>(counts, cell_cap, 0);
-    k_fill<int32_t><<<gc, TB, 0, s>>>(fill, cell_cap, 0);
+    launch_grid_clear(cell_cap, counts, fill, big, s);
     if (dim == 2) k_bcell_count<2><<<gb, TB, 0, s>>>(pts, n_dev, cap, sbox, N, coff, cell, counts);
     else k_bcell_count<3><<<gb, TB, 0, s>>>(pts, n_dev, cap, sbox, N, coff, cell, counts);
     scan_exclusive_i32(counts, starts, cell_cap, tmp, total, s);
@@ -608,15 +582,6 @@ void launch_bvoronoi(int dim, const double* sorted, const uint32_t* seeds, const
     else go(std::integral_constant<int, 3>{});
 }
 
-void launch_bcollect(const int64_t* nq_dev, int64_t cap, const uint32_t* seeds, const int32_t* status, int code,
-                     uint32_t* list, int32_t* flags, int32_t* offs, int32_t* tmp, int32_t* total, int64_t* nout,
-                     hipStream_t s) {
-    const unsigned gb = std::min<unsigned>(nblk(cap), 2048);
-    k_bflag<<<gb, TB, 0, s>>>(nq_dev, cap, seeds, status, code, flags);
-    scan_exclusive_i32(flags, offs, cap, tmp, total, s);
-    k_bcompact<<<gb, TB, 0, s>>>(nq_dev, seeds, flags, offs, total, list, nout);
-}
-
 void launch_bfinalize(const int64_t* n_dev, int64_t cap, int64_t stride, const uint32_t* perm, const int32_t* orig_h,
                       const uint8_t* count, const int32_t* nbr, const double* vol, double vscale, int periodic,
                       double* vol_u, int32_t* o2s, int32_t* hcode, int32_t* bad, hipStream_t s) {
@@ -649,6 +614,10 @@ void launch_btotals(int dim, int nbox, const int64_t* hoff, SimView sv, double* 
 
 void launch_bcount_failed(const int64_t* n_dev, int64_t cap, const int32_t* status, int32_t* nfail, hipStream_t s) {
     k_bcount_failed<2><<<std::min<unsigned>(nblk(cap), 1024), TB, 0, s>>>(n_dev, status, nfail);
+}
+
+void launch_fill_u64(unsigned long long* a, int64_t n, unsigned long long v, hipStream_t s) {
+    k_fill<unsigned long long><<<std::min<unsigned>(nblk(n), 1024), TB, 0, s>>>(a, n, v);
 }
 
 void launch_fill_i32(int32_t* a, int64_t n, int32_t v, hipStream_t s) {

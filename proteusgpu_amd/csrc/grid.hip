@@ -194,12 +194,19 @@ __global__ void __launch_bounds__(TB) k_displace(const double* in, int64_t n, do
 
 inline unsigned nblk(int64_t n) { return (unsigned)((n + TB - 1) / TB); }
 
-__global__ void k_fill_one(int32_t* p) {
-    if (threadIdx.x == 0) *p = 0;
-}
-
-__global__ void __launch_bounds__(TB) k_fill_i32(int32_t* a, int64_t n, int32_t v) {
-    for (int64_t i = (int64_t)blockIdx.x * TB + threadIdx.x; i < n; i += (int64_t)gridDim.x * TB) a[i] = v;
+// Zeroes a grid build's counters: per cell counts, fill and m (optional),
+// and the scalars nbig and alloc (optional).
+__global__ void __launch_bounds__(TB) k_grid_clear(int64_t ncell, int32_t* counts, int32_t* fill, int32_t* m,
+                                                   int32_t* nbig, int32_t* alloc) {
+    for (int64_t i = (int64_t)blockIdx.x * TB + threadIdx.x; i < ncell; i += (int64_t)gridDim.x * TB) {
+        counts[i] = 0;
+        fill[i] = 0;
+        if (m) m[i] = 0;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *nbig = 0;
+        if (alloc) *alloc = 0;
+    }
 }
 
 // One block per listed cell (grid-stride over the list of cells longer than
@@ -298,6 +305,12 @@ void launch_ghost_write(int dim, const double* pts, int64_t n, double buff, cons
         k_ghost_write<3><<<nblk(n), TB, 0, s>>>(pts, n, buff, off, out, gsrc);
 }
 
+void launch_grid_clear(int64_t ncell, int32_t* counts, int32_t* fill, int32_t* nbig, hipStream_t s, int32_t* m,
+                       int32_t* alloc) {
+    k_grid_clear<<<(unsigned)std::min<int64_t>(std::max<int64_t>(nblk(ncell), 1), 2048), TB, 0, s>>>(ncell, counts, fill, m,
+                                                                                                  nbig, alloc);
+}
+
 void launch_cell_count(int dim, const double* pts, int64_t n, int N, int32_t* cell,
                        int32_t* counts, hipStream_t s) {
     if (n <= 0) return;
@@ -316,7 +329,6 @@ void launch_cell_scatter(int64_t n, const int32_t* cell, const int32_t* starts, 
 void launch_cell_sort(int64_t ncell, const int32_t* starts, const int32_t* counts, uint32_t* idx,
                       int32_t* big, int32_t* nbig, hipStream_t s) {
     if (ncell <= 0) return;
-    k_fill_one<<<1, 64, 0, s>>>(nbig);
     k_cell_sort<<<nblk(ncell), TB, 0, s>>>(ncell, starts, counts, idx, big, nbig);
     k_cell_sort_big<<<(unsigned)std::min<int64_t>(ncell, 1024), TB, 0, s>>>(big, nbig, starts, counts, idx);
 }
@@ -325,8 +337,6 @@ void launch_subgrid(int dim, const double* sorted, int64_t n, int N, int64_t nce
                     const int32_t* counts, const int32_t* big, const int32_t* nbig, int32_t* m, int32_t* ptr,
                     int32_t* start, int32_t* cnt, int64_t cap, uint32_t* idx, int32_t* alloc, hipStream_t s) {
     if (ncell <= 0 || n <= 0) return;
-    k_fill_i32<<<(unsigned)std::min<int64_t>(nblk(ncell), 4096), TB, 0, s>>>(m, ncell, 0);
-    k_fill_one<<<1, 64, 0, s>>>(alloc);
     const unsigned nb = (unsigned)std::min<int64_t>(ncell, 1024);
     if (dim == 2)
         k_sub_build<2><<<nb, TB, 0, s>>>(big, nbig, starts, counts, sorted, N, m, ptr, start, cnt, cap, idx, alloc);

@@ -35,7 +35,10 @@ struct CellRec {
 };
 
 void launch_q_from_prim(int dim, SimView sv, const int32_t* o2s, const double* vol_u, hipStream_t s);
-void launch_prim_from_q(int dim, SimView sv, const int32_t* o2s, const double* vol_u, hipStream_t s);
+void launch_prim_from_q(int dim, SimView sv, const int32_t* o2s, const double* vol_u, hipStream_t s,
+                        double* dt_init = nullptr);
+// *total (zeroed before) += the sum of the n face counts.
+void launch_face_total(int64_t n, const uint8_t* count, int32_t* total, hipStream_t s);
 // Owner-computes-once moving-mesh update.  hcode per sorted seed: hydro
 // id, or -1 - (hydro id of the source) for a periodic ghost.  Seeds: n, or
 // *n_dev when n_dev is set (batches: n is then the capacity).

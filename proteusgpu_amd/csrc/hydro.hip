@@ -202,9 +202,13 @@ __global__ void __launch_bounds__(TB) k_q_from_prim(SimView sv, const int32_t* o
     sv.en[i] = sv.E[i] * V;
 }
 
+// dt_init (optional): set to the CFL minimum's start (finite_volume_solver.cpp:153)
+// for the launch_dt_cfl that follows.
 template <int DIM>
-__global__ void __launch_bounds__(TB) k_prim_from_q(SimView sv, const int32_t* o2s, const double* vol_u) {
+__global__ void __launch_bounds__(TB)
+    k_prim_from_q(SimView sv, const int32_t* o2s, const double* vol_u, double* dt_init) {
     int64_t i = (int64_t)blockIdx.x * TB + threadIdx.x;
+    if (i == 0 && dt_init) *dt_init = 1e100;
     if (i >= sv.n_hydro) return;
     const double V = vol_u[o2s[i]];
     const double m = sv.mass[i];
@@ -523,6 +527,20 @@ __global__ void __launch_bounds__(TB) k_totals(SimView sv, double* part) {
         for (int q = 0; q < 5; q++) part[(size_t)5 * blockIdx.x + q] = red[q][0];
 }
 
+// Sum of the face counts (VMesh.num_faces), one atomic per block.
+__global__ void __launch_bounds__(TB) k_face_total(int64_t n, const uint8_t* __restrict__ count, int32_t* total) {
+    int c = 0;
+    for (int64_t s = (int64_t)blockIdx.x * TB + threadIdx.x; s < n; s += (int64_t)gridDim.x * TB) c += count[s];
+    for (int d = 32; d > 0; d >>= 1) c += __shfl_xor(c, d, 64);
+    __shared__ int wc[TB / 64];
+    if ((threadIdx.x & 63) == 0) wc[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < TB / 64; w++) c += wc[w];
+        if (c) atomicAdd(total, c);
+    }
+}
+
 // Copy-out: face counts in original order.
 __global__ void __launch_bounds__(TB) k_counts_orig(int64_t n, const uint32_t* perm,
                                                     const uint8_t* count, int32_t* co) {
@@ -635,10 +653,10 @@ void launch_q_from_prim(int dim, SimView sv, const int32_t* o2s, const double* v
     else k_q_from_prim<3><<<nblk(sv.n_hydro), TB, 0, s>>>(sv, o2s, vol_u);
 }
 
-void launch_prim_from_q(int dim, SimView sv, const int32_t* o2s, const double* vol_u, hipStream_t s) {
+void launch_prim_from_q(int dim, SimView sv, const int32_t* o2s, const double* vol_u, hipStream_t s, double* dt_init) {
     if (sv.n_hydro <= 0) return;
-    if (dim == 2) k_prim_from_q<2><<<nblk(sv.n_hydro), TB, 0, s>>>(sv, o2s, vol_u);
-    else k_prim_from_q<3><<<nblk(sv.n_hydro), TB, 0, s>>>(sv, o2s, vol_u);
+    if (dim == 2) k_prim_from_q<2><<<nblk(sv.n_hydro), TB, 0, s>>>(sv, o2s, vol_u, dt_init);
+    else k_prim_from_q<3><<<nblk(sv.n_hydro), TB, 0, s>>>(sv, o2s, vol_u, dt_init);
 }
 
 // grid: every seed once (host count), or a capped grid-stride grid over
@@ -687,6 +705,11 @@ void launch_drift(int dim, int64_t n, double* x, const double* vel, const double
     if (n <= 0) return;
     if (dim == 2) k_drift<2><<<nblk(n), TB, 0, s>>>(n, x, vel, dt_dev, dt_max, periodic);
     else k_drift<3><<<nblk(n), TB, 0, s>>>(n, x, vel, dt_dev, dt_max, periodic);
+}
+
+void launch_face_total(int64_t n, const uint8_t* count, int32_t* total, hipStream_t s) {
+    if (n <= 0) return;
+    k_face_total<<<std::min<unsigned>(nblk(n), 256), TB, 0, s>>>(n, count, total);
 }
 
 int64_t totals_blocks(int64_t n) { return (int64_t)nblk(n); }

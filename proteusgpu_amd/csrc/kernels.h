@@ -21,6 +21,11 @@ void launch_ghost_count(int dim, const double* pts, int64_t n, double buff, int3
 // ghosts in (point, region) order; ghost_src[g] = source hydro index.
 void launch_ghost_write(int dim, const double* pts, int64_t n, double buff, const int32_t* off,
                         double* out, int64_t* ghost_src, hipStream_t s);
+// Zero a grid build's counters before it: counts, fill (ncell each) and the
+// list length nbig of launch_cell_sort; for a sub-grid build also its m (ncell)
+// and alloc.  By a kernel: the sequence may be captured.
+void launch_grid_clear(int64_t ncell, int32_t* counts, int32_t* fill, int32_t* nbig, hipStream_t s,
+                       int32_t* m = nullptr, int32_t* alloc = nullptr);
 // knn.cpp:119-222: grid cell of every point and per-cell counts.
 void launch_cell_count(int dim, const double* pts, int64_t n, int N, int32_t* cell,
                        int32_t* counts, hipStream_t s);
@@ -29,7 +34,7 @@ void launch_cell_scatter(int64_t n, const int32_t* cell, const int32_t* starts, 
                          uint32_t* idx, hipStream_t s);
 // Sort every cell's range ascending: the order of the reference's serial
 // store loop (knn.cpp:187-204), i.e. stable by input index.  big (ncell
-// int32) and nbig (one int32) are scratch for ranges longer than 32.
+// int32) and nbig (one int32, zeroed) list the ranges longer than 32.
 void launch_cell_sort(int64_t ncell, const int32_t* starts, const int32_t* counts, uint32_t* idx,
                       int32_t* big, int32_t* nbig, hipStream_t s);
 // out = in displaced by at most amp per axis, deterministically from each
@@ -60,7 +65,7 @@ struct SubGrid {
 // Build it after launch_cell_sort (whose list of cells longer than 32 it
 // takes) and launch_gather_points.  m, ptr: ncell int32; start, cnt: cap
 // int32 (cap >= n / 3 + 64 always suffices); idx: n uint32; alloc: one
-// int32 of scratch.
+// int32; m and alloc zeroed (launch_grid_clear).
 void launch_subgrid(int dim, const double* sorted, int64_t n, int N, int64_t ncell, const int32_t* starts,
                     const int32_t* counts, const int32_t* big, const int32_t* nbig, int32_t* m, int32_t* ptr,
                     int32_t* start, int32_t* cnt, int64_t cap, uint32_t* idx, int32_t* alloc, hipStream_t s);
@@ -163,13 +168,13 @@ int clip_slots();
 // Certificate restarts resume saved cells (true) or clip from scratch.
 bool clip_resume();
 void set_clip_resume(bool on);
-// Collect the sorted ids whose status is not SUCCESS (order: ascending id).
-// nfail (device int32) receives the count; tmp as for scan.
-void launch_collect_failed(int64_t n, const int32_t* status, uint32_t* list, int32_t* flags,
-                           int32_t* offs, int32_t* tmp, int32_t* nfail, hipStream_t s);
-void launch_collect_status(int64_t nq, const uint32_t* seeds, const int32_t* status, int code,
-                           uint32_t* list, int32_t* flags, int32_t* offs, int32_t* tmp,
-                           int32_t* nout, hipStream_t s);
+// Collect the seeds (nullptr: 0..nq-1; nq = *nq_dev when nq_dev is set, nq
+// then the capacity) whose status equals code (code < 0: is not SUCCESS)
+// into list (ascending in runs of 2048, the runs in any order).  tally[0],
+// zeroed before, receives their number; with counts, tally[1] the seeds with
+// SLOT_OVERFLOW and tally[2] those with any other status but SUCCESS.
+void launch_collect(int64_t nq, const int64_t* nq_dev, const uint32_t* seeds, const int32_t* status, int code,
+                    uint32_t* list, unsigned long long* tally, bool counts, hipStream_t s);
 
 // ---------------------------------------------------------- learned_k.hip
 // Classifier of the neighbour count: 16 features -> 64 -> 64 -> 6 buckets.
@@ -262,11 +267,9 @@ void launch_bknn(int dim, const double* sorted, const uint32_t* perm, const int3
 void launch_bvoronoi(int dim, const double* sorted, const uint32_t* seeds, const int64_t* nq_dev, int64_t cap,
                      const uint32_t* knn, int k, int max_p, int max_t, int big, int lanes, int slots, FaceArrays fa,
                      int blocks_per_cu, unsigned long long* ticket, bool loop, hipStream_t s);
-void launch_bcollect(const int64_t* nq_dev, int64_t cap, const uint32_t* seeds, const int32_t* status, int code,
-                     uint32_t* list, int32_t* flags, int32_t* offs, int32_t* tmp, int32_t* total, int64_t* nout,
-                     hipStream_t s);
 void launch_bcount_failed(const int64_t* n_dev, int64_t cap, const int32_t* status, int32_t* nfail, hipStream_t s);
 void launch_fill_i32(int32_t* a, int64_t n, int32_t v, hipStream_t s);
+void launch_fill_u64(unsigned long long* a, int64_t n, unsigned long long v, hipStream_t s);
 // ------------------------------------------------------------- noalloc.hip
 // Size of the static device array behind the allocation-free entry points
 // (one copy per GPU, held until the process ends).

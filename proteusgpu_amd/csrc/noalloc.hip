@@ -68,8 +68,7 @@ void noalloc_knn(void* base, int dim, const double* pts, int64_t n, int N, int k
     int32_t* total = carve(1);
     // the array keeps the last call's contents: clear the counters by kernel
     // (no memset node, so the sequence can be captured into a graph)
-    launch_fill_i32(counts, ncell, 0, s);
-    launch_fill_i32(fill, ncell, 0, s);
+    launch_grid_clear(ncell, counts, fill, big, s);
     launch_cell_count(dim, pts, n, N, cell, counts, s);
     scan_exclusive_i32(counts, starts, ncell, tmp, total, s);
     launch_cell_scatter(n, cell, starts, fill, perm, s);

@@ -1,5 +1,5 @@
 // Device-wide exclusive prefix sum (three passes: tile sums, scan of tile
-// sums, tile scan + offset).  Tiles of 1024 int32 per 256-thread block,
+// sums, tile scan + offset; short arrays: one).  Tiles of 1024 int32 per 256-thread block,
 // wave-level scans with DPP-backed shuffles.
 #include "common.h"
 #include "kernels.h"
@@ -85,6 +85,35 @@ __global__ void __launch_bounds__(TB) k_tile_apply(const int32_t* in, int32_t* o
     }
 }
 
+// Short arrays by one block: thread t scans a run of per consecutive values.
+// One launch instead of three (2.5 us each, and the gaps between them, at a
+// few thousand grid cells, where a step's kernels are shorter than that).
+constexpr int SB = 1024;
+constexpr int64_t SCAN_ONE = 16 * SB;
+__global__ void __launch_bounds__(SB) k_scan_one(const int32_t* in, int32_t* out, int n, int32_t* total) {
+    __shared__ int32_t wsum[SB / WAVE];
+    const int per = (n + SB - 1) / SB, b = threadIdx.x * per, e = min(n, b + per);
+    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+    int32_t v = 0;
+    for (int i = b; i < e; i++) v += in[i];
+    const int32_t inc = wave_incl_scan(v);
+    if (lane == WAVE - 1) wsum[w] = inc;
+    __syncthreads();
+    int32_t base = 0, all = 0;
+#pragma unroll
+    for (int i = 0; i < SB / WAVE; i++) {
+        if (i < w) base += wsum[i];
+        all += wsum[i];
+    }
+    int32_t run = base + inc - v;
+    for (int i = b; i < e; i++) {
+        const int32_t x = in[i];
+        out[i] = run;
+        run += x;
+    }
+    if (threadIdx.x == 0 && total) *total = all;
+}
+
 }  // namespace
 
 int64_t scan_tmp_elems(int64_t n) { return (n + TILE - 1) / TILE + 1; }
@@ -94,6 +123,10 @@ void scan_exclusive_i32(const int32_t* in, int32_t* out, int64_t n, int32_t* tmp
     int64_t nt = (n + TILE - 1) / TILE;
     if (nt == 0) {
         if (total) (void)hipMemsetAsync(total, 0, sizeof(int32_t), s);
+        return;
+    }
+    if (n <= SCAN_ONE) {
+        k_scan_one<<<1, SB, 0, s>>>(in, out, (int)n, total);
         return;
     }
     k_tile_sums<<<dim3((unsigned)nt), dim3(TB), 0, s>>>(in, n, tmp);

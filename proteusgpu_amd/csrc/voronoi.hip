@@ -14,12 +14,12 @@ namespace {
 template <int DIM, int G, int S>
 __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_voronoi(ClipArgs a) {
     __shared__ VoroSmem<DIM, G, S> sm[VoroCfg<DIM, G, S>::SPW];
-    voronoi_group<DIM, G, S>(a.pts, a.n_total, a.seeds, a.nq, a.knn, a.k, a.max_p, a.max_t, a.fa.resume, a.fa.cstate,
-                             a.fa.key, sm, xcd_block(blockIdx.x, gridDim.x));
+    // a first pass resumes nothing, and sets every seed's resume entry
+    voronoi_group<DIM, G, S>(a.pts, a.n_total, a.seeds, a.nq, a.knn, a.k, a.max_p, a.max_t, nullptr, nullptr, a.fa.key, sm,
+                             xcd_block(blockIdx.x, gridDim.x));
 }
 
-// The same kernel under its own name for certificate restarts, so that
-// profiles separate the first pass from the restarts.
+// Certificate restarts, which resume saved cells.
 template <int DIM, int G, int S>
 __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_voronoi_restart(ClipArgs a) {
     __shared__ VoroSmem<DIM, G, S> sm[VoroCfg<DIM, G, S>::SPW];
@@ -56,22 +56,57 @@ void run(const ClipArgs& a, bool restart, hipStream_t s) {
 }
 
 constexpr int TB = 256;
+constexpr int PER = 8;  // seeds per thread of a collect
 
-__global__ void __launch_bounds__(TB) k_flag_status(int64_t nq, const uint32_t* seeds,
-                                                    const int32_t* status, int code, int32_t* flags) {
-    int64_t i = (int64_t)blockIdx.x * TB + threadIdx.x;
-    if (i >= nq) return;
-    uint32_t s = seeds ? seeds[i] : (uint32_t)i;
-    int st = status[s];
-    flags[i] = (code < 0) ? (st != SUCCESS) : (st == code);
-}
-
-__global__ void __launch_bounds__(TB) k_compact(int64_t nq, const uint32_t* seeds,
-                                                const int32_t* flags, const int32_t* offs,
-                                                uint32_t* list) {
-    int64_t i = (int64_t)blockIdx.x * TB + threadIdx.x;
-    if (i >= nq || !flags[i]) return;
-    list[offs[i]] = seeds ? seeds[i] : (uint32_t)i;
+// A block's matches are counted first (per wave and round of 256 seeds), take
+// one range of the list by one atomic, and are written in order.  One launch
+// per collect; flags, a scan and a compaction were five.
+__global__ void __launch_bounds__(TB) k_collect(int64_t nq_host, const int64_t* __restrict__ nq_dev,
+                                                const uint32_t* __restrict__ seeds, const int32_t* __restrict__ status,
+                                                int code, uint32_t* __restrict__ list, unsigned long long* tally,
+                                                int counts) {
+    __shared__ int32_t cnt[PER][TB / WAVE];
+    __shared__ int64_t base_s;
+    const int64_t nq = nq_dev ? *nq_dev : nq_host;
+    const int64_t b0 = (int64_t)blockIdx.x * TB * PER;
+    if (b0 >= nq) return;  // whole block
+    const int w = threadIdx.x / WAVE, l = threadIdx.x & (WAVE - 1);
+    uint32_t id[PER];
+    bool hit[PER];
+    int ov = 0, other = 0;
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int64_t i = b0 + r * TB + threadIdx.x;
+        id[r] = i < nq ? (seeds ? seeds[i] : (uint32_t)i) : 0u;
+        const int st = i < nq ? status[id[r]] : SUCCESS;
+        hit[r] = code < 0 ? st != SUCCESS : st == code && i < nq;
+        const uint64_t m = (uint64_t)__ballot(hit[r]);
+        if (l == 0) cnt[r][w] = __popcll(m);
+        ov += st == SLOT_OVERFLOW;
+        other += !hit[r] && st != SUCCESS && st != SLOT_OVERFLOW;
+    }
+    if (counts) {
+        const uint64_t mo = (uint64_t)__ballot(ov != 0), mx = (uint64_t)__ballot(other != 0);
+        if (mo && ov) atomicAdd(tally + 1, (unsigned long long)ov);
+        if (mx && other) atomicAdd(tally + 2, (unsigned long long)other);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int t = 0;
+        for (int r = 0; r < PER; r++)
+            for (int v = 0; v < TB / WAVE; v++) {
+                const int c = cnt[r][v];
+                cnt[r][v] = t;
+                t += c;
+            }
+        base_s = t ? (int64_t)atomicAdd(tally, (unsigned long long)t) : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const uint64_t m = (uint64_t)__ballot(hit[r]);
+        if (hit[r]) list[base_s + cnt[r][w] + __popcll(m & ((1ull << l) - 1ull))] = id[r];
+    }
 }
 
 }  // namespace
@@ -152,19 +187,11 @@ void launch_voronoi_ball(int dim, const double* sorted, int64_t n, const uint32_
     else k_voronoi_ball<3><<<dim3(nb), dim3(64), 0, s>>>(a, bg);
 }
 
-void launch_collect_status(int64_t nq, const uint32_t* seeds, const int32_t* status, int code,
-                           uint32_t* list, int32_t* flags, int32_t* offs, int32_t* tmp,
-                           int32_t* nout, hipStream_t s) {
+void launch_collect(int64_t nq, const int64_t* nq_dev, const uint32_t* seeds, const int32_t* status, int code,
+                    uint32_t* list, unsigned long long* tally, bool counts, hipStream_t s) {
     if (nq <= 0) return;
-    unsigned nb = (unsigned)((nq + TB - 1) / TB);
-    k_flag_status<<<nb, TB, 0, s>>>(nq, seeds, status, code, flags);
-    scan_exclusive_i32(flags, offs, nq, tmp, nout, s);
-    k_compact<<<nb, TB, 0, s>>>(nq, seeds, flags, offs, list);
-}
-
-void launch_collect_failed(int64_t n, const int32_t* status, uint32_t* list, int32_t* flags,
-                           int32_t* offs, int32_t* tmp, int32_t* nfail, hipStream_t s) {
-    launch_collect_status(n, nullptr, status, -1, list, flags, offs, tmp, nfail, s);
+    k_collect<<<(unsigned)((nq + TB * PER - 1) / (TB * PER)), TB, 0, s>>>(nq, nq_dev, seeds, status, code, list, tally,
+                                                                          counts ? 1 : 0);
 }
 
 }  // namespace pg
