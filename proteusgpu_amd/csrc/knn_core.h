@@ -407,9 +407,9 @@ PG_DEV void key_merge_batch(uint32_t (&kk)[M], uint32_t& out, uint32_t a, int l,
 // skip only points outside the ball (the float bounds carry a slack of
 // several float roundings of N), so every point of the ball is seen.
 //
-// What bounds it: VALU issue (810 instructions per query, k = 32 and its 64
+// What bounds it: VALU issue (780 instructions per query, k = 32 and its 64
 // tails; the ring walk with FP64 sorts took 1.75k).  1M uniform 3D queries:
-// k = 32 2.4 -> 1.18 ms, k = 64 3.25 -> 1.50 ms.  One run of points per row
+// k = 32 2.4 -> 1.06 ms, k = 64 3.25 -> 1.39 ms.  One run of points per row
 // of cells replaces 27 and then 98 cells looked at one by one, the mark scan a
 // binary search per candidate, and an exchange of the sort takes three
 // integer instructions instead of a dozen.
@@ -671,8 +671,11 @@ PG_DEV void knn_wave_query(const double* __restrict__ sorted, const uint32_t* __
     };
 
     // points the first ball should hold: k and a margin for the spread of
-    // the count (about 1% of passes come out short on uniform seeds)
-    const float lam = 1.25f * (float)kfull + 3.0f * __builtin_sqrtf((float)kfull) + 6.0f;
+    // the count.  Measured on 1M uniform seeds (ms, 3D k = 32 and 64, 2D k = 16):
+    // 1.25 k + 3 sqrt(k) + 6 1.17, 1.49, .78; this 1.08, 1.42, .73; k +
+    // 1.8 sqrt(k) + 2 1.09, 1.42, .73, with more balls that come out short,
+    // which clustered seeds make dearer
+    const float lam = 1.05f * (float)kfull + 2.2f * __builtin_sqrtf((float)kfull) + 3.0f;
     double r2;  // +inf: no ball (the reference's walk alone)
     {
         // the first ball from the density of the 3^DIM block of cells
