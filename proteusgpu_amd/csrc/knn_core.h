@@ -407,7 +407,7 @@ PG_DEV void key_merge_batch(uint32_t (&kk)[M], uint32_t& out, uint32_t a, int l,
 // skip only points outside the ball (the float bounds carry a slack of
 // several float roundings of N), so every point of the ball is seen.
 //
-// What bounds it: VALU issue (780 instructions per query, k = 32 and its 64
+// What bounds it: VALU issue (710 instructions per query, k = 32 and its 64
 // tails; the ring walk with FP64 sorts took 1.75k).  1M uniform 3D queries:
 // k = 32 2.4 -> 1.06 ms, k = 64 3.25 -> 1.39 ms.  One run of points per row
 // of cells replaces 27 and then 98 cells looked at one by one, the mark scan a
@@ -690,6 +690,40 @@ PG_DEV void knn_wave_query(const double* __restrict__ sorted, const uint32_t* __
         }
         const int tot = (int)read_lane((uint32_t)wave_incl_sum(cnt), 63);
         r2 = knn_guess_r2<DIM>(p, N, tot, __popcll((unsigned long long)__ballot(in)), lam);
+        if (SUB) {
+            // beside and inside crowded cells that block's mean says little: a
+            // cluster within a cell is orders of magnitude denser, and a ball
+            // sized for the mean holds thousands of points to sort.  A seed
+            // with known neighbours takes their density, one in a crowded
+            // cell that of the sub-cells around it (unless they hold too few
+            // points to tell), another that of the cells that are not crowded
+            const int64_t cc = cbase + c;
+            const int m = sg.m[cc];
+            if (kp > 0) {
+                if (lo_d > 0.0)
+                    r2 = lo_d * (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf(lam / (float)kp) * (2.0f / DIM));
+            } else if (m > 0) {
+                int a[3] = {0, 0, 0};
+                const int ix[3] = {ci, cj, ck};
+#pragma unroll
+                for (int d = 0; d < DIM; d++) a[d] = max(0, min(m - 1, (int)floor((P[d] - (double)ix[d]) * (double)m)));
+                cnt = 0;
+                in = false;
+                if (l < (DIM == 3 ? 27 : 9)) {
+                    const int ii = a[0] + l % 3 - 1, jj = a[1] + (l / 3) % 3 - 1, kk = DIM == 3 ? a[2] + l / 9 - 1 : 0;
+                    in = ii >= 0 && jj >= 0 && kk >= 0 && ii < m && jj < m && (DIM == 2 || kk < m);
+                    if (in) cnt = sg.cnt[sg.ptr[cc] + ii + (int64_t)m * (jj + (int64_t)m * kk)];
+                }
+                const int ts = (int)read_lane((uint32_t)wave_incl_sum(cnt), 63);
+                if ((float)(4 * ts) >= lam)
+                    r2 = knn_guess_r2<DIM>(p, N * m, ts, __popcll((unsigned long long)__ballot(in)), lam);
+            } else {
+                const uint64_t open = (uint64_t)__ballot(in && cnt <= SUB_MIN);
+                if (!(in && cnt <= SUB_MIN)) cnt = 0;
+                const int ts = (int)read_lane((uint32_t)wave_incl_sum(cnt), 63);
+                r2 = knn_guess_r2<DIM>(p, N, ts, __popcll((unsigned long long)open), lam);
+            }
+        }
     }
     if (!SUB && M <= 4) {
         if (knn_rows_query<DIM, M>(sorted, perm, N, cbase, starts, counts, q, k, o, smem.rows, p, P, r2, lam, kp, lo_d,
