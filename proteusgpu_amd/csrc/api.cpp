@@ -1412,7 +1412,7 @@ void sim_rebuild(pg_ctx* c, pg_sim* S, Marks* mk) {
     S->mesh.finalized = false;
     mesh_finalize(c, &S->mesh);
     pg_mesh& m = S->mesh;
-    pg::launch_face_twins(nullptr, m.n_seeds, m.n_seeds, m.hcode.as<int32_t>(), m.count.as<uint8_t>(),
+    pg::launch_face_twins(S->prm.mesh.dim, nullptr, m.n_seeds, m.n_seeds, m.hcode.as<int32_t>(), m.count.as<uint8_t>(),
                           m.nbr_cm.as<int32_t>(), m.twin.get<uint8_t>((size_t)m.n_seeds * MAXP),
                           m.solve.get<uint64_t>((size_t)m.n_seeds), c->stream);
     pg::launch_keep_kcert(nullptr, S->mesh.n_seeds, S->mesh.g.perm.as<uint32_t>(), nullptr,
@@ -2053,7 +2053,7 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
     pg::launch_bfinalize(n_dev, cap, cap, B->perm.as<uint32_t>(), B->orig_h.as<int32_t>(), B->count.as<uint8_t>(),
                          B->nbr.as<int32_t>(), B->vol.as<double>(), vs, B->periodic ? 1 : 0, B->vol_u.as<double>(),
                          B->o2s.as<int32_t>(), B->hcode.as<int32_t>(), B->st() + 1, s);
-    pg::launch_face_twins(n_dev, cap, cap, B->hcode.as<int32_t>(), B->count.as<uint8_t>(), B->nbr_cm.as<int32_t>(),
+    pg::launch_face_twins(dim, n_dev, cap, cap, B->hcode.as<int32_t>(), B->count.as<uint8_t>(), B->nbr_cm.as<int32_t>(),
                           B->twin.as<uint8_t>(), B->solve.as<uint64_t>(), s);
     pg::launch_bcount_failed(n_dev, cap, B->status.as<int32_t>(), B->st() + 3, s);
     if (B->km && lk_order_on())

@@ -44,8 +44,8 @@ void launch_face_total(int64_t n, const uint8_t* count, int32_t* total, hipStrea
 // *n_dev when n_dev is set (batches: n is then the capacity).
 // nbr_cm: cell-major neighbour lists (FACE_SLOTS per cell, from the clip
 // kernel); solve: per cell, the mask of the faces it solves.
-void launch_face_twins(const int64_t* n_dev, int64_t n, int64_t stride, const int32_t* hcode, const uint8_t* count,
-                       const int32_t* nbr_cm, uint8_t* twin, uint64_t* solve, hipStream_t s);
+void launch_face_twins(int dim, const int64_t* n_dev, int64_t n, int64_t stride, const int32_t* hcode,
+                       const uint8_t* count, const int32_t* nbr_cm, uint8_t* twin, uint64_t* solve, hipStream_t s);
 struct OwnedUpdate {
     const int64_t* n_dev = nullptr;
     int64_t n = 0, stride = 0, nplane = 0;

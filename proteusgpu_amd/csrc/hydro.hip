@@ -292,6 +292,79 @@ __global__ void __launch_bounds__(TB) k_face_twins(const int64_t* n_dev, int64_t
     }
 }
 
+// The same by L lanes per cell, one face each, for meshes whose cells alone
+// do not fill the chip: there the searches of a cell, one after the other,
+// are a chain of reads.  The faces that need a search (half of them) are
+// gathered per wave, and four lanes search one list, 16 entries (a 64-byte
+// line) per step, 16 lists in flight.  The codes go through LDS, so that a
+// row of a slot plane is written by consecutive lanes.
+template <int L>
+__global__ void __launch_bounds__(TB) k_face_twins_wide(const int64_t* n_dev, int64_t n_host, int64_t stride,
+                                                        const int32_t* __restrict__ hcode,
+                                                        const uint8_t* __restrict__ count,
+                                                        const int32_t* __restrict__ nbr_cm, uint8_t* __restrict__ twin,
+                                                        uint64_t* __restrict__ solve) {
+    constexpr int CELLS = TB / L;
+    __shared__ uint8_t tw[L][CELLS];
+    __shared__ int2 find[TB];  // per wave: (owner, thread) of the faces to search
+    __shared__ int32_t cmax;
+    const int64_t n = seed_count(n_dev, n_host);
+    // a device-side count may end below the capacity that the grid covers
+    const int64_t nb = (n + CELLS - 1) / CELLS;
+    if ((int64_t)blockIdx.x >= nb) return;  // whole block
+    const int64_t s0 = xcd_block(blockIdx.x, nb) * CELLS;
+    const int cell = threadIdx.x / L, l = threadIdx.x % L;
+    const int lane = threadIdx.x & 63, wbase = threadIdx.x & ~63;
+    const int64_t s = s0 + cell;
+    const int c = s < n && hcode[s] >= 0 ? count[s] : 0;
+    if (threadIdx.x == 0) cmax = 0;
+    __syncthreads();
+    if (l == 0 && c > 0) atomicMax(&cmax, c);
+    __syncthreads();
+    const int cm = cmax;
+    const int shift = lane / L * L;  // the cell's lanes of the wave
+    // the cell whose code this thread writes, and its face count
+    const int wcell = threadIdx.x % CELLS, wl = threadIdx.x / CELLS;
+    const int64_t ws = s0 + wcell;
+    const int wc = ws < n && hcode[ws] >= 0 ? count[ws] : 0;
+    uint64_t mask = 0;
+    for (int f0 = 0; f0 < cm; f0 += L) {
+        const int f = f0 + l;
+        tw[l][cell] = SOLVE;
+        int32_t t = -1;
+        if (f < c) t = nbr_cm[s * FACE_SLOTS + f];
+        const bool need = t >= 0 && t < s && hcode[t] >= 0;
+        const uint64_t m = (uint64_t)__ballot(need);
+        if (need) find[wbase + __popcll(m & ((1ull << lane) - 1ull))] = make_int2(t, (int)threadIdx.x);
+        __syncthreads();
+        const int nf = __popcll(m);
+        for (int r = lane >> 2; r < nf; r += 16) {
+            const int2 q = find[wbase + r];
+            const int32_t sq = (int32_t)(s0 + q.y / L);
+            const int ct = count[q.x];
+            const int4* lt = reinterpret_cast<const int4*>(nbr_cm + (int64_t)q.x * FACE_SLOTS);
+            int code = SOLVE;
+            for (int g = 4 * (lane & 3); g < ct; g += 16) {
+                const int4 v = lt[g >> 2];  // entries past ct hold anything
+                if (v.w == sq && g + 3 < ct) code = g + 3;
+                if (v.z == sq && g + 2 < ct) code = g + 2;
+                if (v.y == sq && g + 1 < ct) code = g + 1;
+                if (v.x == sq) code = g;
+                if (code != SOLVE) break;
+            }
+            code = min(code, __shfl_xor(code, 1, 64));
+            code = min(code, __shfl_xor(code, 2, 64));
+            if ((lane & 3) == 0) tw[q.y % L][q.y / L] = (uint8_t)code;
+        }
+        __syncthreads();
+        const uint64_t b = ((uint64_t)__ballot(f < c && tw[l][cell] == SOLVE) >> shift) & ((1ull << L) - 1ull);
+        mask |= b << f0;
+        if (f0 + wl < wc) twin[(int64_t)(f0 + wl) * stride + ws] = tw[wl][wcell];
+        __syncthreads();
+    }
+    if (l == 0 && s < n && hcode[s] >= 0) solve[s] = mask;
+}
+
 template <int DIM>
 __global__ void __launch_bounds__(TB) k_cell_records(const int64_t* n_dev, int64_t n_host,
                                                      const int32_t* __restrict__ hcode, SimView sv,
@@ -391,9 +464,13 @@ __global__ void __launch_bounds__(TB)
         dt0 = *dt_dev;
         if (dt_max > 0 && dt0 > dt_max) dt0 = dt_max;
     }
-    for (int64_t s = (int64_t)blockIdx.x * TB + threadIdx.x; s < n; s += (int64_t)gridDim.x * TB) {
+    // blocks by XCD share: the twins' fluxes of neighbouring cells meet in one
+    // L2 (64 2D boxes 214 -> 155 us; 3D 1M cells 338 us either way)
+    const int64_t nb = (n + TB - 1) / TB;
+    if ((int64_t)blockIdx.x >= nb) return;
+    const int64_t s = xcd_block(blockIdx.x, nb) * TB + threadIdx.x;
+    if (s < n && hcode[s] >= 0) {
         const int32_t i = hcode[s];
-        if (i < 0) continue;
         const double dt = dt_box ? dt_box[hbox[i]] : dt0;
         double q[DIM + 2];
 #pragma unroll
@@ -401,11 +478,12 @@ __global__ void __launch_bounds__(TB)
         const int c = count[s];
         // four faces' records are loaded together (independent loads in
         // flight), then added in face order
-        for (int f0 = 0; f0 < c; f0 += 4) {
-            double v[4][DIM + 2];
-            bool own[4];
+        constexpr int FB = 4;
+        for (int f0 = 0; f0 < c; f0 += FB) {
+            double v[FB][DIM + 2];
+            bool own[FB];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
+            for (int e = 0; e < FB; e++) {
                 own[e] = true;
 #pragma unroll
                 for (int k = 0; k < DIM + 2; k++) v[e][k] = 0.0;
@@ -418,7 +496,7 @@ __global__ void __launch_bounds__(TB)
                 for (int k = 0; k < DIM + 2; k++) v[e][k] = fo[k];
             }
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
+            for (int e = 0; e < FB; e++) {
                 if (f0 + e >= c) break;
 #pragma unroll
                 for (int k = 0; k < DIM + 2; k++) {
@@ -659,37 +737,40 @@ void launch_prim_from_q(int dim, SimView sv, const int32_t* o2s, const double* v
     else k_prim_from_q<3><<<nblk(sv.n_hydro), TB, 0, s>>>(sv, o2s, vol_u, dt_init);
 }
 
-// grid: every seed once (host count), or a capped grid-stride grid over
-// the capacity (device count)
-static unsigned own_blocks(const int64_t* n_dev, int64_t n) {
-    return n_dev ? std::min<unsigned>(nblk(n), 4096) : nblk(n);
+void launch_face_twins(int dim, const int64_t* n_dev, int64_t n, int64_t stride, const int32_t* hcode,
+                       const uint8_t* count, const int32_t* nbr_cm, uint8_t* twin, uint64_t* solve, hipStream_t s) {
+    if (n <= 0) return;
+    // 2D 2k cells 11.7 (a thread per cell) and 5.8 us (8 lanes), 3D 20k cells
+    // 37 and 9.6 us (16 lanes); 3D 1M cells 255 and 264 us, 2M cells 480 and
+    // 498 us: both grow by about 0.25 us per 1k cells from the thread's 40 us
+    // latency on
+    constexpr int64_t WIDE_CELLS = 131072;
+    if (n > WIDE_CELLS)
+        k_face_twins<<<n_dev ? std::min<unsigned>(nblk(n), 4096) : nblk(n), TB, 0, s>>>(n_dev, n, stride, hcode, count,
+                                                                                        nbr_cm, twin, solve);
+    else if (dim == 2)
+        k_face_twins_wide<8><<<(unsigned)((n + 31) / 32), TB, 0, s>>>(n_dev, n, stride, hcode, count, nbr_cm, twin, solve);
+    else
+        k_face_twins_wide<16><<<(unsigned)((n + 15) / 16), TB, 0, s>>>(n_dev, n, stride, hcode, count, nbr_cm, twin, solve);
 }
 
-void launch_face_twins(const int64_t* n_dev, int64_t n, int64_t stride, const int32_t* hcode, const uint8_t* count,
-                       const int32_t* nbr_cm, uint8_t* twin, uint64_t* solve, hipStream_t s) {
-    if (n <= 0) return;
-    k_face_twins<<<own_blocks(n_dev, n), TB, 0, s>>>(n_dev, n, stride, hcode, count, nbr_cm, twin, solve);
+// grid: every seed once (host count), or a capped grid-stride grid over
+// the capacity (device count)
+template <int DIM>
+void hll_owned(const OwnedUpdate& u, hipStream_t s) {
+    const unsigned gb = u.n_dev ? std::min<unsigned>(nblk(u.n), 4096) : nblk(u.n);
+    k_cell_records<DIM><<<gb, TB, 0, s>>>(u.n_dev, u.n, u.hcode, u.sv, u.wgen, u.rec);
+    k_face_flux<DIM><<<dim3(gb, FR), TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.solve, u.nbr, u.nrm,
+                                                 u.area, u.ascale, u.cen, u.sorted, u.scale, u.gam, u.flux_mode, u.move,
+                                                 u.rec, u.fbuf);
+    k_face_sum<DIM><<<nblk(u.n), TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.count, u.twin, u.nbr, u.fbuf,
+                                      u.dt_dev, u.dt_max, u.dt_box, u.hbox, u.sv);
 }
 
 void launch_hll_owned(int dim, OwnedUpdate u, hipStream_t s) {
     if (u.n <= 0) return;
-    const unsigned gb = own_blocks(u.n_dev, u.n);
-    const dim3 gf(gb, FR);
-    if (dim == 2) {
-        k_cell_records<2><<<gb, TB, 0, s>>>(u.n_dev, u.n, u.hcode, u.sv, u.wgen, u.rec);
-        k_face_flux<2><<<gf, TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.solve, u.nbr, u.nrm,
-                                         u.area, u.ascale, u.cen, u.sorted, u.scale, u.gam, u.flux_mode, u.move, u.rec,
-                                         u.fbuf);
-        k_face_sum<2><<<gb, TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.count, u.twin, u.nbr, u.fbuf,
-                                        u.dt_dev, u.dt_max, u.dt_box, u.hbox, u.sv);
-    } else {
-        k_cell_records<3><<<gb, TB, 0, s>>>(u.n_dev, u.n, u.hcode, u.sv, u.wgen, u.rec);
-        k_face_flux<3><<<gf, TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.solve, u.nbr, u.nrm,
-                                         u.area, u.ascale, u.cen, u.sorted, u.scale, u.gam, u.flux_mode, u.move, u.rec,
-                                         u.fbuf);
-        k_face_sum<3><<<gb, TB, 0, s>>>(u.n_dev, u.n, u.stride, u.nplane, u.hcode, u.count, u.twin, u.nbr, u.fbuf,
-                                        u.dt_dev, u.dt_max, u.dt_box, u.hbox, u.sv);
-    }
+    if (dim == 2) hll_owned<2>(u, s);
+    else hll_owned<3>(u, s);
 }
 
 void launch_hll_faces(int dim, int64_t n, double gam, const double* L, const double* R, const double* nrm,
