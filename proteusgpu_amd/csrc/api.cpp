@@ -1966,14 +1966,16 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
                      B->coff.as<int64_t>(), B->cell.as<int32_t>(), B->counts.as<int32_t>(), B->starts.as<int32_t>(),
                      B->fill.as<int32_t>(), B->tmp.as<int32_t>(), B->total.as<int32_t>(), B->perm.as<uint32_t>(),
                      B->sorted.as<double>(), B->sorted_box.as<int32_t>(), B->big.as<int32_t>(), s);
-    auto knn = [&](const uint32_t* q, const int64_t* nq, int k, bool big) {
+    // all seeds: one block per query; the lists of a bucket or a restart, which
+    // may hold any share of the seeds: persistent blocks
+    auto knn = [&](const uint32_t* q, const int64_t* nq, int k, bool big, bool loop) {
         pg::KnnTail tail;  // seeds that resume need only the rest of their row
         if (B->resume.p && !big)
             tail = {B->resume.as<int32_t>(), B->lastnb.as<uint32_t>(), clip_shape_tag(dim, B->lanes, B->slots)};
         pg::launch_bknn(dim, B->sorted.as<double>(), B->perm.as<uint32_t>(), B->sorted_box.as<int32_t>(),
                         B->N.as<int32_t>(), B->coff.as<int64_t>(), B->starts.as<int32_t>(), B->counts.as<int32_t>(),
                         q, nq, cap, k, B->knn.as<uint32_t>(), B->wave_min_k, B->bpc,
-                        B->ticket.as<unsigned long long>(), s, tail);
+                        B->ticket.as<unsigned long long>(), loop, s, tail);
     };
     // first pass and learned buckets: one block per seed group (the clip
     // spills in a persistent loop); the short restart lists: persistent blocks
@@ -1991,7 +1993,7 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
     const std::vector<int>& sched = B->km ? B->ksched_learned : B->ksched;
     int k = sched[0];
     if (!B->km) {
-        knn(nullptr, n_dev, k, false);
+        knn(nullptr, n_dev, k, false, false);
         clip(nullptr, n_dev, k, 0, false);
     } else {
         float* feat = B->feat.as<float>();
@@ -2012,7 +2014,7 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
                            B->total.as<int32_t>(), cap, B->klists.as<uint32_t>(), B->kcnt.as<int64_t>(), s, order);
         for (int c = 0; c < pg::LK_NCLASS; c++) {
             const uint32_t* lc = B->klists.as<uint32_t>() + (size_t)c * cap;
-            knn(lc, B->kcnt.as<int64_t>() + c, pg::lk_bucket(c), false);
+            knn(lc, B->kcnt.as<int64_t>() + c, pg::lk_bucket(c), false, true);
             clip(lc, B->kcnt.as<int64_t>() + c, pg::lk_bucket(c), 0, false);
         }
     }
@@ -2028,7 +2030,7 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
     bool big_done = false;
     auto big_pass = [&](int kk) {
         collect(nullptr, n_dev, pg::SLOT_OVERFLOW, lst[2], cnt[2]);
-        knn(lst[2], cnt[2], kk, true);
+        knn(lst[2], cnt[2], kk, true, true);
         clip(lst[2], cnt[2], kk, 1, true);
         L = nullptr;
         nL = n_dev;
@@ -2041,7 +2043,7 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
         const int d = (L == lst[0]) ? 1 : 0;
         collect(L, nL, PG_SECURITY_RADIUS_NOT_REACHED, lst[d], cnt[d]);
         k = sched[r];
-        knn(lst[d], cnt[d], k, false);
+        knn(lst[d], cnt[d], k, false, true);
         clip(lst[d], cnt[d], k, 0, true);
         L = lst[d];
         nL = cnt[d];

@@ -250,6 +250,36 @@ struct BKnnArgs {
     int k;
 };
 
+// One query by its wave: the qi-th of the list.
+template <int DIM, int M, class Args>
+PG_DEV void bknn_query(const Args* A, int64_t qi, KnnSmem<M>& smem) {
+    const uint32_t q = A->queries ? A->queries[qi] : (uint32_t)qi;
+    const int b = A->sbox[q];
+    const int k = A->k;
+    KnnTail tail;
+    tail.resume = A->tail.resume;
+    tail.lastnb = A->tail.lastnb;
+    tail.tag = A->tail.tag;
+    int kp = 0;
+    uint32_t lo = 0;
+    tail_of(tail, q, k, kp, lo);
+    knn_wave_query<DIM, M>(A->sorted, A->perm, A->N[b], A->coff[b], A->starts, A->counts, q, k,
+                           A->out + (size_t)qi * k, smem, kp, lo);
+}
+
+// Lists that fill their capacity: one block per query over the capacity, as
+// in k_bvoronoi.  Without the item loop the kernel takes 57 registers for 79 (7
+// waves per SIMD for 6): the k = 32 rows of 2M seeds 2.99 -> 2.45 ms.  For the
+// buckets of learned rows, which fill a part of it, the empty blocks eat that
+// gain (six buckets of 1M seeds 3.0 and 3.0 ms): they keep the loop.
+template <int DIM, int M>
+__global__ void __launch_bounds__(64, (M <= 2 ? 6 : 5)) k_bknn_list(BKnnArgs args) {
+    __shared__ KnnSmem<M> smem;
+    const int64_t nq = *args.nq_dev;
+    if (blockIdx.x >= nq) return;  // whole block
+    bknn_query<DIM, M>(&args, xcd_block(blockIdx.x, nq), smem);
+}
+
 template <int DIM, int M>
 __global__ void __launch_bounds__(64, (M <= 2 ? 6 : 5)) k_bknn_wave(BKnnArgs args) {
     __shared__ KnnSmem<M> smem;
@@ -261,19 +291,7 @@ __global__ void __launch_bounds__(64, (M <= 2 ? 6 : 5)) k_bknn_wave(BKnnArgs arg
         if (q0 >= nq) break;
         const int64_t q1 = q0 + chunk < nq ? q0 + chunk : nq;
         for (int64_t qi = q0; qi < q1; qi++) {
-            const auto* A = fresh_args<BKnnArgs>();
-            const uint32_t q = A->queries ? A->queries[qi] : (uint32_t)qi;
-            const int b = A->sbox[q];
-            const int k = A->k;
-            KnnTail tail;
-            tail.resume = A->tail.resume;
-            tail.lastnb = A->tail.lastnb;
-            tail.tag = A->tail.tag;
-            int kp = 0;
-            uint32_t lo = 0;
-            tail_of(tail, q, k, kp, lo);
-            knn_wave_query<DIM, M>(A->sorted, A->perm, A->N[b], A->coff[b], A->starts, A->counts, q, k,
-                                   A->out + (size_t)qi * k, smem, kp, lo);
+            bknn_query<DIM, M>(fresh_args<BKnnArgs>(), qi, smem);
             __syncthreads();
         }
     }
@@ -512,7 +530,12 @@ template <int DIM, int M>
 void bknn_wave(const double* sorted, const uint32_t* perm, const int32_t* sbox, const int32_t* N,
                const int64_t* coff, const int32_t* starts, const int32_t* counts, const uint32_t* q,
                const int64_t* nq_dev, int64_t cap, int k, uint32_t* out, int blocks_per_cu,
-               unsigned long long* ticket, hipStream_t s, KnnTail tail) {
+               unsigned long long* ticket, bool loop, hipStream_t s, KnnTail tail) {
+    if (!loop) {
+        const BKnnArgs args{sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, out, ticket, tail, k};
+        k_bknn_list<DIM, M><<<(unsigned)std::max<int64_t>(cap, 1), 64, 0, s>>>(args);
+        return;
+    }
     static const int occ = occupancy(k_bknn_wave<DIM, M>);
     const unsigned nb = (unsigned)std::min<int64_t>(cap, resident_blocks(occ, 8 * blocks_per_cu));
     k_fill<unsigned long long><<<1, TB, 0, s>>>(ticket, 1, 0ull);
@@ -523,12 +546,12 @@ template <int DIM>
 void bknn_dim(const double* sorted, const uint32_t* perm, const int32_t* sbox, const int32_t* N,
               const int64_t* coff, const int32_t* starts, const int32_t* counts, const uint32_t* q,
               const int64_t* nq_dev, int64_t cap, int k, uint32_t* out, int wave_min_k, int blocks_per_cu,
-              unsigned long long* ticket, hipStream_t s, KnnTail tail) {
+              unsigned long long* ticket, bool loop, hipStream_t s, KnnTail tail) {
     if (k >= wave_min_k || knn_wave_faster(DIM, cap, k)) {
-        if (k <= 64) bknn_wave<DIM, 1>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, s, tail);
-        else if (k <= 128) bknn_wave<DIM, 2>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, s, tail);
-        else if (k <= 192) bknn_wave<DIM, 3>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, s, tail);
-        else bknn_wave<DIM, 4>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, s, tail);
+        if (k <= 64) bknn_wave<DIM, 1>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, loop, s, tail);
+        else if (k <= 128) bknn_wave<DIM, 2>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, loop, s, tail);
+        else if (k <= 192) bknn_wave<DIM, 3>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, loop, s, tail);
+        else bknn_wave<DIM, 4>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, loop, s, tail);
     } else if (k <= 208) {
         bknn_heap<DIM, 64>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, s);
     } else {
@@ -557,13 +580,13 @@ void bclip(const double* pts, const uint32_t* seeds, const int64_t* nq_dev, int6
 void launch_bknn(int dim, const double* sorted, const uint32_t* perm, const int32_t* sbox, const int32_t* N,
                  const int64_t* coff, const int32_t* starts, const int32_t* counts, const uint32_t* queries,
                  const int64_t* nq_dev, int64_t cap, int k, uint32_t* out, int wave_min_k, int blocks_per_cu,
-                 unsigned long long* ticket, hipStream_t s, KnnTail tail) {
+                 unsigned long long* ticket, bool loop, hipStream_t s, KnnTail tail) {
     if (dim == 2)
         bknn_dim<2>(sorted, perm, sbox, N, coff, starts, counts, queries, nq_dev, cap, k, out, wave_min_k,
-                    blocks_per_cu, ticket, s, tail);
+                    blocks_per_cu, ticket, loop, s, tail);
     else
         bknn_dim<3>(sorted, perm, sbox, N, coff, starts, counts, queries, nq_dev, cap, k, out, wave_min_k,
-                    blocks_per_cu, ticket, s, tail);
+                    blocks_per_cu, ticket, loop, s, tail);
 }
 
 void launch_bvoronoi(int dim, const double* sorted, const uint32_t* seeds, const int64_t* nq_dev, int64_t cap,

@@ -256,14 +256,14 @@ void launch_bgrid(int dim, const double* pts, const int64_t* n_dev, int64_t cap,
                   const int32_t* sbox, const int32_t* N, const int64_t* coff, int32_t* cell, int32_t* counts,
                   int32_t* starts, int32_t* fill, int32_t* tmp, int32_t* total, uint32_t* perm, double* sorted,
                   int32_t* sorted_box, int32_t* big, hipStream_t s);
-void launch_bknn(int dim, const double* sorted, const uint32_t* perm, const int32_t* sbox, const int32_t* N,
-                 const int64_t* coff, const int32_t* starts, const int32_t* counts, const uint32_t* queries,
-                 const int64_t* nq_dev, int64_t cap, int k, uint32_t* out, int wave_min_k, int blocks_per_cu,
-                 unsigned long long* ticket, hipStream_t s, KnnTail tail = {});
 // ticket: a device counter, the work queue of the persistent kernels
 // (cleared by the launcher, in stream order)
 // loop: persistent blocks over the list (short lists); else one block per
-// group of seeds over the capacity (lists that fill most of it)
+// query or group of seeds over the capacity (lists that fill most of it)
+void launch_bknn(int dim, const double* sorted, const uint32_t* perm, const int32_t* sbox, const int32_t* N,
+                 const int64_t* coff, const int32_t* starts, const int32_t* counts, const uint32_t* queries,
+                 const int64_t* nq_dev, int64_t cap, int k, uint32_t* out, int wave_min_k, int blocks_per_cu,
+                 unsigned long long* ticket, bool loop, hipStream_t s, KnnTail tail = {});
 void launch_bvoronoi(int dim, const double* sorted, const uint32_t* seeds, const int64_t* nq_dev, int64_t cap,
                      const uint32_t* knn, int k, int max_p, int max_t, int big, int lanes, int slots, FaceArrays fa,
                      int blocks_per_cu, unsigned long long* ticket, bool loop, hipStream_t s);
