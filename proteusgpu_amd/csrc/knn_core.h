@@ -322,19 +322,21 @@ PG_DEV void tail_of(const KnnTail& t, uint32_t q, int k, int& kp, uint32_t& lo) 
 // rows do not depend on it, only the work to find them.
 template <int DIM>
 PG_DEV double knn_guess_r2(const double (&p)[3], int N, int cnt, int nin, float lam) {
-    // float arithmetic and the hardware's log2 / exp2: a heuristic needs
-    // no more
-    const float h = 1.0f / (float)N;
+    // float arithmetic and the hardware's log2, exp2 and reciprocal: a
+    // heuristic needs no more (with IEEE divisions 60 instructions more per
+    // query, 8% of all)
+    const float h = __builtin_amdgcn_rcpf((float)N);
     const float vcell = DIM == 3 ? h * h * h : h * h;
-    const float rho = (float)max(cnt - 1, 1) / ((float)max(nin, 1) * vcell);
     // ball volume lam / rho = (4 pi / 3) R^3 in 3D, pi R^2 in 2D
-    const float v = lam / rho * (DIM == 3 ? 0.2387324146f : 0.3183098862f);
+    const float v = lam * (float)max(nin, 1) * vcell * __builtin_amdgcn_rcpf((float)max(cnt - 1, 1)) *
+                    (DIM == 3 ? 0.2387324146f : 0.3183098862f);
     float R = __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(v) * (1.0f / DIM));
+    const float half_R = 0.5f * __builtin_amdgcn_rcpf(R);
     float f = 1.0f;
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
         const float x = (float)p[d];
-        f *= (fminf(x, R) + fminf(1.0f - x, R)) / (2.0f * R);
+        f *= (fminf(x, R) + fminf(1.0f - x, R)) * half_R;
     }
     f = fmaxf(f, 1.0f / 64.0f);
     R *= __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(f) * (-1.0f / DIM));
@@ -407,9 +409,9 @@ PG_DEV void key_merge_batch(uint32_t (&kk)[M], uint32_t& out, uint32_t a, int l,
 // skip only points outside the ball (the float bounds carry a slack of
 // several float roundings of N), so every point of the ball is seen.
 //
-// What bounds it: VALU issue (710 instructions per query, k = 32 and its 64
+// What bounds it: VALU issue (640 instructions per query, k = 32 and its 64
 // tails; the ring walk with FP64 sorts took 1.75k).  1M uniform 3D queries:
-// k = 32 2.4 -> 1.06 ms, k = 64 3.25 -> 1.39 ms.  One run of points per row
+// k = 32 2.4 -> 0.96 ms, k = 64 3.25 -> 1.27 ms.  One run of points per row
 // of cells replaces 27 and then 98 cells looked at one by one, the mark scan a
 // binary search per candidate, and an exchange of the sort takes three
 // integer instructions instead of a dozen.
@@ -492,12 +494,12 @@ PG_DEV bool knn_rows_query(const double* __restrict__ sorted, const uint32_t* __
                 }
                 if (__ballot(near) != 0ull) {
                     if (near) {
-                        double pc[3] = {0, 0, 0};
+                        int ring = 0;
 #pragma unroll
-                        for (int e = 0; e < DIM; e++) pc[e] = sorted[(size_t)DIM * cs + e];
-                        const int a = grid_cell<DIM>(p, N), b = grid_cell<DIM>(pc, N);
-                        int ring = max(abs(a % N - b % N), abs((a / N) % N - (b / N) % N));
-                        if (DIM == 3) ring = max(ring, abs(a / (N * N) - b / (N * N)));
+                        for (int e = 0; e < DIM; e++) {  // grid_cell of both, per axis
+                            const int a = (int)floor(P[e]), b = (int)floor(sorted[(size_t)DIM * cs + e] * (double)N);
+                            ring = max(ring, abs(max(0, min(a, N - 1)) - max(0, min(b, N - 1))));
+                        }
                         const double md = (double)(ring - 1) / (double)N;
                         odd = odd || (ring >= 2 && d < md * md);
                     }
@@ -635,8 +637,9 @@ PG_DEV void knn_wave_query(const double* __restrict__ sorted, const uint32_t* __
     double P[3] = {0, 0, 0};
 #pragma unroll
     for (int d = 0; d < DIM; d++) P[d] = p[d] * (double)N;
-    const int c = grid_cell<DIM>(p, N);
-    const int ci = c % N, cj = (c / N) % N, ck = DIM == 3 ? c / (N * N) : 0;
+    // the query's cell (grid_cell), per axis
+    const int ci = max(0, min((int)floor(P[0]), N - 1)), cj = max(0, min((int)floor(P[1]), N - 1));
+    const int ck = DIM == 3 ? max(0, min((int)floor(P[2]), N - 1)) : 0;
 
     double kd[M];
     uint32_t ks[M];
@@ -697,7 +700,7 @@ PG_DEV void knn_wave_query(const double* __restrict__ sorted, const uint32_t* __
             // with known neighbours takes their density, one in a crowded
             // cell that of the sub-cells around it (unless they hold too few
             // points to tell), another that of the cells that are not crowded
-            const int64_t cc = cbase + c;
+            const int64_t cc = cbase + ci + cj * N + (int64_t)ck * N * N;
             const int m = sg.m[cc];
             if (kp > 0) {
                 if (lo_d > 0.0)
