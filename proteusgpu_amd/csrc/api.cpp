@@ -1366,8 +1366,10 @@ int pg_dt_cfl(pg_ctx* c, const pg_mesh* mc, const pg_state* st, double gamma, do
         argchk(st->n == m->n_hydro && st->dim == m->prm.dim, "state does not match mesh");
         mesh_finalize(c, m);
         unsigned long long* d = const_cast<pg_state*>(st)->dt.get<unsigned long long>(1);
-        double init = 1e100;  // finite_volume_solver.cpp:153
-        HIPCHK(hipMemcpyAsync(d, &init, sizeof(double), hipMemcpyHostToDevice, c->stream));
+        const double init = 1e100;  // finite_volume_solver.cpp:153
+        unsigned long long bits;
+        std::memcpy(&bits, &init, sizeof(bits));
+        pg::launch_fill_u64(d, 1, bits, c->stream);
         const int b = st->cur;
         pg::launch_dt_cfl(st->dim, st->n, m->o2s.as<int32_t>(), m->vol_u.as<double>(), gamma, cfl,
                           st->rho[b].as<double>(), st->vel[b].as<double>(), st->E[b].as<double>(), d,

@@ -86,8 +86,13 @@ struct KnnTail {
 // (2D k = 16: 170 us for 2,000 to 100,000 queries, wave 17 to 99 us) that full
 // launches of short rows hide: at 1.4M queries 2D k = 16 1150 us (wave 1138),
 // k = 12 769 (1081), k = 8 447 (1050); 3D k = 16 2481 (1442), k = 12 1637
-// (1369), k = 8 1095 (1348).
-inline bool knn_wave_faster(int dim, int64_t nq, int k) { return k >= (dim == 2 ? 16 : 12) || nq <= 400000; }
+// (1369), k = 8 1095 (1348).  Between, the heap's chain grows with k: whole
+// calls of 2D k = 8 take 180 (wave 122) us at 100,000 queries, 210 (269) at
+// 300,000; k = 16 412 (282); 3D k = 8 380 (329).
+inline bool knn_wave_faster(int dim, int64_t nq, int k) {
+    if (dim == 2) return k >= 16 || nq <= 22000 * (int64_t)k;
+    return k >= 12 || nq <= 400000;
+}
 
 // k nearest neighbours of queries (sorted ids; nullptr = all n points).
 // Rows ascending by (FP64 dist^2, original index); out row stride k.
