@@ -2075,10 +2075,13 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
                      B->fill.as<int32_t>(), B->tmp.as<int32_t>(), B->total.as<int32_t>(), B->perm.as<uint32_t>(),
                      B->sorted.as<double>(), B->sorted_box.as<int32_t>(), B->big.as<int32_t>(), s);
     // all seeds: one block per query; the lists of a bucket or a restart, which
-    // may hold any share of the seeds: persistent blocks
-    auto knn = [&](const uint32_t* q, const int64_t* nq, int k, bool big, bool loop) {
-        pg::KnnTail tail;  // seeds that resume need only the rest of their row
-        if (B->resume.p && !big)
+    // may hold any share of the seeds: persistent blocks.  Seeds that resume
+    // need only the rest of their row, but only a restart list may look at the
+    // resume entries: they are this rebuild's from the first clip on, and
+    // another rebuild's or whatever the memory held before it
+    auto knn = [&](const uint32_t* q, const int64_t* nq, int k, bool resumes, bool loop) {
+        pg::KnnTail tail;
+        if (B->resume.p && resumes)
             tail = {B->resume.as<int32_t>(), B->lastnb.as<uint32_t>(), clip_shape_tag(dim, B->lanes, B->slots)};
         pg::launch_bknn(dim, B->sorted.as<double>(), B->perm.as<uint32_t>(), B->sorted_box.as<int32_t>(),
                         B->N.as<int32_t>(), B->coff.as<int64_t>(), B->starts.as<int32_t>(), B->counts.as<int32_t>(),
@@ -2138,7 +2141,7 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
     bool big_done = false;
     auto big_pass = [&](int kk) {
         collect(nullptr, n_dev, pg::SLOT_OVERFLOW, lst[2], cnt[2]);
-        knn(lst[2], cnt[2], kk, true, true);
+        knn(lst[2], cnt[2], kk, false, true);
         clip(lst[2], cnt[2], kk, 1, true);
         L = nullptr;
         nL = n_dev;
@@ -2151,7 +2154,7 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
         const int d = (L == lst[0]) ? 1 : 0;
         collect(L, nL, PG_SECURITY_RADIUS_NOT_REACHED, lst[d], cnt[d]);
         k = sched[r];
-        knn(lst[d], cnt[d], k, false, true);
+        knn(lst[d], cnt[d], k, true, true);
         clip(lst[d], cnt[d], k, 0, true);
         L = lst[d];
         nL = cnt[d];
