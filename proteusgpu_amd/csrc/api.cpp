@@ -199,6 +199,7 @@ struct pg_ctx {
     hipStream_t stream = nullptr;
     void* scratch = nullptr;  // this GPU's static scratch array (allocation-free entry points)
     DBuf hll_io[5];  // pg_hll_flux staging (left, right, normal, wall, flux), grow-only
+    DBuf dt;         // CFL minimum of pg_dt_cfl (the state is const there)
 };
 
 namespace {
@@ -324,7 +325,6 @@ struct pg_mesh {
         pg::launch_fill_i32(b, 3, 0, s);
         return b;
     }
-    DBuf srec;  // static-mesh update: states by sorted seed
     // owner-computes-once update: hydro code per sorted seed, twin code per
     // face slot, and scratch for the sorted cell records and the per-slot
     // face fluxes
@@ -369,7 +369,10 @@ struct pg_kmodel {
 struct pg_state {
     int dim = 3;
     int64_t n = 0;
-    DBuf rho[2], vel[2], E[2], dt;
+    DBuf rho[2], vel[2], E[2];
+    // static-mesh update: this state by sorted seed (here and not in the mesh,
+    // which states of several threads may share)
+    DBuf rec;
     int cur = 0;
 };
 
@@ -1365,7 +1368,7 @@ int pg_dt_cfl(pg_ctx* c, const pg_mesh* mc, const pg_state* st, double gamma, do
         pg_mesh* m = const_cast<pg_mesh*>(mc);
         argchk(st->n == m->n_hydro && st->dim == m->prm.dim, "state does not match mesh");
         mesh_finalize(c, m);
-        unsigned long long* d = const_cast<pg_state*>(st)->dt.get<unsigned long long>(1);
+        unsigned long long* d = c->dt.get<unsigned long long>(1);
         const double init = 1e100;  // finite_volume_solver.cpp:153
         unsigned long long bits;
         std::memcpy(&bits, &init, sizeof(bits));
@@ -1394,7 +1397,7 @@ int pg_hydro_step(pg_ctx* c, const pg_mesh* mc, pg_state* st, double gamma, doub
                               m->count.as<uint8_t>(), m->nbr.as<int32_t>(), m->nrm.as<double>(), m->area.as<double>(),
                               st->dim == 2 ? sc : sc * sc, m->vol_u.as<double>(), gamma, dt, flux_mode,
                               st->rho[b].as<double>(), st->vel[b].as<double>(), st->E[b].as<double>(),
-                              m->srec.get<double>((size_t)m->n_seeds * pg::static_rec_doubles(st->dim)),
+                              st->rec.get<double>((size_t)m->n_seeds * pg::static_rec_doubles(st->dim)),
                               st->rho[nb].as<double>(), st->vel[nb].as<double>(), st->E[nb].as<double>(), c->stream);
         HIPCHK(hipGetLastError());
         st->cur = nb;
