@@ -395,8 +395,9 @@ int pg_mesh_compute_k(pg_ctx* ctx, const pg_mesh_params* params, const pg_kmodel
 typedef struct {
     int clip_lanes;      /* lanes per seed of the fast 3D clip kernel: 8 or 16         */
     int clip_slots;      /* vertex slots per seed of the fast 3D clip kernel: 48 or 64 */
-    int knn_wave_min_k;  /* rows at least this long always use the wave-per-query
-                          * KNN (shorter ones where it is the faster one)        */
+    int knn_wave_min_k;  /* rows at least this long use the wave-per-query KNN,
+                          * shorter ones the heap per thread; the default, 20,
+                          * leaves shorter rows to the kernel measured faster    */
     int blocks_per_cu;   /* resident blocks per CU of the persistent KNN and clip
                           * kernels (KNN, 2D clip, restart clips), at most their
                           * occupancy (default 64: all)                          */

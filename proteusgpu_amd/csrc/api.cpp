@@ -1993,7 +1993,7 @@ struct pg_batch {
     std::vector<int64_t> hoff_h;
     std::vector<int> ksched, ksched_learned;
     // tuning (timing only; results do not depend on it)
-    int lanes = 16, slots = 64, wave_min_k = 20, bpc = 64;
+    int lanes = 16, slots = 64, wave_min_k = pg::KNN_WAVE_MIN_K, bpc = 64;
     bool use_graph = true;
     const pg_kmodel* km = nullptr;  // learned k (nullptr: fixed k)
     // static

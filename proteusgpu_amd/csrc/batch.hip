@@ -547,7 +547,7 @@ void bknn_dim(const double* sorted, const uint32_t* perm, const int32_t* sbox, c
               const int64_t* coff, const int32_t* starts, const int32_t* counts, const uint32_t* q,
               const int64_t* nq_dev, int64_t cap, int k, uint32_t* out, int wave_min_k, int blocks_per_cu,
               unsigned long long* ticket, bool loop, hipStream_t s, KnnTail tail) {
-    if (k >= wave_min_k || knn_wave_faster(DIM, cap, k)) {
+    if (knn_by_wave(DIM, cap, k, wave_min_k)) {
         if (k <= 64) bknn_wave<DIM, 1>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, loop, s, tail);
         else if (k <= 128) bknn_wave<DIM, 2>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, loop, s, tail);
         else if (k <= 192) bknn_wave<DIM, 3>(sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, cap, k, out, blocks_per_cu, ticket, loop, s, tail);

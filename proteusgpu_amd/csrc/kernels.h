@@ -81,8 +81,11 @@ struct KnnTail {
     int32_t tag = 0;
 };
 
+// Rows of at least KNN_WAVE_MIN_K always go to the wave-per-query kernel.
+constexpr int KNN_WAVE_MIN_K = 20;
+
 // Whether the wave-per-query kernel beats the per-thread heap for nq queries
-// with rows of k < 20.  The heap is a chain of one thread's LDS updates
+// with rows of k < KNN_WAVE_MIN_K.  The heap is a chain of one thread's LDS updates
 // (2D k = 16: 170 us for 2,000 to 100,000 queries, wave 17 to 99 us) that full
 // launches of short rows hide: at 1.4M queries 2D k = 16 1150 us (wave 1138),
 // k = 12 769 (1081), k = 8 447 (1050); 3D k = 16 2481 (1442), k = 12 1637
@@ -92,6 +95,12 @@ struct KnnTail {
 inline bool knn_wave_faster(int dim, int64_t nq, int k) {
     if (dim == 2) return k >= 16 || nq <= 22000 * (int64_t)k;
     return k >= 12 || nq <= 400000;
+}
+
+// The choice for wave_min_k as set: the default leaves shorter rows to the
+// measured rule, a program's own value draws the line there and nowhere else.
+inline bool knn_by_wave(int dim, int64_t nq, int k, int wave_min_k) {
+    return k >= wave_min_k || (wave_min_k == KNN_WAVE_MIN_K && knn_wave_faster(dim, nq, k));
 }
 
 // k nearest neighbours of queries (sorted ids; nullptr = all n points).

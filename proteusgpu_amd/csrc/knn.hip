@@ -63,15 +63,15 @@ void launch_knn(int dim, const double* sorted, const uint32_t* perm, int64_t n, 
                 int k, uint32_t* out, hipStream_t s, KnnTail tail, SubGrid sg) {
     (void)n;
     if (nq <= 0) return;
-    // Long rows and short query lists go to the wave-per-query kernel; the row
-    // length can be moved with PGPU_KNN_WAVE_MIN_K for tuning runs.
+    // Long rows and short query lists go to the wave-per-query kernel; a row
+    // length in PGPU_KNN_WAVE_MIN_K takes the rule's place for tuning runs.
     static const int wave_min_k = [] {
         const char* e = getenv("PGPU_KNN_WAVE_MIN_K");
-        return e ? atoi(e) : 20;
+        return e ? atoi(e) : KNN_WAVE_MIN_K;
     }();
     // the LDS heap holds at most 256 entries per query, and only the wave
     // kernel takes crowded cells through their sub-grids
-    if (k >= wave_min_k || k > 256 || sg.m != nullptr || knn_wave_faster(dim, nq, k)) {
+    if (k > 256 || sg.m != nullptr || knn_by_wave(dim, nq, k, wave_min_k)) {
         if (dim == 2) dispatch_wave<2>(sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
         else dispatch_wave<3>(sorted, perm, N, starts, counts, queries, nq, k, out, tail, sg, s);
         return;
