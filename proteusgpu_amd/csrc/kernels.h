@@ -91,10 +91,12 @@ constexpr int KNN_WAVE_MIN_K = 20;
 // k = 12 769 (1081), k = 8 447 (1050); 3D k = 16 2481 (1442), k = 12 1637
 // (1369), k = 8 1095 (1348).  Between, the heap's chain grows with k: whole
 // calls of 2D k = 8 take 180 (wave 122) us at 100,000 queries, 210 (269) at
-// 300,000; k = 16 412 (282); 3D k = 8 380 (329).
+// 300,000; k = 16 412 (282); 3D k = 8 436 (327) at 400,000, k = 5 337 (310),
+// k = 4 175 (170) at 200,000 and 201 (238) at 300,000, k = 1 78 (52) at 50,000,
+// 82 (88) at 100,000 and 124 (235) at 300,000.
 inline bool knn_wave_faster(int dim, int64_t nq, int k) {
     if (dim == 2) return k >= 16 || nq <= 22000 * (int64_t)k;
-    return k >= 12 || nq <= 400000;
+    return k >= 12 || nq <= (k >= 5 ? 400000 : 50000 * (int64_t)k);
 }
 
 // The choice for wave_min_k as set: the default leaves shorter rows to the

@@ -32,6 +32,16 @@ def by_wave(tmp_path_factory):
     return ask
 
 
+def test_faster_kernel_at_measured_sizes(by_wave):
+    """Sizes at which one kernel was measured faster by a tenth or more."""
+    wave = [(2, 14000, 1), (2, 50000, 4), (2, 100000, 8), (2, 200000, 12), (2, 1000000, 16), (3, 14000, 1),
+            (3, 50000, 1), (3, 100000, 2), (3, 200000, 5), (3, 300000, 8), (3, 400000, 6), (3, 400000, 10), (3, 1000000, 12)]
+    heap = [(2, 100000, 1), (2, 200000, 4), (2, 300000, 8), (2, 1000000, 12), (3, 200000, 1), (3, 200000, 2),
+            (3, 300000, 1), (3, 300000, 4), (3, 400000, 4), (3, 1000000, 6)]
+    assert all(by_wave(*((*q, 20) for q in wave)))
+    assert not any(by_wave(*((*q, 20) for q in heap)))
+
+
 def test_a_set_line_is_kept(by_wave):
     """A program's own row length decides alone, whatever the list's length."""
     q = [(dim, nq, k, line) for dim in (2, 3) for nq in (1000, 300000, 5000000) for k in (1, 8, 16, 24, 32, 100, 256)
