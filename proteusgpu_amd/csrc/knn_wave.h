@@ -18,10 +18,10 @@ template <int DIM, int M, bool SUB>
 __global__ void __launch_bounds__(64, knn_wave_occupancy<M>())
     k_knn_wave(const double* __restrict__ sorted, const uint32_t* __restrict__ perm, int N,
                const int32_t* __restrict__ starts, const int32_t* __restrict__ counts,
-               const uint32_t* __restrict__ queries, int64_t nq, int k, uint32_t* __restrict__ out,
+               const uint32_t* __restrict__ queries, int64_t q0, int64_t nq, int k, uint32_t* __restrict__ out,
                KnnTail tail, SubGrid sg) {
     __shared__ KnnSmem<M> smem;
-    const int64_t qi = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t qi = q0 + xcd_block(blockIdx.x, gridDim.x);
     if (qi >= nq) return;  // whole block
     const uint32_t q = queries ? queries[qi] : (uint32_t)qi;
     int kp = 0;
@@ -34,12 +34,16 @@ template <int DIM, int M>
 void run_wave(const double* sorted, const uint32_t* perm, int N, const int32_t* starts,
               const int32_t* counts, const uint32_t* queries, int64_t nq, int k, uint32_t* out,
               KnnTail tail, SubGrid sg, hipStream_t s) {
-    if (sg.m != nullptr)
-        k_knn_wave<DIM, M, true><<<(unsigned)nq, 64, 0, s>>>(sorted, perm, N, starts, counts, queries, nq, k, out,
-                                                             tail, sg);
-    else
-        k_knn_wave<DIM, M, false><<<(unsigned)nq, 64, 0, s>>>(sorted, perm, N, starts, counts, queries, nq, k, out,
-                                                              tail, sg);
+    // a launch of 2^32 threads or more wraps without an error: one block of 64
+    // per query goes up to 2^26 queries
+    constexpr int64_t MOST = (int64_t)1 << 25;
+    for (int64_t q0 = 0; q0 < nq; q0 += MOST) {
+        const unsigned nb = (unsigned)(nq - q0 < MOST ? nq - q0 : MOST);
+        if (sg.m != nullptr)
+            k_knn_wave<DIM, M, true><<<nb, 64, 0, s>>>(sorted, perm, N, starts, counts, queries, q0, nq, k, out, tail, sg);
+        else
+            k_knn_wave<DIM, M, false><<<nb, 64, 0, s>>>(sorted, perm, N, starts, counts, queries, q0, nq, k, out, tail, sg);
+    }
 }
 
 }  // namespace
