@@ -95,10 +95,10 @@ __global__ void __launch_bounds__(TB) k_cell_scatter(int64_t n, const int32_t* c
 // Bound by the chain count, range, store: a thread per cell with an insertion
 // sort took 12.6 us at 3k cells, this 3.0, and 17.3 us at 320k cells, this 11.8.
 constexpr int SL = 8;
-__global__ void __launch_bounds__(TB) k_cell_sort(int64_t ncell, const int32_t* starts,
+__global__ void __launch_bounds__(TB) k_cell_sort(int64_t c0, int64_t ncell, const int32_t* starts,
                                                   const int32_t* counts, uint32_t* idx, int32_t* big,
                                                   int32_t* nbig) {
-    const int64_t c = ((int64_t)blockIdx.x * TB + threadIdx.x) / SL;
+    const int64_t c = c0 + ((int64_t)blockIdx.x * TB + threadIdx.x) / SL;
     const int l = threadIdx.x % SL, base = (threadIdx.x & (WAVE - 1)) - l;
     int len = c < ncell ? counts[c] : 0;
     if (len > 32) {
@@ -340,7 +340,11 @@ void launch_cell_scatter(int64_t n, const int32_t* cell, const int32_t* starts, 
 void launch_cell_sort(int64_t ncell, const int32_t* starts, const int32_t* counts, uint32_t* idx,
                       int32_t* big, int32_t* nbig, hipStream_t s) {
     if (ncell <= 0) return;
-    k_cell_sort<<<nblk(ncell * SL), TB, 0, s>>>(ncell, starts, counts, idx, big, nbig);
+    // a launch of 2^32 threads or more wraps without an error (2^29 cells, as
+    // 1.7e9 points have)
+    constexpr int64_t MOST = (int64_t)1 << 24;
+    for (int64_t c0 = 0; c0 < ncell; c0 += MOST)
+        k_cell_sort<<<nblk(std::min(MOST, ncell - c0) * SL), TB, 0, s>>>(c0, ncell, starts, counts, idx, big, nbig);
     k_cell_sort_big<<<(unsigned)std::min<int64_t>(ncell, 1024), TB, 0, s>>>(big, nbig, starts, counts, idx);
 }
 

@@ -1,6 +1,7 @@
 """Neighbour lists of more queries than one launch of a wave per query can
 hold (2^26), by the wave kernel and by the heap, against torch in 64 bits for
-queries on both sides of the launches' ends."""
+queries on both sides of the launches' ends; and the cell order that such a
+set is sorted into, whose kernel takes 2^24 cells per launch."""
 import numpy as np
 import pytest
 import torch
@@ -18,6 +19,16 @@ def problem(ctx):
     print(f"n={N} N_grid={kp.N_grid}", flush=True)
     yield kp, torch.from_numpy(kp.get_points()).cuda()
     kp.free()
+
+
+def test_points_of_a_cell_in_input_order(problem):
+    kp, pts = problem
+    m = kp.N_grid
+    assert m * m > (1 << 24)
+    perm = torch.from_numpy(kp.get_permutation().astype(np.int64)).cuda()
+    c = torch.clamp(torch.floor(pts * m).long(), 0, m - 1)
+    cell = c[:, 0] + m * c[:, 1]
+    assert bool(torch.all((cell[1:] > cell[:-1]) | ((cell[1:] == cell[:-1]) & (perm[1:] > perm[:-1]))))
 
 
 @pytest.mark.parametrize("k", [12, 16])
