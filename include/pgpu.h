@@ -398,9 +398,10 @@ typedef struct {
     int knn_wave_min_k;  /* rows at least this long use the wave-per-query KNN,
                           * shorter ones the heap per thread; the default, 20,
                           * leaves shorter rows to the kernel measured faster    */
-    int blocks_per_cu;   /* resident blocks per CU of the persistent KNN and clip
-                          * kernels (KNN, 2D clip, restart clips), at most their
-                          * occupancy (default 64: all)                          */
+    int blocks_per_cu;   /* resident blocks per CU of the clip kernels (8 times as
+                          * many of the KNN's) but the 3D first pass's, at most
+                          * their occupancy (default 64: all; where nothing is
+                          * capped the first passes are no persistent blocks)    */
     int use_graph;       /* 1: capture the step in a hipGraph, 0: plain launches     */
 } pg_batch_tuning;
 

@@ -319,7 +319,7 @@ __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_bvoronoi_lo
         if (vb >= nvb) break;
         const auto* A = fresh_args<ClipArgs>();
         voronoi_group<DIM, G, S>(A->pts, INT64_MAX, A->seeds, *A->nq_dev, A->knn, A->k, A->max_p, A->max_t,
-                                 A->fa.resume, A->fa.cstate, A->fa.key, sm, vb);
+                                 A->from, A->fa.cstate, A->fa.key, sm, vb);
         __syncthreads();
     }
 }
@@ -531,12 +531,12 @@ void bknn_wave(const double* sorted, const uint32_t* perm, const int32_t* sbox, 
                const int64_t* coff, const int32_t* starts, const int32_t* counts, const uint32_t* q,
                const int64_t* nq_dev, int64_t cap, int k, uint32_t* out, int blocks_per_cu,
                unsigned long long* ticket, bool loop, hipStream_t s, KnnTail tail) {
-    if (!loop) {
+    static const int occ = occupancy(k_bknn_wave<DIM, M>);
+    if (!loop && 8 * blocks_per_cu >= occ) {  // a cap on the resident blocks needs the loop
         const BKnnArgs args{sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, out, ticket, tail, k};
         k_bknn_list<DIM, M><<<(unsigned)std::max<int64_t>(cap, 1), 64, 0, s>>>(args);
         return;
     }
-    static const int occ = occupancy(k_bknn_wave<DIM, M>);
     const unsigned nb = (unsigned)std::min<int64_t>(cap, resident_blocks(occ, 8 * blocks_per_cu));
     k_fill<unsigned long long><<<1, TB, 0, s>>>(ticket, 1, 0ull);
     const BKnnArgs args{sorted, perm, sbox, N, coff, starts, counts, q, nq_dev, out, ticket, tail, k};
@@ -563,9 +563,10 @@ void bclip(const double* pts, const uint32_t* seeds, const int64_t* nq_dev, int6
            int max_p, int max_t, FaceArrays fa, int blocks_per_cu, unsigned long long* ticket, bool loop,
            hipStream_t s) {
     using C = VoroCfg<DIM, G, S>;
-    const ClipArgs args{pts, INT64_MAX, seeds, 0, nq_dev, knn, ticket, fa, k, max_p, max_t};
-    if (loop) {
-        static const int occ = occupancy(k_bvoronoi_loop<DIM, G, S>);
+    const ClipArgs args{pts, INT64_MAX, seeds, 0, nq_dev, knn, ticket, fa, k, max_p, max_t, loop ? fa.resume : nullptr};
+    static const int occ = occupancy(k_bvoronoi_loop<DIM, G, S>);
+    // 2D first passes keep to a cap on the resident blocks too
+    if (loop || (DIM == 2 && blocks_per_cu < occ)) {
         const unsigned nb =
             (unsigned)std::min<int64_t>((cap + C::SPW - 1) / C::SPW, resident_blocks(occ, blocks_per_cu));
         k_fill<unsigned long long><<<1, TB, 0, s>>>(ticket, 1, 0ull);

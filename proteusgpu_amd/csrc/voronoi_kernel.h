@@ -625,6 +625,7 @@ struct ClipArgs {
     unsigned long long* ticket;
     FaceArrays fa;
     int k, max_p, max_t;
+    const int32_t* from = nullptr;  // batches: resume entries the pass goes on from (first pass: none)
 };
 
 // The first argument of the running kernel, through a pointer the compiler

@@ -2,8 +2,11 @@
 
 The KNN's line between heap and wave rows at, below and above the row length
 (short 2D rows, 3D rows, and rows long enough for the heap's half-filled
-blocks), for all the batch's passes, and the 3D clip shapes: states equal to
-the bit, and equal to the boxes run alone.
+blocks), for all the batch's passes, the 3D clip shapes, and caps on the
+resident blocks below and above the kernels' occupancy, which make the first
+passes persistent blocks or a block per query or group (with rows so short
+that nearly every cell goes on from its saved state, and without restarts):
+states equal to the bit, and equal to the boxes run alone.
 """
 import itertools
 
@@ -61,3 +64,13 @@ def test_clip_shapes_3d(ctx):
     for lanes, slots in itertools.product((8, 16), (48, 64)):
         for a, b in zip(_run(ctx, *case, clip_lanes=lanes, clip_slots=slots), ref):
             assert np.array_equal(a, b), (lanes, slots)
+
+
+@pytest.mark.parametrize("dim,k,restart", [(2, 10, True), (2, 16, True), (2, 64, False), (3, 24, True)])
+def test_caps_on_resident_blocks(ctx, dim, k, restart):
+    sizes, pts, st, kw = _case(dim, k)
+    kw["restart"] = restart
+    ref = _alone(ctx, sizes, pts, st, kw)
+    for cap, graph in itertools.product((1, 2, 8, 64), (True, False)):
+        for a, b in zip(_run(ctx, sizes, pts, st, kw, blocks_per_cu=cap, use_graph=graph), ref):
+            assert np.array_equal(a, b), (cap, graph)
