@@ -424,8 +424,8 @@ int pg_batch_set_tuning(pg_batch* batch, const pg_batch_tuning* t);
  * the model must outlive its use.  Results do not change. */
 int pg_batch_set_kmodel(pg_batch* batch, const pg_kmodel* model);
 int pg_batch_get_tuning(const pg_batch* batch, pg_batch_tuning* t);
-/* Time every tuning candidate (clip shape x KNN kernel choice x grid size)
- * on `reps` steps from the current state, restore the state and keep the
+/* Time every tuning candidate (3D clip shape x KNN kernel choice x grid size,
+ * as far as they differ) on `reps` steps from the current state, restore the state and keep the
  * fastest.  Results never depend on the tuning. */
 int pg_batch_autotune(pg_ctx* ctx, pg_batch* batch, int reps, pg_batch_tuning* best, double* best_ms);
 /* Primitives and generator positions, box-major. */

@@ -8,6 +8,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/pgpu.h"
@@ -2517,13 +2518,16 @@ int pg_batch_autotune(pg_ctx* c, pg_batch* B, int reps, pg_batch_tuning* best, d
         const pg_batch_tuning start{B->lanes, B->slots, B->wave_min_k, B->bpc, B->use_graph ? 1 : 0};
         pg_batch_tuning winner = start;
         double wms = 1e300;
-        const int shape_c[4][2] = {{16, 64}, {16, 48}, {8, 64}, {8, 48}};
-        const int wave_c[2] = {33, 1};
-        const int bpc_c[2] = {8, 64};
-        for (int a = 0; a < 4; a++)
-            for (int w = 0; w < 2; w++)
-                for (int q = 0; q < 2; q++) {
-                    const pg_batch_tuning t{shape_c[a][0], shape_c[a][1], wave_c[w], bpc_c[q], 1};
+        // only settings that change a kernel: 2D clips have one shape (the
+        // batch keeps the one set), and no row of a fixed k of 33 or more is
+        // the heap's either way
+        using Shapes = std::vector<std::pair<int, int>>;
+        const Shapes shapes = B->dim == 2 ? Shapes{{B->lanes, B->slots}} : Shapes{{16, 64}, {16, 48}, {8, 64}, {8, 48}};
+        const std::vector<int> waves = B->km || B->prm.mesh.k < 33 ? std::vector<int>{33, 1} : std::vector<int>{1};
+        for (const auto& shape : shapes)
+            for (const int wave : waves)
+                for (const int bpc : {8, 64}) {
+                    const pg_batch_tuning t{shape.first, shape.second, wave, bpc, 1};
                     if (pg_batch_set_tuning(B, &t) != PG_OK) throw Error{PG_ERR_ARG, g_err};
                     double tot = 0;
                     for (int r = 0; r < reps; r++) {

@@ -74,3 +74,21 @@ def test_caps_on_resident_blocks(ctx, dim, k, restart):
     for cap, graph in itertools.product((1, 2, 8, 64), (True, False)):
         for a, b in zip(_run(ctx, sizes, pts, st, kw, blocks_per_cu=cap, use_graph=graph), ref):
             assert np.array_equal(a, b), (cap, graph)
+
+
+def test_autotune_leaves_what_it_cannot_time(ctx):
+    """2D clips have one shape, so the setting stays as it was; every candidate's
+    step still gives the same states."""
+    sizes, pts, st, kw = _case(2, 16)
+    ref = _alone(ctx, sizes, pts, st, kw)
+    for lanes, slots in ((8, 48), (16, 48)):
+        B = api.Batch(ctx, sizes, pts, *st, **kw)
+        B.set_tuning(clip_lanes=lanes, clip_slots=slots)
+        best, _ = B.autotune(reps=1)
+        assert (best["clip_lanes"], best["clip_slots"]) == (lanes, slots)
+        assert B.tuning == best
+        B.step()
+        B.step()
+        for a, b in zip(B.get(), ref):
+            assert np.array_equal(a, b)
+        B.free()
