@@ -64,6 +64,10 @@ int pg_device_count(int* count);
 int pg_ctx_create(int device, pg_ctx** out);
 int pg_ctx_destroy(pg_ctx* ctx);
 int pg_ctx_sync(pg_ctx* ctx);
+/* Free the device memory that destroyed objects left for later ones (at most
+ * 8 GiB per device, held while a context lives), for other allocators of the
+ * process; objects that live are not touched. */
+int pg_ctx_trim(pg_ctx* ctx);
 /* No reference counterpart: streams `bytes` device-to-device `reps` times and
  * returns the mean kernel time (HIP events); measured HBM bandwidth =
  * 2*bytes/ms.  Also the calibration kernel for HBM traffic counters. */

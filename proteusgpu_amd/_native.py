@@ -90,6 +90,7 @@ def _signatures():
         "pg_set_clip_resume": ([i32], i32),
         "pg_get_clip_resume": ([C.POINTER(C.c_int)], i32),
         "pg_ctx_create": ([i32, pp], i32), "pg_ctx_destroy": ([vp], i32), "pg_ctx_sync": ([vp], i32),
+        "pg_ctx_trim": ([vp], i32),
         "pg_stream_copy_probe": ([vp, i64, i32, C.POINTER(C.c_double)], i32),
         "pg_knn_init": ([vp, i32, vp, i64, pp], i32), "pg_knn_solve": ([vp, vp, i32], i32),
         "pg_knn_info": ([vp, C.POINTER(C.c_int64), C.POINTER(C.c_int), C.POINTER(C.c_int)], i32),

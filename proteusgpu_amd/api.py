@@ -70,6 +70,10 @@ class Context:
     def sync(self):
         check(lib().pg_ctx_sync(self.h))
 
+    def trim(self):
+        """Free the device memory held for later objects (for other allocators)."""
+        check(lib().pg_ctx_trim(self.h))
+
     def stream_copy_probe(self, nbytes: int = 1 << 30, reps: int = 10) -> float:
         """Measured device copy bandwidth in GB/s (reads + writes)."""
         ms = C.c_double()

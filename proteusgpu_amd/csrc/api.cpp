@@ -54,7 +54,8 @@ int guarded(F&& f) {
 // 400k 3D one (on machines that map memory slowly 90 of 170).
 //  - At most KEEP bytes per device are held, the oldest go first, and only
 //    while a context of the device lives: the last one's end frees them all.
-//    An allocation that fails frees them and tries again.
+//    An allocation that fails frees them and tries again, and a program that
+//    needs the memory elsewhere has pg_ctx_trim.
 //  - A block may have been left with work on it in flight, on any stream: the
 //    first one taken since waits for the device (as hipFree would have at its
 //    release), which clears all blocks left until then.  Where the wait is
@@ -78,6 +79,10 @@ public:
     void context_removed() {
         std::lock_guard<std::mutex> g(mu);
         if (--contexts == 0) drop_to(0);
+    }
+    void trim() {
+        std::lock_guard<std::mutex> g(mu);
+        drop_to(0);
     }
     // a block of at least bytes (cap: its size), or null
     void* take(size_t bytes, size_t& cap) {
@@ -957,6 +962,13 @@ int pg_ctx_sync(pg_ctx* c) {
     return guarded([&] {
         use(c);
         HIPCHK(hipStreamSynchronize(c->stream));
+    });
+}
+
+int pg_ctx_trim(pg_ctx* c) {
+    return guarded([&] {
+        use(c);
+        BlockPool::of(c->device).trim();
     });
 }
 
