@@ -434,7 +434,7 @@ int pg_batch_get_tuning(const pg_batch* batch, pg_batch_tuning* t);
 int pg_batch_autotune(pg_ctx* ctx, pg_batch* batch, int reps, pg_batch_tuning* best, double* best_ms);
 /* Primitives and generator positions, box-major. */
 int pg_batch_get(pg_ctx* ctx, pg_batch* batch, double* pts, double* rho, double* vel, double* E);
-/* CFL step each box took in the last step (nbox doubles). */
+/* CFL step each box took in the last step (nbox doubles; 0 before the first). */
 int pg_batch_dt(pg_ctx* ctx, const pg_batch* batch, double* dt);
 /* FP64 totals per box: [mass, px, py, pz, energy] x nbox. */
 int pg_batch_totals(pg_ctx* ctx, pg_batch* batch, double* tot);

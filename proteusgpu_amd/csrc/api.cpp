@@ -2393,7 +2393,8 @@ int pg_batch_create(pg_ctx* c, const pg_sim_params* prm, int nbox, const int64_t
             B->mass_s.get<double>(n);
             B->mom_s.get<double>(n * d);
             B->en_s.get<double>(n);
-            B->dt_box.get<double>(nbox);
+            // 0 until the first step sets it (pg_batch_dt)
+            pg::launch_fill_u64(B->dt_box.get<unsigned long long>(nbox), nbox, 0ull, s);
             B->gcnt.get<int32_t>(n);
             B->goff.get<int32_t>(n);
             B->gtot.get<int32_t>(1);

@@ -58,3 +58,15 @@ def test_first_pass_ignores_what_its_memory_held(ctx, dim, boundary, sizes, k, l
         assert np.array_equal(a, np.concatenate(b))
     B.free()
     like.free()
+
+
+def test_no_step_no_dt(ctx):
+    """The CFL steps of a batch that has not stepped are 0, whatever its memory held."""
+    sizes = np.array([1500, 1700, 1600])
+    pts = batch_points(sizes, 2, 520)
+    _leave(ctx, 64, 0x3ff01234)
+    B = api.Batch(ctx, sizes, pts, *kelvin_helmholtz_state(pts), boundary="periodic", buff=0.1, k=16)
+    assert np.array_equal(B.dt(), np.zeros(3))
+    B.step()
+    assert np.all(B.dt() > 0)
+    B.free()
