@@ -252,14 +252,25 @@ struct KnnPend {
     uint32_t s[128];
 };
 
-// Candidates of the row search (knn_rows_query): key and sorted id, up to CAP.
+// Candidates of the row search (knn_rows_query): key and sorted id, up to CAP;
+// then, where ranks tie (knn_rows_ties), the kept ones' exact distance,
+// quantized distance and input index by rank.
 template <int M>
 struct KnnRows {
     static constexpr int BITS = M <= 2 ? 8 : 9;  // bits of a candidate's position in its key
     static constexpr int CAP = 1 << BITS;
-    uint32_t key[CAP], id[CAP];
+    static constexpr int KEPT = M <= 4 ? 64 * M : 1;
+    union {
+        struct {
+            uint32_t key[CAP], id[CAP];
+        };
+        struct {
+            double d[KEPT];
+            uint32_t qd[KEPT], ord[KEPT];
+        };
+    };
     int32_t shift[64];  // per row of cells: first sorted id minus the row's first candidate index
-    uint32_t mark[64];  // rows starting in the current 64 candidates
+    uint32_t mark[64];  // rows starting in the current 64 candidates; ids of the last ranks' run of ties
 };
 
 // LDS of one wave query.
@@ -398,16 +409,17 @@ PG_DEV void key_merge_batch(uint32_t (&kk)[M], uint32_t& out, uint32_t a, int l,
 // and a max-scan give each lane its row).  The points inside the ball wait in
 // LDS under a 32-bit key, their squared distance quantized (monotone) above
 // their position in the buffer; the keys are sorted across the wave with
-// integer min / max.  Equal quantized distances among the kept ranks are put in
-// the exact (d^2, input index) order afterwards.
+// integer min / max.  Where quantized distances tie among the ranks asked for
+// nothing is written and -n tells that the n candidates of the buffer are left
+// to knn_rows_ties.
 //
-// false: nothing was written, and the ring walk has to answer: fewer than k
-// points after a second, wider ball, more than the buffer or the row limit
-// holds, a candidate below its ring's distance bound (the argument of
-// knn_wave_query), or ties that reach past the kept keys.  With the ball's k
-// first in order the row is the ring walk's by the same argument: the rows
-// skip only points outside the ball (the float bounds carry a slack of
-// several float roundings of N), so every point of the ball is seen.
+// ROWS_DONE: the row is written.  ROWS_NONE: nothing was written, and the ring
+// walk has to answer: fewer than k points after a second, wider ball, more than
+// the buffer or the row limit holds, or a candidate below its ring's distance
+// bound (the argument of knn_wave_query).  With the ball's k first in order
+// the row is the ring walk's by the same argument: the rows skip only points
+// outside the ball (the float bounds carry a slack of several float roundings
+// of N), so every point of the ball is seen.
 //
 // What bounds it: VALU issue (640 instructions per query, k = 32 and its 64
 // tails; the ring walk with FP64 sorts took 1.75k).  1M uniform 3D queries:
@@ -415,8 +427,9 @@ PG_DEV void key_merge_batch(uint32_t (&kk)[M], uint32_t& out, uint32_t a, int l,
 // of cells replaces 27 and then 98 cells looked at one by one, the mark scan a
 // binary search per candidate, and an exchange of the sort takes three
 // integer instructions instead of a dozen.
+constexpr int ROWS_DONE = 1, ROWS_NONE = 0;
 template <int DIM, int M>
-PG_DEV bool knn_rows_query(const double* __restrict__ sorted, const uint32_t* __restrict__ perm, int N, int64_t cbase,
+PG_DEV int knn_rows_query(const double* __restrict__ sorted, const uint32_t* __restrict__ perm, int N, int64_t cbase,
                            const int32_t* __restrict__ starts, const int32_t* __restrict__ counts, uint32_t q, int k,
                            uint32_t* __restrict__ o, KnnRows<M>& sm, const double (&p)[3], const double (&P)[3],
                            double r2, float lam, int kp, double lo_d, uint32_t lo_s) {
@@ -432,7 +445,7 @@ PG_DEV bool knn_rows_query(const double* __restrict__ sorted, const uint32_t* __
         const int klo = DIM == 3 ? max(0, min(N - 1, (int)floorf(Pz - Rc))) : 0;
         const int khi = DIM == 3 ? max(0, min(N - 1, (int)floorf(Pz + Rc))) : 0;
         const int nj = jhi - jlo + 1, nrows = nj * (khi - klo + 1);
-        if (nrows > 256) return false;
+        if (nrows > 256) return ROWS_NONE;
         const float rnj = 1.0f / (float)nj;
         const float rr2 = Rc * Rc;
         // the smallest quantum that keeps every d^2 <= r2 below 2^QB
@@ -506,7 +519,7 @@ PG_DEV bool knn_rows_query(const double* __restrict__ sorted, const uint32_t* __
                 }
                 const uint64_t surv = (uint64_t)__ballot(take);
                 const int ns = __popcll((unsigned long long)surv);
-                if (n + ns > CAP) return false;
+                if (n + ns > CAP) return ROWS_NONE;
                 if (take) {
                     const int at = n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(surv >> 32),
                                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)surv, 0u));
@@ -517,9 +530,9 @@ PG_DEV bool knn_rows_query(const double* __restrict__ sorted, const uint32_t* __
             }
             __syncthreads();
         }
-        if (__ballot(odd) != 0ull) return false;
+        if (__ballot(odd) != 0ull) return ROWS_NONE;
         if (n >= k) break;
-        if (pass >= 1) return false;
+        if (pass >= 1) return ROWS_NONE;
         // fewer than k points in the ball: a wider one
         const float g = __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(lam / ((float)(kp + n) + 1.0f)) * (2.0f / DIM));
         r2 *= (double)fminf(fmaxf(g, 1.5f), 16.0f);
@@ -534,7 +547,7 @@ PG_DEV bool knn_rows_query(const double* __restrict__ sorted, const uint32_t* __
 #pragma unroll
         for (int j = 0; j < M; j++)
             if (j == (k - 1) >> 6) kth = read_lane(kk[j], (k - 1) & 63);
-        if (__ballot((out >> BITS) <= (kth >> BITS)) != 0ull) return false;
+        if (__ballot((out >> BITS) <= (kth >> BITS)) != 0ull) return -n;
     }
     // equal quantized distances at neighbouring ranks, up to rank k
     bool tie = false;
@@ -550,37 +563,90 @@ PG_DEV bool knn_rows_query(const double* __restrict__ sorted, const uint32_t* __
         const int r = 64 * j + l;
         tie = tie || (r < k && r + 1 < n && (nx >> BITS) == (kk[j] >> BITS));
     }
-    uint32_t id[M];
-#pragma unroll
-    for (int j = 0; j < M; j++) id[j] = 64 * j + l < n ? sm.id[kk[j] & (CAP - 1)] : 0xffffffffu;
-    if (__ballot(tie) != 0ull) {
-        if (M > 1) return false;  // ties in longer rows: the ring walk's
-        double d = __builtin_inf();
-        if (l < n) {
-            double pc[3] = {0, 0, 0};
-#pragma unroll
-            for (int e = 0; e < DIM; e++) pc[e] = sorted[(size_t)DIM * id[0] + e];
-            d = dist2<DIM>(p, pc);
-        }
-        // odd-even transpositions in the exact order (already in order but
-        // for the ties) until nothing moves
-        for (int still = 0, ph = 0; still < 2; ph ^= 1) {
-            const int pl = ((l + ph) ^ 1) - ph;
-            const int src = pl < 0 || pl > 63 ? l : pl;
-            const double pd = __shfl(d, src, 64);
-            const uint32_t pi = (uint32_t)__shfl((int)id[0], src, 64);
-            const bool up = src > l;
-            const bool swap = src != l && src < n && l < n && (up ? ent_less(perm, pd, pi, d, id[0]) : ent_less(perm, d, id[0], pd, pi));
-            if (swap) {
-                d = pd;
-                id[0] = pi;
-            }
-            still = __ballot(swap) != 0ull ? 0 : still + 1;
-        }
-    }
+    if (__ballot(tie) != 0ull) return -n;
 #pragma unroll
     for (int j = 0; j < M; j++)
-        if (64 * j + l < k) o[64 * j + l] = id[j];
+        if (64 * j + l < k) o[64 * j + l] = sm.id[kk[j] & (CAP - 1)];
+    return ROWS_DONE;
+}
+
+// The row of k out of the n candidates that knn_rows_query left in the buffer,
+// some of whose quantized distances tie among the first k ranks (lattices: every
+// shell of neighbours).  A run of ties that is kept whole is ranked in the exact
+// order by its members in LDS; the last one, where members of it left the
+// sorted list, is gathered from the buffer and ranked by comparing all pairs.
+// false: more than 64 candidates tie with rank k, and nothing was written.
+//
+// The keys are sorted again here, so that none of this stays live across the
+// search (in line with it uniform rows took 2% longer).  Whole calls on exact
+// lattices of 200,000 points, ms, by the ring walk after the search (M > 1, or
+// members of the last run gone) or a transposition sort and now: 2D k = 16 0.33
+// and 0.30, k = 64 0.80, 0.43; 3D k = 16 0.42, 0.37, k = 32 0.61, 0.51.
+template <int DIM, int M>
+PG_DEV bool knn_rows_ties(const double* __restrict__ sorted, const uint32_t* __restrict__ perm, uint32_t q, int k,
+                          uint32_t* __restrict__ o, KnnRows<M>& sm, const double (&p)[3], int n) {
+    const int l = threadIdx.x;
+    constexpr int BITS = KnnRows<M>::BITS, CAP = KnnRows<M>::CAP;
+    uint32_t kk[M], id[M], out = ~0u;
+#pragma unroll
+    for (int j = 0; j < M; j++) kk[j] = ~0u;
+    for (int b = 0; b < n; b += 64) key_merge_batch<M>(kk, out, b + l < n ? sm.key[b + l] : ~0u, l, b == 0);
+#pragma unroll
+    for (int j = 0; j < M; j++) id[j] = 64 * j + l < n ? sm.id[kk[j] & (CAP - 1)] : 0xffffffffu;
+    auto exact_d = [&](uint32_t t) __attribute__((always_inline)) {
+        double pc[3] = {0, 0, 0};
+#pragma unroll
+        for (int e = 0; e < DIM; e++) pc[e] = sorted[(size_t)DIM * t + e];
+        return dist2<DIM>(p, pc);
+    };
+    int whole = min(n, 64 * M);  // ranks of runs kept whole
+    uint32_t last = 0;           // quantized distance of rank k
+#pragma unroll
+    for (int j = 0; j < M; j++)
+        if (j == (k - 1) >> 6) last = read_lane(kk[j], (k - 1) & 63) >> BITS;
+    if (n > 64 * M && __ballot((out >> BITS) <= last) != 0ull) {
+        int nl = 0;
+        for (int b = 0; b < n; b += 64) {
+            const bool hit = b + l < n && (sm.key[b + l] >> BITS) == last;
+            const uint64_t m = (uint64_t)__ballot(hit);
+            const int at = nl + __popcll(m & ((1ull << l) - 1ull));
+            if (hit && at < 64) sm.mark[at] = sm.id[b + l];
+            nl += __popcll(m);
+        }
+        if (nl > 64) return false;
+        whole = 0;
+#pragma unroll
+        for (int j = 0; j < M; j++) whole += __popcll(__ballot((kk[j] >> BITS) < last));
+        __syncthreads();
+        const uint32_t t = l < nl ? sm.mark[l] : q;
+        const double d = exact_d(t);
+        const uint32_t od = perm[t];
+        int r = whole;
+        for (int i = 0; i < nl; i++) r += cand_less(read_lane_d(d, i), read_lane(od, i), d, od) ? 1 : 0;
+        if (l < nl && r < k) o[r] = t;
+    }
+    __syncthreads();  // the buffer's last read
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        const int r = 64 * j + l;
+        if (r < whole) {
+            sm.d[r] = exact_d(id[j]);
+            sm.qd[r] = kk[j] >> BITS;
+            sm.ord[r] = perm[id[j]];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        const int r = 64 * j + l;
+        if (r >= whole) continue;
+        const double d = sm.d[r];
+        const uint32_t qd = kk[j] >> BITS, od = sm.ord[r];
+        int at = r;
+        for (int i = r - 1; i >= 0 && sm.qd[i] == qd; i--) at -= cand_less(d, od, sm.d[i], sm.ord[i]) ? 1 : 0;
+        for (int i = r + 1; i < whole && sm.qd[i] == qd; i++) at += cand_less(sm.d[i], sm.ord[i], d, od) ? 1 : 0;
+        if (at < k) o[at] = id[j];
+    }
     return true;
 }
 
@@ -729,9 +795,10 @@ PG_DEV void knn_wave_query(const double* __restrict__ sorted, const uint32_t* __
         }
     }
     if (!SUB && M <= 4) {
-        if (knn_rows_query<DIM, M>(sorted, perm, N, cbase, starts, counts, q, k, o, smem.rows, p, P, r2, lam, kp, lo_d,
-                                   lo_s))
-            return;
+        const int got = knn_rows_query<DIM, M>(sorted, perm, N, cbase, starts, counts, q, k, o, smem.rows, p, P, r2, lam,
+                                               kp, lo_d, lo_s);
+        if (got == ROWS_DONE) return;
+        if (got < 0 && knn_rows_ties<DIM, M>(sorted, perm, q, k, o, smem.rows, p, -got)) return;
         __syncthreads();
     }
     bool odd_l = false;  // a kept candidate below its ring's distance bound
