@@ -302,11 +302,10 @@ __global__ void __launch_bounds__(64, (M <= 2 ? 6 : 5)) k_bknn_wave(BKnnArgs arg
 // list's capacity; blocks past the device-side count end at once (each
 // costs a dispatch, so it suits lists that fill most of their capacity).
 // k_bvoronoi_loop: persistent blocks taking groups from a counter, the
-// arguments re-read per group (in a loop the compiler still keeps values
-// across groups, and the clip's registers spill: it suits the short lists
-// of the certificate restarts, where capacity-sized grids would be mostly
-// empty blocks).
-// The arguments are re-read per group (fewer spills).
+// arguments re-read per group (fewer spills; in a loop the compiler still keeps
+// values across groups, and the clip's registers spill: it suits the short
+// lists of the certificate restarts, where capacity-sized grids would be mostly
+// empty blocks, and 2D first passes whose resident blocks are capped).
 template <int DIM, int G, int S>
 __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_bvoronoi_loop(ClipArgs args) {
     using C = VoroCfg<DIM, G, S>;

@@ -8,9 +8,10 @@
 namespace pg {
 namespace {
 
-// Fast kernel: 16 lanes x 4 slots = 64 vertex slots per seed, 4 seeds per
-// wave.  Large kernel: 16 lanes x 8 slots = 128 slots, for seeds whose cell
-// outgrows 64 vertices before max_t (rare).
+// Fast kernel: in 3D 16 lanes x 4 slots = 64 vertex slots and 48 planes per
+// seed, 4 seeds per wave; in 2D 8 lanes x 2 slots = 16 vertices and 24 planes, 8
+// seeds per wave.  Large kernel: 16 lanes x 8 slots = 128 slots and 64 planes,
+// for seeds whose cell outgrows these before max_t and max_p (rare).
 template <int DIM, int G, int S>
 __global__ void __launch_bounds__(64, (VoroCfg<DIM, G, S>::WAVES)) k_voronoi(ClipArgs a) {
     __shared__ VoroSmem<DIM, G, S> sm[VoroCfg<DIM, G, S>::SPW];

@@ -1,4 +1,4 @@
-"""The neighbour search by rows of grid cells (rows of 20 and more).
+"""The neighbour search by rows of grid cells.
 
 Neighbour lists must equal the oracle's: row lengths around the kept 64 keys
 per slot, equal distances (lattices, whose shells tie inside and across the
