@@ -20,6 +20,7 @@ and a CPU baseline (the FP64 oracle on a bounded sample of the same
 workload, timed on this host).
 """
 import argparse
+import hashlib
 import json
 import os
 import sys
@@ -65,16 +66,27 @@ def parse():
     return ap.parse_args()
 
 
+def clip_profile(name, root=ROOT):
+    """A committed counter summary of profiles/ that was counted on the clip
+    kernel of this tree (it holds the sha1 of the kernel's source), else None:
+    another kernel's counts say nothing beside this one's times."""
+    try:
+        with open(os.path.join(root, "profiles", name)) as f:
+            d = json.load(f)
+        with open(os.path.join(root, "proteusgpu_amd", "csrc", "voronoi_kernel.h"), "rb") as f:
+            return d if d.get("voronoi_kernel_h_sha1") == hashlib.sha1(f.read()).hexdigest() else None
+    except OSError:
+        return None
+
+
 def clip_traffic(launches):
     """HBM bytes per launch of the first clip pass at this workload: the
     FETCH_SIZE + WRITE_SIZE of its launches in one step (rocprofv3 --pmc,
     scaled by a copy kernel of known size), from the committed summary in
     profiles/, divided by the launches per step; None without a summary."""
-    path = os.path.join(ROOT, "profiles", "k_voronoi_1m_traffic.json")
-    if not os.path.exists(path) or launches <= 0:
+    d = clip_profile("k_voronoi_1m_traffic.json")
+    if d is None or launches <= 0:
         return None
-    with open(path) as f:
-        d = json.load(f)
     per_step = d.get("learned_first_pass_bytes_per_step")
     return None if per_step is None else round(per_step / launches, 1)
 
@@ -225,11 +237,9 @@ def clip_valu(launches, avg_launch_ms):
     profiles/) x 4 cycles per wave instruction over the SIMD-cycles of one
     launch (1024 SIMDs x 2.4 GHz x the launch time measured here); None
     without a summary."""
-    path = os.path.join(ROOT, "profiles", "k_voronoi_1m_valu.json")
-    if not os.path.exists(path) or launches <= 0:
+    d = clip_profile("k_voronoi_1m_valu.json")
+    if d is None or launches <= 0:
         return None
-    with open(path) as f:
-        d = json.load(f)
     per_launch = d["valu_insts_per_step"] / launches
     simd_cycles = 1024 * 2.4e9 * avg_launch_ms * 1e-3
     return {"insts_per_launch": round(per_launch, 1), "issue_share": round(4.0 * per_launch / simd_cycles, 4),
