@@ -56,12 +56,14 @@ int guarded(F&& f) {
 //    while a context of the device lives: the last one's end frees them all.
 //    An allocation that fails frees them and tries again, and a program that
 //    needs the memory elsewhere has pg_ctx_trim.
-//  - A block may have been left with work on it in flight, on any stream: the
-//    first one taken since waits for the device (as hipFree would have at its
-//    release), which clears all blocks left until then.  Where the wait is
-//    refused (a stream of the calling thread is being captured), new memory
-//    is taken.
-//  - All of it under one lock.
+//  - A block may have been left with work on it in flight, on the stream of any
+//    context: the first one taken since waits for all of them (as hipFree would
+//    have at its release), which clears all blocks left until then.  A stream
+//    that is being captured must not be waited for, from no thread (nor the
+//    device: that ends every thread's capture with an error): no one waits
+//    during a capture of this library, whose own thread takes new memory, as
+//    does who meets another's capture.
+//  - All of it under one lock, which a capture holds to its end.
 class BlockPool {
 public:
     // never destroyed: buffers may outlive static destructors
@@ -72,31 +74,48 @@ public:
     static constexpr int MAX_DEVICES = 64;
     static constexpr size_t KEEP = (size_t)8 << 30;
 
-    void context_added() {
-        std::lock_guard<std::mutex> g(mu);
-        contexts++;
+    void context_added(hipStream_t s) {
+        std::lock_guard<std::recursive_mutex> g(mu);
+        streams.push_back(s);
     }
-    void context_removed() {
-        std::lock_guard<std::mutex> g(mu);
-        if (--contexts == 0) drop_to(0);
+    // before the stream ends (idle)
+    void context_leaves(hipStream_t s) noexcept {
+        std::lock_guard<std::recursive_mutex> g(mu);
+        streams.erase(std::remove(streams.begin(), streams.end(), s), streams.end());
+    }
+    // after the context's own buffers went
+    void context_gone() noexcept {
+        std::lock_guard<std::recursive_mutex> g(mu);
+        if (streams.empty()) drop_to(0);
     }
     void trim() {
-        std::lock_guard<std::mutex> g(mu);
+        std::lock_guard<std::recursive_mutex> g(mu);
         drop_to(0);
     }
+    // Held by the thread that captures, from before the capture to its end.
+    class Capture {
+    public:
+        explicit Capture(int device) : pool(of(device)), g(pool.mu) { pool.capturing = true; }
+        ~Capture() { pool.capturing = false; }
+        Capture(const Capture&) = delete;
+        Capture& operator=(const Capture&) = delete;
+
+    private:
+        BlockPool& pool;
+        std::lock_guard<std::recursive_mutex> g;
+    };
     // a block of at least bytes (cap: its size), or null
     void* take(size_t bytes, size_t& cap) {
-        std::lock_guard<std::mutex> g(mu);
+        std::lock_guard<std::recursive_mutex> g(mu);
         size_t best = free.size();
         for (size_t i = 0; i < free.size(); i++)
             if (free[i].cap >= bytes && free[i].cap <= bytes + bytes / 4 + SLACK &&
                 (best == free.size() || free[i].cap < free[best].cap))
                 best = i;
         if (best < free.size() && !free[best].idle) {
-            if (hipDeviceSynchronize() == hipSuccess) {
+            if (wait()) {
                 for (Block& b : free) b.idle = true;
             } else {
-                (void)hipGetLastError();
                 best = free.size();
             }
         }
@@ -122,9 +141,9 @@ public:
         return p;
     }
     void give(void* p, size_t cap) noexcept {
-        std::lock_guard<std::mutex> g(mu);
+        std::lock_guard<std::recursive_mutex> g(mu);
         bool kept = false;
-        if (contexts > 0 && cap <= KEEP) {
+        if (!streams.empty() && cap <= KEEP) {
             drop_to(KEEP - cap);
             try {
                 free.push_back({p, cap, false});
@@ -143,10 +162,24 @@ private:
         bool idle;  // no work left on it
     };
     static constexpr size_t SLACK = 4096;
-    std::mutex mu;
+    std::recursive_mutex mu;
     std::vector<Block> free;  // oldest first
     size_t held = 0;
-    int contexts = 0;
+    std::vector<hipStream_t> streams;  // of the contexts
+    bool capturing = false;
+    // Whether everything that the contexts' streams held is done.
+    bool wait() noexcept {
+        if (capturing) return false;  // by this thread: the others wait at the lock
+        for (hipStream_t s : streams) {
+            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone ||
+                hipStreamSynchronize(s) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+        }
+        return true;
+    }
     void drop_to(size_t bytes) noexcept {
         size_t n = 0;
         for (; held > bytes; n++) {
@@ -941,7 +974,13 @@ int pg_ctx_create(int device, pg_ctx** out) {
             delete c;
             hipchk(e, "hipStreamCreate");
         }
-        BlockPool::of(device).context_added();
+        try {
+            BlockPool::of(device).context_added(c->stream);
+        } catch (...) {
+            (void)hipStreamDestroy(c->stream);
+            delete c;
+            throw;
+        }
         *out = c;
     });
 }
@@ -951,10 +990,11 @@ int pg_ctx_destroy(pg_ctx* c) {
         if (!c) return;
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
-        (void)hipStreamDestroy(c->stream);
         const int device = c->device;
+        BlockPool::of(device).context_leaves(c->stream);
+        (void)hipStreamDestroy(c->stream);
         delete c;
-        BlockPool::of(device).context_removed();
+        BlockPool::of(device).context_gone();
     });
 }
 
@@ -2265,17 +2305,21 @@ void batch_capture(pg_ctx* c, pg_batch* B) {
         B->exec = nullptr;
     }
     hipGraph_t g = nullptr;
-    HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
-    try {
-        batch_hydro(B, c->stream);
-        batch_rebuild(B, c->stream);
-    } catch (...) {
-        // end the capture so that the stream is usable again
-        if (hipStreamEndCapture(c->stream, &g) == hipSuccess && g) (void)hipGraphDestroy(g);
-        (void)hipGetLastError();
-        throw;
+    hipError_t e;
+    {
+        BlockPool::Capture alone(c->device);
+        HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
+        try {
+            batch_hydro(B, c->stream);
+            batch_rebuild(B, c->stream);
+        } catch (...) {
+            // end the capture so that the stream is usable again
+            if (hipStreamEndCapture(c->stream, &g) == hipSuccess && g) (void)hipGraphDestroy(g);
+            (void)hipGetLastError();
+            throw;
+        }
+        e = hipStreamEndCapture(c->stream, &g);
     }
-    hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         hipchk(e, "hipStreamEndCapture");
