@@ -508,6 +508,14 @@ int next_k(int k, int cap) {
 constexpr int BIG_ROW = 256;
 int big_row(int k, int cap, bool restart) { return restart ? std::max(k, std::min(cap, BIG_ROW)) : k; }
 
+// Learned builds whose restarts do not end at the longest bucket's row or a
+// longer one: a seed that outgrows the small 2D kernel is redone at its own
+// bucket's row, so that it has the row it would have without (elsewhere, and in
+// 3D, where that is rare, the chain after the buckets redoes it).
+bool overflow_by_bucket(const pg_mesh_params& p) {
+    return p.dim == 2 && !(p.restart && p.k_max >= pg::lk_bucket(pg::LK_NCLASS - 1));
+}
+
 // What a restart chain knows of the statuses it leaves (of all its seeds):
 // nothing when !known.
 struct ChainEnd {
@@ -817,6 +825,12 @@ void mesh_build_once(pg_ctx* c, pg_mesh* m, const double* pts, int64_t n, bool o
                 m->info.row_entries += hc[c] * bk[c];
             }
         HIPCHK(hipGetLastError());
+        for (int c = 0; c < pg::LK_NCLASS && overflow_by_bucket(p); c++) {
+            uint32_t* ov = m->list3.get<uint32_t>(ns);
+            const int64_t no = collect_list(m, kl + (size_t)c * ns, hc[c], pg::SLOT_OVERFLOW, ov, s);
+            run_list(m, ov, no, bk[c], 1, s);
+            m->info.n_restarted += no;
+        }
         if (mk) mk->mark(MK_CLIP, s);
         // every rejected seed (any bucket) continues in one restart chain:
         // a seed recomputed at a row length at least its certified k gives
@@ -2155,6 +2169,8 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
         pg::launch_fill_u64((unsigned long long*)nout, 1, 0ull, s);
         pg::launch_collect(cap, nL, L, B->status.as<int32_t>(), code, out, (unsigned long long*)nout, false, s);
     };
+    uint32_t* lst[3] = {B->lists.as<uint32_t>(), B->lists.as<uint32_t>() + cap, B->lists.as<uint32_t>() + 2 * cap};
+    int64_t* cnt[3] = {B->ncount.as<int64_t>(), B->ncount.as<int64_t>() + 1, B->ncount.as<int64_t>() + 2};
     // first pass: every seed at the fixed k, or every bucket of the learned
     // k at its own k; then the restart chain of the single-box build
     const std::vector<int>& sched = B->km ? B->ksched_learned : B->ksched;
@@ -2183,10 +2199,13 @@ void batch_rebuild(pg_batch* B, hipStream_t s) {
             const uint32_t* lc = B->klists.as<uint32_t>() + (size_t)c * cap;
             knn(lc, B->kcnt.as<int64_t>() + c, pg::lk_bucket(c), false, true);
             clip(lc, B->kcnt.as<int64_t>() + c, pg::lk_bucket(c), 0, false);
+            if (overflow_by_bucket(p)) {  // as in the single-box build
+                collect(lc, B->kcnt.as<int64_t>() + c, pg::SLOT_OVERFLOW, lst[2], cnt[2]);
+                knn(lst[2], cnt[2], pg::lk_bucket(c), false, true);
+                clip(lst[2], cnt[2], pg::lk_bucket(c), 1, true);
+            }
         }
     }
-    uint32_t* lst[3] = {B->lists.as<uint32_t>(), B->lists.as<uint32_t>() + cap, B->lists.as<uint32_t>() + 2 * cap};
-    int64_t* cnt[3] = {B->ncount.as<int64_t>(), B->ncount.as<int64_t>() + 1, B->ncount.as<int64_t>() + 2};
     const uint32_t* L = nullptr;
     const int64_t* nL = n_dev;
     // overflowed seeds keep that status through the chain; the 128-slot
