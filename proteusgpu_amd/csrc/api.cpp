@@ -52,8 +52,9 @@ int guarded(F&& f) {
 // some 50 buffers and gives them back with itself; hipMalloc and hipFree took
 // 0.5 of the 1.3 ms of a 10k 2D mesh's call and 12 of the 78 ms of a clustered
 // 400k 3D one (on machines that map memory slowly 90 of 170).
-//  - At most KEEP bytes per device are held, the oldest go first, and only
-//    while a context of the device lives: the last one's end frees them all.
+//  - At most KEEP bytes in MOST blocks per device are held (a block of few bytes
+//    takes a page, and every take looks through them), the oldest go first, and
+//    only while a context of the device lives: the last one's end frees them all.
 //    An allocation that fails frees them and tries again, and a program that
 //    needs the memory elsewhere has pg_ctx_trim.
 //  - A block may have been left with work on it in flight, on the stream of any
@@ -72,7 +73,7 @@ public:
         return pools[device];
     }
     static constexpr int MAX_DEVICES = 64;
-    static constexpr size_t KEEP = (size_t)8 << 30;
+    static constexpr size_t KEEP = (size_t)8 << 30, MOST = 4096;
 
     void context_added(hipStream_t s) {
         std::lock_guard<std::recursive_mutex> g(mu);
@@ -145,6 +146,7 @@ public:
         bool kept = false;
         if (!streams.empty() && cap <= KEEP) {
             drop_to(KEEP - cap);
+            if (free.size() >= MOST) drop(MOST / 4);
             try {
                 free.push_back({p, cap, false});
                 held += cap;
@@ -180,13 +182,18 @@ private:
         }
         return true;
     }
-    void drop_to(size_t bytes) noexcept {
-        size_t n = 0;
-        for (; held > bytes; n++) {
-            (void)hipFree(free[n].p);
-            held -= free[n].cap;
+    // the n oldest blocks
+    void drop(size_t n) noexcept {
+        for (size_t i = 0; i < n; i++) {
+            (void)hipFree(free[i].p);
+            held -= free[i].cap;
         }
         free.erase(free.begin(), free.begin() + (ptrdiff_t)n);
+    }
+    void drop_to(size_t bytes) noexcept {
+        size_t n = 0, left = held;
+        for (; left > bytes; n++) left -= free[n].cap;
+        drop(n);
     }
 };
 
